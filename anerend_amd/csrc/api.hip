@@ -1088,7 +1088,7 @@ extern "C" int ane_ddgi_create(const ane_ddgi_config* cfg, ane_ddgi_ctx** out)
   }
   // FP8 radiance scales: one float per (probe, channel, 32 rays)
   ANE_A(d_rad_scale, c->P * 3 * ((c->N + 31) / 32));
-  ANE_A(d_work, 4);
+  ANE_A(d_work, kTraceWorkWords);
   ANE_A(d_stats, 4);
   ANE_A(d_overflow, 1);
   ANE_A(d_tiles, (int64_t)(g.nx + 1) + (int64_t)(g.ny + 1) * (g.nz + 1));
@@ -1285,7 +1285,7 @@ extern "C" int ane_ddgi_trace(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddg
   const int nprobes = fk.layer_count * c->g.nx * c->g.nz;
   ANE_TRY(c->timers[kStSetup].begin(st));
   ANE_TRY(do_frame_setup(c, fk, bake, st));
-  fill_u32(c->d_work, 0u, 4, st);
+  fill_u32(c->d_work, 0u, kTraceWorkWords, st);
   if (c->counting) fill_u32(reinterpret_cast<uint32_t*>(c->d_stats), 0u, 8, st);
   ANE_TRY(c->timers[kStSetup].end(st));
   TraceArgs a = trace_args(c, s, fk);
@@ -1373,7 +1373,7 @@ int ddgi_update_front(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame*
   const bool bake = (fk.flags & ANE_FLAG_BAKE) != 0;
   const int nprobes = fk.layer_count * c->g.nx * c->g.nz;
   ANE_TRY(do_frame_setup(c, fk, bake, st));
-  fill_u32(c->d_work, 0u, 4, st);
+  fill_u32(c->d_work, 0u, kTraceWorkWords, st);
   if (c->counting) fill_u32(reinterpret_cast<uint32_t*>(c->d_stats), 0u, 8, st);
   TraceArgs a = trace_args(c, s, fk);
   a.work = c->d_work;
@@ -1656,7 +1656,7 @@ extern "C" int ane_ddgi_mirror_reflections(ane_ddgi_ctx* c, const ane_scene* s, 
   }
   if (!c->d_mr_work || !c->d_mr_stats || !c->d_mr_ov) {  // all three, or redo them
     dfree(c->d_mr_work); dfree(c->d_mr_stats); dfree(c->d_mr_ov);
-    ANE_TRY(dalloc(&c->d_mr_work, 2, nullptr));
+    ANE_TRY(dalloc(&c->d_mr_work, 2 * kTraceWorkWords, nullptr));
     ANE_TRY(dalloc(&c->d_mr_stats, 4, nullptr));
     ANE_TRY(dalloc(&c->d_mr_ov, 1, nullptr));
   }
@@ -1669,7 +1669,7 @@ extern "C" int ane_ddgi_mirror_reflections(ane_ddgi_ctx* c, const ane_scene* s, 
     ANE_TRY(dalloc(&c->d_mr_spill, sd * lanes, nullptr));
     c->mr_spill_words = sd * lanes;
   }
-  fill_u32(c->d_mr_work, 0u, 2, st);
+  fill_u32(c->d_mr_work, 0u, 2 * kTraceWorkWords, st);
   fill_u32(reinterpret_cast<uint32_t*>(c->d_mr_stats), 0u, 8, st);
   fill_u32(c->d_mr_ov, 0u, 1, st);
   // mirror_reflections.rgen:57-79: reflection rays over [0.1, 50], closest hit
@@ -1705,7 +1705,7 @@ extern "C" int ane_ddgi_mirror_reflections(ane_ddgi_ctx* c, const ane_scene* s, 
   }
   a.skip_if_set = skip;
   a.hits = c->d_mr_hits[1];
-  a.work = c->d_mr_work + 1;
+  a.work = c->d_mr_work + kTraceWorkWords;
   a.stats = c->d_mr_stats + 2;
   a.ray_orig = c->d_mr_orig[1];
   a.ray_dir = c->d_mr_dir[1];
@@ -1933,7 +1933,7 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
   }
   if (!s->d_sh_work || !s->d_sh_stats || !s->d_sh_ov) {  // all three, or redo them
     dfree(s->d_sh_work); dfree(s->d_sh_stats); dfree(s->d_sh_ov);
-    ANE_TRY(dalloc(&s->d_sh_work, 1, nullptr));
+    ANE_TRY(dalloc(&s->d_sh_work, kTraceWorkWords, nullptr));
     ANE_TRY(dalloc(&s->d_sh_stats, 2, nullptr));
     ANE_TRY(dalloc(&s->d_sh_ov, 1, nullptr));
   }
@@ -1959,7 +1959,7 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
     }
   }
   launch_shadow_rays(depth, width, height, ivp16, light3, s->d_sh_orig, s->d_sh_dir, st, skip);
-  fill_u32(s->d_sh_work, 0u, 1, st);
+  fill_u32(s->d_sh_work, 0u, kTraceWorkWords, st);
   fill_u32(reinterpret_cast<uint32_t*>(s->d_sh_stats), 0u, 4, st);
   fill_u32(s->d_sh_ov, 0u, 1, st);
   TraceArgs a{};
@@ -2059,7 +2059,7 @@ extern "C" int ane_scene_light_shadows(ane_scene* s, const ane_light* lights, in
     ANE_CHECK_HIP(hipMemcpy(s->d_lt_dirs, dirs.data(), sizeof(float) * dirs.size(), hipMemcpyHostToDevice));
     ANE_CHECK_HIP(hipMemcpy(s->d_lt_wt, lw.data(), sizeof(float) * lw.size(), hipMemcpyHostToDevice));
     ANE_CHECK_HIP(hipMemcpy(s->d_lt_idx, li.data(), sizeof(int32_t) * li.size(), hipMemcpyHostToDevice));
-    ANE_TRY(dalloc(&s->d_lt_work, 1, nullptr));
+    ANE_TRY(dalloc(&s->d_lt_work, kTraceWorkWords, nullptr));
     ANE_TRY(dalloc(&s->d_lt_stats, 2, nullptr));
     ANE_TRY(dalloc(&s->d_lt_ov, 1, nullptr));
     s->lt_kmax = kmax;
@@ -2091,7 +2091,7 @@ extern "C" int ane_scene_light_shadows(ane_scene* s, const ane_light* lights, in
                                hipMemcpyHostToDevice, st));
   launch_light_rays(s->d_lt_lights, num_lights, s->d_lt_dirs, s->d_lt_order, s->d_lt_orig, s->d_lt_dir,
                     s->d_lt_tmax, st);
-  fill_u32(s->d_lt_work, 0u, 1, st);
+  fill_u32(s->d_lt_work, 0u, kTraceWorkWords, st);
   fill_u32(reinterpret_cast<uint32_t*>(s->d_lt_stats), 0u, 4, st);
   fill_u32(s->d_lt_ov, 0u, 1, st);
   TraceArgs a{};
@@ -2147,7 +2147,7 @@ extern "C" int ane_scene_trace_rays(const ane_scene* s, const float* origins, co
   int st_ = ANE_OK;
   auto cleanup = [&]() { dfree(d_o); dfree(d_d); dfree(d_h); dfree(d_work); dfree(d_stats); dfree(d_ov); dfree(d_spill); };
   if ((st_ = dalloc(&d_o, num_rays * 3, nullptr)) || (st_ = dalloc(&d_d, num_rays * 3, nullptr)) ||
-      (st_ = dalloc(&d_h, num_rays, nullptr)) || (st_ = dalloc(&d_work, 1, nullptr)) ||
+      (st_ = dalloc(&d_h, num_rays, nullptr)) || (st_ = dalloc(&d_work, kTraceWorkWords, nullptr)) ||
       (st_ = dalloc(&d_stats, 2, nullptr)) || (st_ = dalloc(&d_ov, 1, nullptr)) ||
       (st_ = dalloc(&d_spill, sd * lanes, nullptr))) {
     cleanup();
@@ -2160,7 +2160,7 @@ extern "C" int ane_scene_trace_rays(const ane_scene* s, const float* origins, co
     cleanup();
     return fail_hip(e, "upload", __FILE__, __LINE__);
   }
-  fill_u32(d_work, 0u, 1, st);
+  fill_u32(d_work, 0u, kTraceWorkWords, st);
   TraceArgs a{};
   a.sc = s->view;
   a.g.t_min = t_min;
@@ -2204,7 +2204,8 @@ extern "C" int ane_scene_trace_rays(const ane_scene* s, const float* origins, co
 // hipGetSymbolAddress, once per device with that device current.
 // ===========================================================================
 static constexpr int64_t kScratchBytes = (int64_t)16 << 20;  // per GPU, held until the process ends
-static constexpr int64_t kScratchSpillWord = 64;              // spill area starts at byte 256
+static constexpr int64_t kScratchStatsWord = kTraceWorkWords;      // after the ray counters: two 64-bit work counters,
+static constexpr int64_t kScratchSpillWord = kTraceWorkWords + 64; // the fault flag, then the spill area
 static __device__ __align__(256) uint32_t scratch[kScratchBytes / 4];
 
 static constexpr int kMaxDevices = 64;
@@ -2257,9 +2258,10 @@ extern "C" int ane_scene_trace_rays_noalloc(const ane_scene* s, const float* ori
                 "more than the %lld-byte scratch", s->depth, (long long)(depth * 4), (long long)((int64_t)cus * tb),
                 (long long)kScratchBytes);
   hipStream_t st = S(stream);
-  // scratch words 0 ray counter, 2-5 the two 64-bit work counters, 6 the fault flag:
-  // cleared by a kernel (the array keeps the previous call's contents)
-  fill_u32(sp, 0u, 8, st);
+  // the ray counters, the two 64-bit work counters and the fault flag are cleared by a
+  // kernel (the array keeps the previous call's contents)
+  uint32_t* head = sp + kScratchStatsWord;
+  fill_u32(sp, 0u, kScratchStatsWord + 5, st);
   TraceArgs a{};
   a.sc = s->view;
   a.g.t_min = t_min;
@@ -2267,8 +2269,8 @@ extern "C" int ane_scene_trace_rays_noalloc(const ane_scene* s, const float* ori
   a.g.rays = 1;
   a.hits = hits;
   a.work = sp;
-  a.stats = reinterpret_cast<unsigned long long*>(sp + 2);
-  a.overflow = sp + 6;
+  a.stats = reinterpret_cast<unsigned long long*>(head);
+  a.overflow = head + 4;
   a.spill = reinterpret_cast<int32_t*>(sp + kScratchSpillWord);
   a.spill_depth = (int32_t)depth;
   a.total_lanes = (int32_t)lanes;
@@ -2281,8 +2283,8 @@ extern "C" int ane_scene_trace_rays_noalloc(const ane_scene* s, const float* ori
   ANE_CHECK_HIP(hipGetLastError());
   uint32_t ov = 0;
   unsigned long long c2[2] = {0, 0};
-  ANE_CHECK_HIP(hipMemcpyAsync(&ov, sp + 6, 4, hipMemcpyDeviceToHost, st));
-  if (counters2) ANE_CHECK_HIP(hipMemcpyAsync(c2, sp + 2, 16, hipMemcpyDeviceToHost, st));
+  ANE_CHECK_HIP(hipMemcpyAsync(&ov, head + 4, 4, hipMemcpyDeviceToHost, st));
+  if (counters2) ANE_CHECK_HIP(hipMemcpyAsync(c2, head, 16, hipMemcpyDeviceToHost, st));
   ANE_CHECK_HIP(hipStreamSynchronize(st));
   if (ov) return fail(ANE_ERR_DEVICE, "traversal stack exceeded its spill capacity");
   if (counters2) { counters2[0] = c2[0]; counters2[1] = c2[1]; }

@@ -129,6 +129,12 @@ void launch_sun_grid_build(const SceneK& sc, const SunGridParams& g, SunGridPara
 // probe traces can take a sun grid (k_probe_shadow_grid runs their shadow rays)
 bool trace_grid_supported();
 
+// Claim counters of a traversal launch (TraceArgs::work): kTraceCounters (a power of
+// two) words, one per kTraceCounterStride so that each lies in a cache line of its own
+static constexpr int kTraceCounters = 16;
+static constexpr int kTraceCounterStride = 32;
+static constexpr int kTraceWorkWords = kTraceCounters * kTraceCounterStride;
+
 struct TraceArgs {
   SceneK sc;
   GridK g;
@@ -141,7 +147,10 @@ struct TraceArgs {
   int32_t div_shift;
   ane_hit* hits;          // out: closest hit per ray
   uint8_t* shadow;        // out (probe rays): 0 lit, 1 shadowed, 255 miss
-  uint32_t* work;         // dynamic ray counter (zeroed before launch)
+  uint32_t* work;         // [kTraceWorkWords] claim counters (zeroed before launch)
+  uint32_t ncounters;
+  uint32_t chunk;         // rays a wave takes at a time (set by launch_trace)
+  uint32_t static_rays;   // rays of the waves' first chunks, which need no claim (set by launch_trace)
   unsigned long long* stats; // counting kernels: nodes, triangles [, shadow nodes, shadow triangles]
   uint32_t* overflow;     // set to 1 when a ray ends without a result: a stack would exceed the
                           // spill capacity, the step limit ran out or the hierarchy is malformed

@@ -40,13 +40,10 @@ namespace ane {
 #define ANE_TRACE_STACK 16
 #endif
 #ifndef ANE_TRACE_CHUNK
-#define ANE_TRACE_CHUNK 256  // probe rays claimed by a wave at a time (64-byte nodes)
-#endif
-#ifndef ANE_TRACE_CHUNK_RAYS
-#define ANE_TRACE_CHUNK_RAYS 128  // caller rays claimed by a wave at a time (64-byte nodes)
+#define ANE_TRACE_CHUNK 64  // rays a wave takes at a time
 #endif
 #ifndef ANE_TRACE_REFILL
-#define ANE_TRACE_REFILL 32
+#define ANE_TRACE_REFILL 16
 #endif
 #ifndef ANE_TRACE_UNROLL
 #define ANE_TRACE_UNROLL 5  // traversal steps per refill check
@@ -74,33 +71,32 @@ namespace ane {
 #endif
 static constexpr int kTB = ANE_TRACE_BLOCK;      // threads per traversal block
 static constexpr int kSS = ANE_TRACE_STACK;      // LDS stack entries per lane (ring, any size)
-// Every claim is one device-scope atomic on the launch's counter, which all 8 XCDs
-// share: with 128-ray chunks the 8.4M probe rays of an update made 65k claims and the
-// trace waited on them (terrain1m trace 1.028 ms; 256: 0.895, 384: 0.906, 512: 0.979,
-// 64: 1.69).  Caller rays (1-2M per pass) keep 128: larger chunks unbalance their
-// launch's end (mirror pass 0.78 -> 0.87 ms at 256).
-static constexpr int kChunk = ANE_TRACE_CHUNK;
-static constexpr int kChunkRays = ANE_TRACE_CHUNK_RAYS;
-static constexpr int kRefill = ANE_TRACE_REFILL; // idle lanes that trigger a refill
+// Rays a wave takes at a time: one per lane.  A claim is a device-scope atomic, and one
+// address takes about 80 of them per microsecond from the 8 XCDs: with a single counter
+// for all waves and 64-ray chunks the 8.4M probe rays of an update waited on their claims
+// (terrain1m update 2.2 ms; 128 / 256-ray chunks 1.53 / 1.38), and 256-ray chunks left
+// most waves of a launch under 1.8M rays without any (131k rays of a room: 391 us).  So a
+// wave's first chunk needs no claim, and the others are claimed from kTraceCounters
+// counters in turn: the update 1.35 ms, the room 184 us, 65k light rays 292 -> 153 us, a
+// 1080p mirror pass 750 -> 590 us.  Counter k's claims walk over the residues modulo
+// kTraceCounters: with fixed residues a counter owned one range of directions (512 rays
+// per probe are 8 chunks) and the counters ended far apart (1.83 ms).  1 / 2 / 4 / 8
+// counters: 2.22 / 1.49 / 1.52 / 1.35 ms; chunks of 16 / 32 / 128 / 256 rays: 202 / 184 /
+// 229 / 305 us for the room, 1.34 ms for the update from 128 up.
+static constexpr uint32_t kChunk = ANE_TRACE_CHUNK;
+// Idle lanes that trigger a refill (24 / 32: 1.335 / 1.347 ms against 1.338 for the terrain1m
+// update, 586 / 592 us against 579 for the 1080p mirror pass; 8 / 24 on quantized nodes: 13.35 /
+// 13.32 ms per frame of the 4.04M-triangle scene against 13.27)
+static constexpr int kRefill = ANE_TRACE_REFILL;
 // The quantized-node traversal serves scenes whose nodes miss the caches: its
-// lanes wait on memory rather than on VALU issue, so it refills earlier and claims
-// larger chunks (4.04M-triangle scene: trace 10.0 -> 9.0 ms against 32 / 128), and
-// checks for refills every 7 steps (9.09 -> 8.98 ms against 5); chunks of 384 / 512
-// measured 8.98 / 9.60 ms against 8.84
-#ifndef ANE_TRACE_CHUNK_Q
-#define ANE_TRACE_CHUNK_Q 256
-#endif
-#ifndef ANE_TRACE_REFILL_Q
-#define ANE_TRACE_REFILL_Q 16
-#endif
+// lanes wait on memory rather than on VALU issue, and it checks for refills
+// every 7 steps (4.04M-triangle scene: trace 9.09 -> 8.98 ms against 5)
 #ifndef ANE_TRACE_UNROLL_Q
 #define ANE_TRACE_UNROLL_Q 7  // steps per refill check (quantized nodes)
 #endif
 #ifndef ANE_TRACE_LEAFBATCH_Q
 #define ANE_TRACE_LEAFBATCH_Q ANE_TRACE_LEAFBATCH
 #endif
-static constexpr int kChunkQ = ANE_TRACE_CHUNK_Q;
-static constexpr int kRefillQ = ANE_TRACE_REFILL_Q;
 static constexpr int kLeafBatchProbe = ANE_TRACE_LEAFBATCH;
 static constexpr int kLeafBatchRays = ANE_TRACE_LEAFBATCH_RAYS;
 static constexpr int kShadeUnroll = ANE_SHADE_UNROLL;
@@ -338,7 +334,11 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
   int32_t ray = -1;  // active ray (processing index), -1 idle
   bool exhausted = false;
   bool sph = ANY;    // the lane's ray is an any-hit (shadow) ray
-  uint32_t cbeg = 0, cend = 0;  // wave-uniform: remaining part of the claimed chunk
+  // wave-uniform: remaining part of the wave's chunk.  The first one is its own
+  // (wave w: rays [w kChunk, (w + 1) kChunk)), further ones are claimed.
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kTB / 64) + (tid >> 6))) * kChunk;
+  uint32_t cbeg = first < nrays ? first : nrays;
+  uint32_t cend = cbeg + kChunk < nrays ? cbeg + kChunk : nrays;
   RayPre r;
   float tbest = 0.0f, bu = 0.0f, bv = 0.0f;
   int32_t bid = -1, node = kDone, sp = 0, out = 0;
@@ -378,14 +378,23 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
     const uint64_t im = __ballot(idle);
     const uint64_t am = __ballot(ray >= 0);
     const uint32_t need = (uint32_t)__popcll(im);
-    constexpr uint32_t chunk = (uint32_t)(Q ? kChunkQ : (RAYS ? kChunkRays : kChunk));
-    if (need != 0u && (am == 0ull || need >= (uint32_t)(Q ? kRefillQ : kRefill))) {
-      if (cbeg >= cend) {  // claim the next chunk (one atomic per wave and chunk)
-        uint32_t base = 0;
-        if (lane == __ffsll((unsigned long long)im) - 1) base = atomicAdd(a.work, chunk);
-        base = __shfl(base, __ffsll((unsigned long long)im) - 1, 64);
+    if (need != 0u && (am == 0ull || need >= (uint32_t)kRefill)) {
+      if (cbeg >= cend) {  // the next chunk: none when every ray was in a first chunk
+        uint32_t base = nrays;
+        if (a.static_rays < nrays) {
+          // claim i of counter k: chunk (k + i) % K of the i-th group of K chunks
+          // (in 32 bits: a wave makes one claim past the end)
+          constexpr uint32_t K = (uint32_t)kTraceCounters;
+          const uint32_t k = blockIdx.x & (K - 1u);
+          const int who = __ffsll((unsigned long long)im) - 1;
+          uint32_t i = 0u;
+          if (lane == who) i = atomicAdd(a.work + k * kTraceCounterStride, 1u);
+          i = (uint32_t)__builtin_amdgcn_readlane((int)i, who);
+          base = a.static_rays + (i * K + ((k + i) & (K - 1u))) * kChunk;
+          base = base < nrays ? base : nrays;
+        }
         cbeg = base;
-        cend = base + chunk < nrays ? base + chunk : nrays;
+        cend = base + kChunk < nrays ? base + kChunk : nrays;
       }
       const uint32_t avail = cend > cbeg ? cend - cbeg : 0u;
       const uint32_t rank = (uint32_t)__popcll(im & lt);
@@ -760,12 +769,15 @@ int trace_lanes_per_launch()
 void launch_trace(const TraceArgs& a, bool any_hit, bool rays, bool count, hipStream_t s)
 {
   // a persistent grid of every resident block, or fewer when the caller caps the
-  // lanes (a.total_lanes > 0: the spill area is sized for that many)
+  // lanes (a.total_lanes > 0: the spill area is sized for that many) or the rays run out
   const int full = trace_lanes_per_launch() / kTB;
   const int want = a.total_lanes > 0 ? a.total_lanes / kTB : full;
-  const int blocks = want < 1 ? 1 : (want < full ? want : full);
+  const int fed = (int)(((int64_t)a.nrays + kChunk * (kTB / 64) - 1) / (kChunk * (kTB / 64)));  // blocks with rays
+  const int most = want < full ? want : full;
+  const int blocks = fed < 1 || most < 1 ? 1 : (fed < most ? fed : most);
   TraceArgs b = a;
   b.total_lanes = blocks * kTB;
+  b.static_rays = (uint32_t)(blocks * (kTB / 64)) * kChunk;
 #define ANE_TR(S, R, C)                                                                             \
   do {                                                                                              \
     if (b.sc.qnodes) hipLaunchKernelGGL((k_trace<S, R, C, true>), dim3(blocks), dim3(kTB), 0, s, b);  \
