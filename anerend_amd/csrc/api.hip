@@ -159,84 +159,14 @@ static float to_linear_host(float c)
   return (c < 0.04045f) ? c / 12.92f : powf((c + 0.055f) / 1.055f, 2.4f);
 }
 
-// Ring of hipEvent pairs per stage: recording never waits on the device; a
-// slot is harvested (elapsed time accumulated) before it is reused or when
-// statistics are read.
-struct StageTimer {
-  static constexpr int kSlots = 32;
-  hipEvent_t s[kSlots] = {};
-  hipEvent_t e[kSlots] = {};
-  bool pending[kSlots] = {};
-  int next = 0, cur = -1;
-  bool off = false;  // no events (while an update is captured into a graph)
-  double acc_ms = 0.0;
-  uint64_t count = 0;
-  float last_ms = 0.0f;
-
-  int init()
-  {
-    for (int i = 0; i < kSlots; ++i) {
-      ANE_CHECK_HIP(hipEventCreate(&s[i]));
-      ANE_CHECK_HIP(hipEventCreate(&e[i]));
-    }
-    return 0;
-  }
-  void destroy()
-  {
-    for (int i = 0; i < kSlots; ++i) {
-      if (s[i]) (void)hipEventDestroy(s[i]);
-      if (e[i]) (void)hipEventDestroy(e[i]);
-      s[i] = e[i] = nullptr;
-    }
-  }
-  int harvest(int i)
-  {
-    if (!pending[i]) return 0;
-    ANE_CHECK_HIP(hipEventSynchronize(e[i]));
-    float t = 0.0f;
-    ANE_CHECK_HIP(hipEventElapsedTime(&t, s[i], e[i]));
-    acc_ms += t;
-    ++count;
-    last_ms = t;
-    pending[i] = false;
-    return 0;
-  }
-  int harvest_all()
-  {
-    for (int k = 0; k < kSlots; ++k) {
-      int i = (next + k) % kSlots;  // oldest first
-      int st = harvest(i);
-      if (st) return st;
-    }
-    return 0;
-  }
-  int begin(hipStream_t st)
-  {
-    if (off) return 0;
-    cur = next;
-    int r = harvest(cur);
-    if (r) return r;
-    ANE_CHECK_HIP(hipEventRecord(s[cur], st));
-    return 0;
-  }
-  int end(hipStream_t st)
-  {
-    if (off) return 0;
-    ANE_CHECK_HIP(hipEventRecord(e[cur], st));
-    pending[cur] = true;
-    next = (cur + 1) % kSlots;
-    return 0;
-  }
-  void reset()
-  {
-    acc_ms = 0.0;
-    count = 0;
-  }
-};
-
 enum { kStSetup = 0, kStTrace, kStSunGrid, kStShade, kStConv, kStTrans, kStShadow, kStages };
 static_assert(kStages == sizeof(((ane_ddgi_stats*)nullptr)->mean_ms) / sizeof(float),
-              "one stats entry per stage timer");
+              "one stats entry per stage");
+
+// The stage clocks of a context: one per kind of call, with the stages of its calls
+enum { kClkTrace = 0, kClkConv, kClkTrans, kClocks };
+static constexpr int kClkStage[kClocks][kClockStages] = {
+    {kStSetup, kStSunGrid, kStTrace, kStShadow, kStShade}, {kStConv, -1, -1, -1, -1}, {kStTrans, -1, -1, -1, -1}};
 
 }  // namespace ane
 
@@ -289,6 +219,7 @@ struct SunGridCache {
              dir[1] == o.dir[1] && dir[2] == o.dir[2];
     }
   } built, seen;
+  uint64_t builds = 0;        // grids built so far
   // the validity flag of a build, read back without blocking: copied to pinned
   // memory behind an event (not under stream capture) and taken once the event
   // has completed.  `known` is the build whose flag last_valid holds; a newer
@@ -363,10 +294,10 @@ struct SunGridCache {
   // components take the reciprocal of +-1e-30) culls boxes whose triangles the
   // watertight test would touch on an edge, so a grid's answer could differ
   // from the traversal's there.
-  // timer (nullable) brackets a build's launches on the stream
+  // clk, stage: the stage stamp of a build
   // rays: the rays of the request (the eager-build rule)
   int update(const SceneK& view, int32_t ntri, const void* scene, uint64_t version, const float* dir3,
-             int64_t rays, hipStream_t st, bool* use, StageTimer* timer = nullptr)
+             int64_t rays, hipStream_t st, bool* use, const ClockArg& clk = ClockArg{}, int stage = 0)
   {
     *use = false;
     for (int k = 0; k < 3; ++k)
@@ -393,11 +324,10 @@ struct SunGridCache {
     ANE_TRY(alloc(ntri));
     SunGridParams p;
     sun_grid_setup(p, dir3, g, g);
-    if (timer) ANE_TRY(timer->begin(st));
-    launch_sun_grid_build(view, p, params, acc, start, cur, list, cap, scan, est, st);
-    if (timer) ANE_TRY(timer->end(st));
+    launch_sun_grid_build(view, p, params, acc, start, cur, list, cap, scan, est, clk, stage, st);
     ANE_CHECK_HIP(hipGetLastError());
     built = k;
+    ++builds;
     if (!capturing) {
       if (!h_valid) ANE_CHECK_HIP(hipHostMalloc((void**)&h_valid, sizeof(uint32_t), hipHostMallocDefault));
       if (!ev) ANE_CHECK_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -979,7 +909,10 @@ struct ane_ddgi_ctx {
   uint32_t step_limit = 0;          // ane_ddgi_set_traversal_limit
   int32_t* d_spill = nullptr;
   int64_t spill_words = 0;
-  StageTimer timers[kStages];
+  StageClock* d_clock = nullptr;  // [kClocks]
+  uint64_t calls[kStages] = {};   // since the last reset, of each stage
+  int clock_set[kClocks] = {};    // the stamp set of the last call of each kind
+  int32_t clock_khz = 0;          // ticks per ms
   int32_t last_cell[2] = {0, 0};
   int32_t rad_begin = -1, rad_count = 0;  // layers held in the radiance buffer
   bool rad_bake = false;
@@ -1014,7 +947,7 @@ static void ctx_free(ane_ddgi_ctx* c)
   if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
   for (int k = 0; k < 2; ++k) { dfree(c->d_mr_orig[k]); dfree(c->d_mr_dir[k]); dfree(c->d_mr_hits[k]); }
   dfree(c->d_mr_work); dfree(c->d_mr_stats); dfree(c->d_mr_ov); dfree(c->d_mr_spill);
-  for (auto& t : c->timers) t.destroy();
+  dfree(c->d_clock);
 }
 
 static int validate_config(const ane_ddgi_config* c)
@@ -1091,13 +1024,10 @@ extern "C" int ane_ddgi_create(const ane_ddgi_config* cfg, ane_ddgi_ctx** out)
   ANE_A(d_work, kTraceWorkWords);
   ANE_A(d_stats, 4);
   ANE_A(d_overflow, 1);
+  ANE_A(d_clock, kClocks);
   ANE_A(d_tiles, (int64_t)(g.nx + 1) + (int64_t)(g.ny + 1) * (g.nz + 1));
 #undef ANE_A
   hipError_t e;
-  for (auto& t : c->timers)
-    if ((st = t.init()) != ANE_OK) {
-      ctx_free(c); delete c; return st;
-    }
   {
     // tile texture bounds, the operations of sampleSingleProbe (pbr_light.glsl:177-183)
     // in binary32: start = (2 * s0 + 1) / (2 * extent), end for s0 + 7
@@ -1132,7 +1062,8 @@ extern "C" int ane_ddgi_create(const ane_ddgi_config* cfg, ane_ddgi_ctx** out)
       (e = hipMemcpy(c->d_atlas[1], clear.data(), clear.size() * 4, hipMemcpyHostToDevice)) ||
       (e = hipMemcpy(c->d_base_dirs, dirs.data(), dirs.size() * 4, hipMemcpyHostToDevice)) ||
       (e = hipMemcpy(c->d_order, order.data(), order.size() * 4, hipMemcpyHostToDevice)) ||
-      (e = hipMemset(c->d_overflow, 0, 4))) {
+      (e = hipMemset(c->d_overflow, 0, 4)) || (e = hipMemset(c->d_clock, 0, kClocks * sizeof(StageClock))) ||
+      (e = hipDeviceGetAttribute(&c->clock_khz, hipDeviceAttributeWallClockRate, c->device))) {
     st = fail_hip(e, "hipMemcpy", __FILE__, __LINE__);
     ctx_free(c); delete c; return st;
   }
@@ -1265,11 +1196,32 @@ static TraceArgs trace_args(ane_ddgi_ctx* c, const ane_scene* s, const FrameK& f
   return a;
 }
 
-static int do_frame_setup(ane_ddgi_ctx* c, const FrameK& fk, bool bake, hipStream_t st)
+// The stage clock of a call of kind `k` on `st` and its next stamp set; none while the
+// call is captured into a graph, whose replays are not counted.
+static int clock_of(ane_ddgi_ctx* c, int k, hipStream_t st, ClockArg* out)
+{
+  *out = ClockArg{};
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  ANE_CHECK_HIP(hipStreamIsCapturing(st, &cs));
+  if (cs != hipStreamCaptureStatusNone) return ANE_OK;
+  c->clock_set[k] ^= 1;
+  out->c = c->d_clock + k;
+  out->set = c->clock_set[k];
+  return ANE_OK;
+}
+
+// a stage of the call with the clock `clk` was launched
+static void count_stage(ane_ddgi_ctx* c, const ClockArg& clk, int stage)
+{
+  if (clk.c) ++c->calls[stage];
+}
+
+static int do_frame_setup(ane_ddgi_ctx* c, const FrameK& fk, bool bake, hipStream_t st,
+                          const ClockArg& clk = ClockArg{})
 {
   launch_frame_setup(c->g, fk, c->d_base_dirs, c->d_order, c->d_dirs, c->d_dirpre, c->d_probe_org, c->d_w32,
                      c->d_wsum, c->d_wbf16, c->d_wfp8, c->d_wfp8_scale, bake,
-                     c->cfg.precision == ANE_PRECISION_FP16, st);
+                     c->cfg.precision == ANE_PRECISION_FP16, c->d_work, clk, st);
   ANE_CHECK_HIP(hipGetLastError());
   return ANE_OK;
 }
@@ -1283,34 +1235,34 @@ extern "C" int ane_ddgi_trace(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddg
   hipStream_t st = S(stream);
   const bool bake = (fk.flags & ANE_FLAG_BAKE) != 0;
   const int nprobes = fk.layer_count * c->g.nx * c->g.nz;
-  ANE_TRY(c->timers[kStSetup].begin(st));
-  ANE_TRY(do_frame_setup(c, fk, bake, st));
-  fill_u32(c->d_work, 0u, kTraceWorkWords, st);
+  ClockArg clk;
+  ANE_TRY(clock_of(c, kClkTrace, st, &clk));
+  ANE_TRY(do_frame_setup(c, fk, bake, st, clk));
+  count_stage(c, clk, kStSetup);
   if (c->counting) fill_u32(reinterpret_cast<uint32_t*>(c->d_stats), 0u, 8, st);
-  ANE_TRY(c->timers[kStSetup].end(st));
   TraceArgs a = trace_args(c, s, fk);
   a.work = c->d_work;
+  a.clk = clk;
   if (sun_grid_wanted(c)) {
     bool use = false;
-    ANE_TRY(c->sgc.update(s->view, s->ntri, s, s->version, a.sun, a.nrays, st, &use, &c->timers[kStSunGrid]));
+    const uint64_t builds = c->sgc.builds;
+    ANE_TRY(c->sgc.update(s->view, s->ntri, s, s->version, a.sun, a.nrays, st, &use, clk, kTraceSunGrid));
+    if (c->sgc.builds != builds) count_stage(c, clk, kStSunGrid);
     if (use) a.sg = c->sgc.view();
   }
   // primary rays in one persistent launch (with the shadow rays of their hits
   // unless a sun grid is in use), then the sun-grid shadow rays
-  ANE_TRY(c->timers[kStTrace].begin(st));
   launch_trace(a, false, false, c->counting, st);
-  ANE_TRY(c->timers[kStTrace].end(st));
+  count_stage(c, clk, kStTrace);
   if (a.sg.list) {
-    ANE_TRY(c->timers[kStShadow].begin(st));
     launch_probe_shadow_grid(a, c->counting, st);
-    ANE_TRY(c->timers[kStShadow].end(st));
+    count_stage(c, clk, kStShadow);
   }
-  ANE_TRY(c->timers[kStShade].begin(st));
   launch_shade(s->view, c->g, fk, c->d_probe_org, c->d_hits, c->d_shadow,
                c->d_atlas[c->cur], c->cfg.precision, c->d_rad, c->d_rad_scale, nprobes,
-               a.probe_base, st);
+               a.probe_base, clk, st);
   ANE_CHECK_HIP(hipGetLastError());
-  ANE_TRY(c->timers[kStShade].end(st));
+  count_stage(c, clk, kStShade);
   c->rad_begin = fk.layer_begin;
   c->rad_count = fk.layer_count;
   c->rad_bake = bake;
@@ -1334,12 +1286,13 @@ extern "C" int ane_ddgi_convolve(ane_ddgi_ctx* c, const ane_ddgi_frame* f, void*
   hipStream_t st = S(stream);
   const int nprobes = fk.layer_count * c->g.nx * c->g.nz;
   const int probe_base = fk.layer_begin * c->g.nx * c->g.nz;
-  ANE_TRY(c->timers[kStConv].begin(st));
+  ClockArg clk;
+  ANE_TRY(clock_of(c, kClkConv, st, &clk));
   launch_convolve(c->g, fk, c->cfg.precision, c->d_rad, c->d_rad_scale, c->d_w32, c->d_wsum,
                   c->d_wbf16, c->d_wfp8, c->d_wfp8_scale, c->d_atlas[c->cur], nprobes, probe_base,
-                  bake, st);
+                  bake, clk, st);
   ANE_CHECK_HIP(hipGetLastError());
-  ANE_TRY(c->timers[kStConv].end(st));
+  count_stage(c, clk, kStConv);
   return ANE_OK;
 }
 
@@ -1355,7 +1308,7 @@ namespace ane {
 // updates it in place from each new capture (kernel arguments change with the
 // frame; the node structure changes only with the layer range or the bake flag,
 // which re-instantiates it).  Validation and allocation happen before the
-// capture; stage timers record nothing meanwhile, so the graph holds kernel
+// capture; the stage clocks stamp nothing meanwhile, and the graph holds kernel
 // nodes only (counters are cleared by a fill kernel).  Counting contexts update
 // directly.
 // The front of an update for the request loop's fused stages: frame setup, sun
@@ -1373,7 +1326,6 @@ int ddgi_update_front(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame*
   const bool bake = (fk.flags & ANE_FLAG_BAKE) != 0;
   const int nprobes = fk.layer_count * c->g.nx * c->g.nz;
   ANE_TRY(do_frame_setup(c, fk, bake, st));
-  fill_u32(c->d_work, 0u, kTraceWorkWords, st);
   if (c->counting) fill_u32(reinterpret_cast<uint32_t*>(c->d_stats), 0u, 8, st);
   TraceArgs a = trace_args(c, s, fk);
   a.work = c->d_work;
@@ -1431,16 +1383,13 @@ int ddgi_update_graph(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame*
   ANE_TRY(ensure_spill(c, s->depth));
   if (sun_grid_wanted(c)) ANE_TRY(c->sgc.alloc(s->ntri));  // allocation outside the capture
   if (c->counting) return ane_ddgi_update(c, s, f, st);
-  for (auto& t : c->timers) t.off = true;
   hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) {
-    for (auto& t : c->timers) t.off = false;
     return fail(ANE_ERR_DEVICE, "hipStreamBeginCapture: %s", hipGetErrorString(e));
   }
   const int r = ane_ddgi_update(c, s, f, st);
   hipGraph_t g = nullptr;
   e = hipStreamEndCapture(st, &g);
-  for (auto& t : c->timers) t.off = false;
   if (r != ANE_OK || e != hipSuccess || !g) {
     if (g) (void)hipGraphDestroy(g);
     return r != ANE_OK ? r : fail(ANE_ERR_DEVICE, "hipStreamEndCapture: %s", hipGetErrorString(e));
@@ -1475,11 +1424,12 @@ extern "C" int ane_ddgi_translate(ane_ddgi_ctx* c, const float* cam, int32_t* sh
   c->last_cell[0] = ix;
   c->last_cell[1] = iz;
   hipStream_t st = S(stream);
-  ANE_TRY(c->timers[kStTrans].begin(st));
+  ClockArg clk;
+  ANE_TRY(clock_of(c, kClkTrans, st, &clk));
   launch_translate(c->g, reinterpret_cast<const float4*>(c->d_atlas[c->cur]),
-                   reinterpret_cast<float4*>(c->d_atlas[1 - c->cur]), dx, dz, st);
+                   reinterpret_cast<float4*>(c->d_atlas[1 - c->cur]), dx, dz, clk, st);
   ANE_CHECK_HIP(hipGetLastError());
-  ANE_TRY(c->timers[kStTrans].end(st));
+  count_stage(c, clk, kStTrans);
   c->cur = 1 - c->cur;
   if (shifted) *shifted = 1;
   return ANE_OK;
@@ -1827,19 +1777,42 @@ extern "C" int ane_ddgi_set_counting(ane_ddgi_ctx* c, int32_t enable)
   return ANE_OK;
 }
 
+// Waits for the context's queued calls and reads the stage clocks, the last calls' stamps
+// folded into the sums (on the host copy).
+static int read_clocks(ane_ddgi_ctx* c, StageClock* out)
+{
+  ANE_CHECK_HIP(hipDeviceSynchronize());
+  ANE_CHECK_HIP(hipMemcpy(out, c->d_clock, kClocks * sizeof(StageClock), hipMemcpyDeviceToHost));
+  for (int k = 0; k < kClocks; ++k) {
+    StageSet& p = out[k].set[c->clock_set[k]];
+    unsigned long long end = 0;
+    for (int i = 0; i < kClockSlots; ++i) end = std::max(end, p.end[i * kClockSlotStride]);
+    for (int i = 0; i < kClockStages; ++i) {
+      if (!p.begin[i]) continue;
+      out[k].last[i] = stage_ticks(p.begin, i, end);
+      out[k].sum[i] += out[k].last[i];
+    }
+    p = StageSet{};
+  }
+  return ANE_OK;
+}
+
 extern "C" int ane_ddgi_stats_get(const ane_ddgi_ctx* cc, ane_ddgi_stats* out)
 {
   if (!cc || !out) return fail(ANE_ERR_INVALID_ARG, "NULL argument");
   ane_ddgi_ctx* c = const_cast<ane_ddgi_ctx*>(cc);
   ane_ddgi_stats s = c->stats;
   s.device_bytes = ctx_device_bytes(c);
-  for (int k = 0; k < kStages; ++k) {
-    StageTimer& t = c->timers[k];
-    ANE_TRY(t.harvest_all());
-    s.last_ms[k] = t.last_ms;
-    s.mean_ms[k] = t.count ? (float)(t.acc_ms / (double)t.count) : 0.0f;
-    s.calls[k] = t.count;
-  }
+  StageClock clocks[kClocks];
+  ANE_TRY(read_clocks(c, clocks));
+  for (int k = 0; k < kClocks; ++k)
+    for (int i = 0; i < kClockStages; ++i) {
+      const int stage = kClkStage[k][i];
+      if (stage < 0) continue;
+      s.last_ms[stage] = (float)((double)clocks[k].last[i] / c->clock_khz);
+      s.calls[stage] = c->calls[stage];
+      s.mean_ms[stage] = c->calls[stage] ? (float)((double)clocks[k].sum[i] / c->clock_khz / (double)c->calls[stage]) : 0.0f;
+    }
   (void)hipGetLastError();
   if (c->counting) {
     unsigned long long v[4] = {0, 0, 0, 0};
@@ -1880,10 +1853,11 @@ static int take_faults(ane_ddgi_ctx* c, hipStream_t st, uint32_t* probe, uint32_
 extern "C" int ane_ddgi_stats_reset(ane_ddgi_ctx* c)
 {
   if (!c) return fail(ANE_ERR_INVALID_ARG, "NULL context");
-  for (auto& t : c->timers) {
-    ANE_TRY(t.harvest_all());
-    t.reset();
-  }
+  StageClock clocks[kClocks];
+  ANE_TRY(read_clocks(c, clocks));
+  for (int k = 0; k < kClocks; ++k) std::fill(clocks[k].sum, clocks[k].sum + kClockStages, 0ull);
+  std::fill(c->calls, c->calls + kStages, 0ull);
+  ANE_CHECK_HIP(hipMemcpy(c->d_clock, clocks, sizeof(clocks), hipMemcpyHostToDevice));
   uint32_t p = 0, m = 0;
   return take_faults(c, nullptr, &p, &m);
 }

@@ -66,8 +66,9 @@ static constexpr int kKC = 32;
 
 __global__ __launch_bounds__(256) void k_conv_fp32(GridK g, const float* rad, const float* w32,
                                                    const float* wsum, float4* atlas, int nprobes,
-                                                   int probe_base, int32_t bake)
+                                                   int probe_base, int32_t bake, ClockArg clk)
 {
+  clock_begin(clk, 0);
   __shared__ float Ws[kKC][64];
   __shared__ float Ls[kPB][3 * kKC + 1];
   const int n = g.rays;
@@ -108,6 +109,7 @@ __global__ __launch_bounds__(256) void k_conv_fp32(GridK g, const float* rad, co
     }
     __syncthreads();
   }
+  if (blockIdx.x == 0 && threadIdx.x >= 192) clock_fold(clk);
   const int pq = p0 + pl;
   if (pq >= nprobes) return;
   const int q = probe_base + pq;
@@ -119,6 +121,7 @@ __global__ __launch_bounds__(256) void k_conv_fp32(GridK g, const float* rad, co
     const float4 old = atlas[ti];
     atlas[ti] = blend_texel(old, acc[j][0], acc[j][1], acc[j][2], wsum[t], h, bake != 0);
   }
+  clock_end(clk);
 }
 
 // ---------------------------------------------------------------------------
@@ -326,10 +329,13 @@ __global__ __launch_bounds__(64 * kConvWaves) void k_conv_mfma(GridK g, const vo
                                                               const float* rad_scale, const void* wq,
                                                               const float* wscale, const float* wsum,
                                                               float4* atlas, int nprobes,
-                                                              int probe_base, int32_t bake)
+                                                              int probe_base, int32_t bake, ClockArg clk)
 {
+  clock_begin(clk, 0);
   __shared__ ConvPart part;
   conv_block<PREC>(g, rad, rad_scale, wq, wscale, wsum, atlas, nprobes, probe_base, bake, blockIdx.x, part);
+  clock_end(clk);
+  if (blockIdx.x == 0 && threadIdx.x >= 64 * (kConvWaves - 1)) clock_fold(clk);
 }
 
 // The convolutions of many updates in one launch (the request loop's fused
@@ -551,9 +557,13 @@ __device__ __forceinline__ void conv_stream_block(const GridK& g, const void* ra
 template <int PREC, int D>
 __global__ __launch_bounds__(256) void k_conv_stream(GridK g, const void* rad, const float* rad_scale,
                                                      const void* wq, const float* wscale, const float* wsum,
-                                                     float4* atlas, int nprobes, int probe_base, int32_t bake)
+                                                     float4* atlas, int nprobes, int probe_base, int32_t bake,
+                                                     ClockArg clk)
 {
+  clock_begin(clk, 0);
   conv_stream_block<PREC, D>(g, rad, rad_scale, wq, wscale, wsum, atlas, nprobes, probe_base, bake, blockIdx.x);
+  clock_end(clk);
+  if (blockIdx.x == 0 && threadIdx.x >= 192) clock_fold(clk);
 }
 
 // The streaming convolutions of many updates in one launch (the request loop's
@@ -596,12 +606,12 @@ template <int PREC, int D>
 static void launch_stream_d(int S, bool jobs, const GridK& g, const void* rad, const float* rad_scale,
                             const void* wq, const float* wscale, const float* wsum, float4* atlas, int num_probes,
                             int probe_base, bool bake, const ConvJob* job_table, int njobs, int blocks, size_t lds,
-                            hipStream_t s)
+                            const ClockArg& clk, hipStream_t s)
 {
   if constexpr (D > 1) {
     if (S % D != 0) {
       launch_stream_d<PREC, D / 2>(S, jobs, g, rad, rad_scale, wq, wscale, wsum, atlas, num_probes, probe_base,
-                                   bake, job_table, njobs, blocks, lds, s);
+                                   bake, job_table, njobs, blocks, lds, clk, s);
       return;
     }
   }
@@ -617,7 +627,7 @@ static void launch_stream_d(int S, bool jobs, const GridK& g, const void* rad, c
     hipLaunchKernelGGL((k_conv_stream_jobs<PREC, D>), dim3((unsigned)blocks), dim3(256), lds, s, job_table, njobs);
   } else {
     hipLaunchKernelGGL((k_conv_stream<PREC, D>), dim3((unsigned)blocks), dim3(256), lds, s, g, rad, rad_scale, wq,
-                       wscale, wsum, atlas, num_probes, probe_base, (int32_t)bake);
+                       wscale, wsum, atlas, num_probes, probe_base, (int32_t)bake, clk);
   }
 }
 
@@ -625,31 +635,32 @@ template <int PREC>
 static void launch_conv_stream(int S, bool jobs, const GridK& g, const void* rad, const float* rad_scale,
                                const void* wq, const float* wscale, const float* wsum, float4* atlas,
                                int num_probes, int probe_base, bool bake, const ConvJob* job_table, int njobs,
-                               int blocks, size_t lds, hipStream_t s)
+                               int blocks, size_t lds, const ClockArg& clk, hipStream_t s)
 {
   constexpr int D = PREC == ANE_PRECISION_FP32 ? ANE_CONV_DEPTH32
                     : PREC == ANE_PRECISION_FP8 ? ANE_CONV_DEPTH8 : ANE_CONV_DEPTH16;
   launch_stream_d<PREC, D>(S, jobs, g, rad, rad_scale, wq, wscale, wsum, atlas, num_probes, probe_base, bake,
-                           job_table, njobs, blocks, lds, s);
+                           job_table, njobs, blocks, lds, clk, s);
 }
 
 static void launch_conv_stream_any(int precision, int S, bool jobs, const GridK& g, const void* rad,
                                    const float* rad_scale, const void* wq, const float* wscale, const float* wsum,
                                    float4* atlas, int num_probes, int probe_base, bool bake,
-                                   const ConvJob* job_table, int njobs, int blocks, size_t lds, hipStream_t s)
+                                   const ConvJob* job_table, int njobs, int blocks, size_t lds,
+                                   const ClockArg& clk, hipStream_t s)
 {
   if (precision == ANE_PRECISION_FP32)
     launch_conv_stream<ANE_PRECISION_FP32>(S, jobs, g, rad, rad_scale, wq, wscale, wsum, atlas, num_probes,
-                                           probe_base, bake, job_table, njobs, blocks, lds, s);
+                                           probe_base, bake, job_table, njobs, blocks, lds, clk, s);
   else if (precision == ANE_PRECISION_FP16)
     launch_conv_stream<ANE_PRECISION_FP16>(S, jobs, g, rad, rad_scale, wq, wscale, wsum, atlas, num_probes,
-                                           probe_base, bake, job_table, njobs, blocks, lds, s);
+                                           probe_base, bake, job_table, njobs, blocks, lds, clk, s);
   else if (precision == ANE_PRECISION_BF16)
     launch_conv_stream<ANE_PRECISION_BF16>(S, jobs, g, rad, rad_scale, wq, wscale, wsum, atlas, num_probes,
-                                           probe_base, bake, job_table, njobs, blocks, lds, s);
+                                           probe_base, bake, job_table, njobs, blocks, lds, clk, s);
   else
     launch_conv_stream<ANE_PRECISION_FP8>(S, jobs, g, rad, rad_scale, wq, wscale, wsum, atlas, num_probes,
-                                          probe_base, bake, job_table, njobs, blocks, lds, s);
+                                          probe_base, bake, job_table, njobs, blocks, lds, clk, s);
 }
 
 int conv_job_blocks(int precision, int rays, int num_probes)
@@ -664,7 +675,8 @@ void launch_conv_jobs(int precision, const ConvJob* jobs, int njobs, int total_b
   if (njobs <= 0 || total_blocks <= 0) return;
   if (stream) {
     launch_conv_stream_any(precision, rays_gcd / 32, true, GridK{}, nullptr, nullptr, nullptr, nullptr, nullptr,
-                           nullptr, 0, 0, false, jobs, njobs, total_blocks, conv_stream_lds(precision, max_rays), s);
+                           nullptr, 0, 0, false, jobs, njobs, total_blocks, conv_stream_lds(precision, max_rays),
+                           ClockArg{}, s);
     return;
   }
   const dim3 grid((unsigned)total_blocks), block(64 * kConvWaves);
@@ -681,7 +693,7 @@ void launch_conv_jobs(int precision, const ConvJob* jobs, int njobs, int total_b
 void launch_convolve(const GridK& g, const FrameK& f, int precision, const void* rad,
                      const float* rad_scale, const float* w32, const float* wsum,
                      const uint16_t* wbf16, const uint8_t* wfp8, const float* wfp8_scale,
-                     float* atlas, int num_probes, int probe_base, bool bake, hipStream_t s)
+                     float* atlas, int num_probes, int probe_base, bool bake, const ClockArg& clk, hipStream_t s)
 {
   (void)f;
   if (num_probes <= 0) return;
@@ -692,31 +704,31 @@ void launch_convolve(const GridK& g, const FrameK& f, int precision, const void*
                      : precision == ANE_PRECISION_FP8 ? (const void*)wfp8 : (const void*)wbf16;
     const int blocks = (num_probes + kStreamProbes - 1) / kStreamProbes;
     launch_conv_stream_any(precision, g.rays / 32, false, g, rad, rad_scale, wq, wfp8_scale, wsum, a4, num_probes,
-                           probe_base, bake, nullptr, 0, blocks, conv_stream_lds(precision, g.rays), s);
+                           probe_base, bake, nullptr, 0, blocks, conv_stream_lds(precision, g.rays), clk, s);
     return;
   }
   if (precision == ANE_PRECISION_FP32) {
     if (g.rays % 32 != 0) {  // the register-tiled kernel takes any ray count
       const unsigned b32 = (unsigned)((num_probes + kPB - 1) / kPB);
       hipLaunchKernelGGL(k_conv_fp32, dim3(b32), dim3(256), 0, s, g, (const float*)rad, w32, wsum,
-                         a4, num_probes, probe_base, (int32_t)bake);
+                         a4, num_probes, probe_base, (int32_t)bake, clk);
       return;
     }
     hipLaunchKernelGGL(k_conv_mfma<ANE_PRECISION_FP32>, dim3(blocks), dim3(64 * kConvWaves), 0, s, g, rad,
                        rad_scale, (const void*)w32, wfp8_scale, wsum, a4, num_probes, probe_base,
-                       (int32_t)bake);
+                       (int32_t)bake, clk);
   } else if (precision == ANE_PRECISION_FP16) {
     hipLaunchKernelGGL(k_conv_mfma<ANE_PRECISION_FP16>, dim3(blocks), dim3(64 * kConvWaves), 0, s, g,
                        rad, rad_scale, (const void*)wbf16, wfp8_scale, wsum, a4,
-                       num_probes, probe_base, (int32_t)bake);
+                       num_probes, probe_base, (int32_t)bake, clk);
   } else if (precision == ANE_PRECISION_BF16) {
     hipLaunchKernelGGL(k_conv_mfma<ANE_PRECISION_BF16>, dim3(blocks), dim3(64 * kConvWaves), 0, s, g,
                        rad, rad_scale, (const void*)wbf16, wfp8_scale, wsum, a4,
-                       num_probes, probe_base, (int32_t)bake);
+                       num_probes, probe_base, (int32_t)bake, clk);
   } else {
     hipLaunchKernelGGL(k_conv_mfma<ANE_PRECISION_FP8>, dim3(blocks), dim3(64 * kConvWaves), 0, s, g,
                        rad, rad_scale, (const void*)wfp8, wfp8_scale, wsum, a4, num_probes,
-                       probe_base, (int32_t)bake);
+                       probe_base, (int32_t)bake, clk);
   }
 }
 

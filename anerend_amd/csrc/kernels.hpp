@@ -64,6 +64,78 @@ void launch_fit(float4* tris, int n, NodeBuild* nodes, float* node_box, uint4* q
 // cross_kids[k]: the children of crossing node cross[k], for the total crossing
 // nodes of the fit plan (once per build)
 void launch_cross_kids(const int32_t* cross, const int4* topo, int total, int2* kids, hipStream_t s);
+// Stage times, taken by the kernels themselves from the device's wall clock: the first
+// block of a stage's first kernel stamps its begin, and a stage ends where the next one
+// of its call begins; the waves of a call's last kernel stamp its end (a maximum, over
+// kClockSlots words in cache lines of their own).  The stamps of a call go to one of two
+// sets; the next call of the same kind adds up the other set and clears it, so nothing
+// but kernel stores is queued.  (hipEvent pairs around each stage put about 10 us between
+// the kernels of an update: 50 of the 157 us of one layer of a small room.)
+static constexpr int kClockStages = 5;
+static constexpr int kClockSlots = 16;
+static constexpr int kClockSlotStride = 8;
+struct StageSet {
+  unsigned long long begin[8];  // [kClockStages] in launch order; 0: the stage did not run
+  unsigned long long end[kClockSlots * kClockSlotStride];
+};
+struct StageClock {
+  StageSet set[2];
+  unsigned long long sum[kClockStages], last[kClockStages];  // clock ticks
+};
+// the stages of a call of each kind, in launch order (trace: ane_ddgi_trace)
+enum { kTraceSetup = 0, kTraceSunGrid, kTraceRays, kTraceShadow, kTraceShade };
+struct ClockArg {
+  StageClock* c;  // null: no stamps
+  int32_t set;    // the call's stamp set
+};
+
+__device__ __forceinline__ void clock_begin(const ClockArg& k, int stage)
+{
+  if (k.c && blockIdx.x == 0 && threadIdx.x == 0) k.c->set[k.set].begin[stage] = wall_clock64();
+}
+// by every wave whose end can be the kernel's
+__device__ __forceinline__ void clock_end(const ClockArg& k)
+{
+  if (k.c && (threadIdx.x & 63) == 0)
+    atomicMax(&k.c->set[k.set].end[(blockIdx.x % kClockSlots) * kClockSlotStride],
+              (unsigned long long)wall_clock64());
+}
+// the ticks of stage i of a call that ended at `end`, 0 if it did not run
+__host__ __device__ __forceinline__ unsigned long long stage_ticks(const unsigned long long* begin, int i,
+                                                                   unsigned long long end)
+{
+  unsigned long long next = end;
+  for (int j = kClockStages - 1; j > i; --j)
+    if (begin[j]) next = begin[j];
+  return begin[i] && next > begin[i] ? next - begin[i] : 0ull;
+}
+// the previous call's set into the sums (one whole wave of the call's launches; the
+// previous call's kernels have completed)
+__device__ __forceinline__ void clock_fold(const ClockArg& k)
+{
+  if (!k.c) return;
+  StageSet& p = k.c->set[k.set ^ 1];
+  const int lane = threadIdx.x & 63;
+  unsigned long long e = lane < kClockSlots ? p.end[lane * kClockSlotStride] : 0ull;
+#pragma unroll
+  for (int d = kClockSlots / 2; d >= 1; d >>= 1) {
+    const unsigned long long o = __shfl_xor(e, d, 64);
+    e = o > e ? o : e;
+  }
+  if (lane == 0) {
+    unsigned long long b[kClockStages];
+    for (int i = 0; i < kClockStages; ++i) b[i] = p.begin[i];
+    for (int i = 0; i < kClockStages; ++i) {
+      if (!b[i]) continue;
+      const unsigned long long t = stage_ticks(b, i, e);
+      k.c->sum[i] += t;
+      k.c->last[i] = t;
+      p.begin[i] = 0ull;
+    }
+  }
+  if (lane < kClockSlots) p.end[lane * kClockSlotStride] = 0ull;
+}
+
 // trace.hip
 // Sun grid of the probe shadow rays (sungrid.hip): projected along the sun
 // direction, cell (cx, cy) of a point = (sun_cell(X, x0, icw, gx), sun_cell(Y, y0, ich, gy))
@@ -125,7 +197,7 @@ void launch_anyhit_grid(const float* orig, const float* dirs, int64_t n, const S
 int64_t sun_grid_scratch_words(int32_t ntri);
 void launch_sun_grid_build(const SceneK& sc, const SunGridParams& g, SunGridParams* d_params, uint32_t* acc,
                            uint32_t* cnt, uint32_t* cur, uint32_t* list, uint32_t cap, uint32_t* scan_scratch,
-                           float* est, hipStream_t s);
+                           float* est, const ClockArg& clk, int stage, hipStream_t s);
 // probe traces can take a sun grid (k_probe_shadow_grid runs their shadow rays)
 bool trace_grid_supported();
 
@@ -168,6 +240,7 @@ struct TraceArgs {
   const float* ray_tmax;   // caller rays: per-ray t_max (null: t_max for every ray)
   SunGridK sg;             // probe rays: candidates of the shadow rays (list null: traversal)
   const uint32_t* skip_if_set; // caller rays: the launch does nothing when *skip_if_set != 0
+  ClockArg clk;            // probe rays: stage stamps
 };
 
 // A probe update's shading and convolution as job records, so that the request
@@ -222,7 +295,8 @@ int trace_block_size();
 void launch_trace(const TraceArgs& a, bool any_hit, bool rays, bool count, hipStream_t s);
 void launch_frame_setup(const GridK& g, const FrameK& f, const float* base_dirs,
                         const uint32_t* order, float* dirs, float4* dirpre, float4* probe_org, float* w32, float* wsum, uint16_t* wbf16,
-                        uint8_t* wfp8, float* wfp8_scale, bool bake, bool f16, hipStream_t s);
+                        uint8_t* wfp8, float* wfp8_scale, bool bake, bool f16, uint32_t* work, const ClockArg& clk,
+                        hipStream_t s);
 struct RayDiv {
   uint64_t magic;
   int32_t shift;
@@ -232,7 +306,7 @@ RayDiv ray_div_magic(int64_t nrays, int n);
 void launch_shade(const SceneK& sc, const GridK& g, const FrameK& f, const float4* probe_org,
                   const ane_hit* hits,
                   const uint8_t* shadow, const float* atlas, int precision, void* rad,
-                  float* rad_scale, int num_probes, int probe_base, hipStream_t s);
+                  float* rad_scale, int num_probes, int probe_base, const ClockArg& clk, hipStream_t s);
 
 // conv.hip
 // FP64 validation of a convolution (see conv.hip): out_max (the bits of a
@@ -244,7 +318,7 @@ void launch_conv_err64(const GridK& g, const float* dirs, const double* texel_di
 void launch_convolve(const GridK& g, const FrameK& f, int precision, const void* rad,
                      const float* rad_scale, const float* w32, const float* wsum,
                      const uint16_t* wbf16, const uint8_t* wfp8, const float* wfp8_scale,
-                     float* atlas, int num_probes, int probe_base, bool bake, hipStream_t s);
+                     float* atlas, int num_probes, int probe_base, bool bake, const ClockArg& clk, hipStream_t s);
 void launch_quantize(int precision, const float* src, void* dst, float* scale, int num_probes,
                      int n, hipStream_t s);
 void launch_dequantize(int precision, const void* src, const float* scale, float* dst,
@@ -280,7 +354,7 @@ void launch_mirror_shade(const SceneK& sc, const GridK& g, const FrameK& f, cons
                          int64_t n, float* out, hipStream_t s);
 
 // translate.hip
-void launch_translate(const GridK& g, const float4* src, float4* dst, int dx, int dz,
+void launch_translate(const GridK& g, const float4* src, float4* dst, int dx, int dz, const ClockArg& clk,
                       hipStream_t s);
 // atlas <-> RGBA16F (binary16 per channel, round to nearest even), texels float4 <-> uint2
 void launch_atlas_to_half(const float4* src, uint2* dst, int64_t texels, hipStream_t s);

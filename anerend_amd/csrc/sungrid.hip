@@ -52,8 +52,9 @@ static constexpr int kBoundBlocks = 256;
 // per block, [6][kBoundBlocks]: min X, min Y, max X, max Y, max |coordinate|,
 // non-finite seen (ordered encodings); k_sun_params reduces the blocks
 __global__ __launch_bounds__(256) void k_sun_bounds(const float4* tris, int32_t ntri, SunGridParams g,
-                                                    uint32_t* part)
+                                                    uint32_t* part, ClockArg clk, int stage)
 {
+  clock_begin(clk, stage);
   __shared__ uint32_t red[6][256];
   uint32_t mnx = 0xFFFFFFFFu, mny = 0xFFFFFFFFu, mxx = 0u, mxy = 0u, mr = 0u, bad = 0u;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (int64_t)ntri * 3;
@@ -467,11 +468,11 @@ void sun_grid_setup(SunGridParams& g, const float* dir3, int gx, int gy)
 
 void launch_sun_grid_build(const SceneK& sc, const SunGridParams& g, SunGridParams* d_params, uint32_t* acc,
                            uint32_t* cnt, uint32_t* cur, uint32_t* list, uint32_t cap, uint32_t* scan_scratch,
-                           float* est, hipStream_t s)
+                           float* est, const ClockArg& clk, int stage, hipStream_t s)
 {
   const int64_t ncell = (int64_t)g.gx * g.gy;
+  hipLaunchKernelGGL(k_sun_bounds, dim3(kBoundBlocks), dim3(256), 0, s, sc.tris, sc.ntri, g, acc, clk, stage);
   fill_u32(cnt, 0u, ncell + 1, s);
-  hipLaunchKernelGGL(k_sun_bounds, dim3(kBoundBlocks), dim3(256), 0, s, sc.tris, sc.ntri, g, acc);
   hipLaunchKernelGGL(k_sun_params, dim3(1), dim3(kBoundBlocks), 0, s, g, (const uint32_t*)acc, d_params);
   const unsigned tb = (unsigned)((sc.ntri + 255) / 256);
   uint16_t* tab = reinterpret_cast<uint16_t*>(est + 2 * (int64_t)tb);  // after the estimate partials

@@ -139,9 +139,14 @@ __global__ __launch_bounds__(256) void k_frame_setup(GridK g, FrameK f, Mat3 rot
                                                      float* dirs, float4* dirpre,
                                                      float4* probe_org, float* w32, float* wsum,
                                                      uint16_t* wbf16, uint8_t* wfp8,
-                                                     float* wfp8_scale, int32_t bake, int32_t f16)
+                                                     float* wfp8_scale, int32_t bake, int32_t f16, uint32_t* work,
+                                                     ClockArg clk)
 {
   const int t = blockIdx.x;  // texel 0..63
+  clock_begin(clk, kTraceSetup);
+  if (t == 2 && threadIdx.x < 64) clock_fold(clk);
+  if (t == 3)  // the claim counters of the traversal that follows
+    for (int i = threadIdx.x; i < kTraceWorkWords; i += blockDim.x) work[i] = 0u;
   // probe origins of the whole grid (rgen:60-84), read by ray generation and shading
   const int P = g.nx * g.ny * g.nz;
   for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < P; q += gridDim.x * blockDim.x) {
@@ -236,13 +241,15 @@ __global__ __launch_bounds__(256) void k_frame_setup(GridK g, FrameK f, Mat3 rot
 
 void launch_frame_setup(const GridK& g, const FrameK& f, const float* base_dirs,
                         const uint32_t* order, float* dirs, float4* dirpre, float4* probe_org, float* w32, float* wsum, uint16_t* wbf16,
-                        uint8_t* wfp8, float* wfp8_scale, bool bake, bool f16, hipStream_t s)
+                        uint8_t* wfp8, float* wfp8_scale, bool bake, bool f16, uint32_t* work, const ClockArg& clk,
+                        hipStream_t s)
 {
   Mat3 rot;
   for (int i = 0; i < 16; ++i) rot.m[i] = f.rot[i];
   const f3 sun = normalize(mk(-f.light_dir[0], -f.light_dir[1], -f.light_dir[2]));
   hipLaunchKernelGGL(k_frame_setup, dim3(64), dim3(256), 0, s, g, f, rot, sun, base_dirs, order,
-                     dirs, dirpre, probe_org, w32, wsum, wbf16, wfp8, wfp8_scale, (int32_t)bake, (int32_t)f16);
+                     dirs, dirpre, probe_org, w32, wsum, wbf16, wfp8, wfp8_scale, (int32_t)bake, (int32_t)f16,
+                     work, clk);
 }
 
 // Division of a ray index x < nrays by n as (x * m) >> k, m = ceil(2^k / n).
@@ -318,6 +325,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
   const bool sgrid = !RAYS && a.sg.list != nullptr && a.sg.params->valid != 0u;
   __shared__ int32_t stk[kSS][kTB];
   if (RAYS && a.skip_if_set && *a.skip_if_set != 0u) return;  // a sun grid answered these rays
+  if (!RAYS) clock_begin(a.clk, kTraceRays);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int gl = blockIdx.x * kTB + tid;
@@ -746,6 +754,7 @@ __device__ __forceinline__ void probe_shadow_group(const TraceArgs& a, int64_t f
 template <bool COUNT>
 __global__ __launch_bounds__(kShadowTB) void k_probe_shadow_grid(TraceArgs a)
 {
+  clock_begin(a.clk, kTraceShadow);
   const SunGridParams* gq = a.sg.params;
   if (gq->valid == 0u) return;  // no grid in use: the traversal ran the shadow rays
   probe_shadow_group<COUNT>(a, (int64_t)blockIdx.x * kShadowTB);
@@ -1192,14 +1201,16 @@ __device__ __forceinline__ void shade_probe(const SceneK& sc, const GridK& g, co
 template <int PREC, int TB>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(ANE_SHADE_WAVES))) void k_shade(SceneK sc, GridK g, FrameK f, const float4* probe_org,
                                               const ane_hit* hits, const uint8_t* shadow, const float4* atlas, void* rad,
-                                              float* rad_scale, int probe_base)
+                                              float* rad_scale, int probe_base, ClockArg clk)
 {
+  clock_begin(clk, kTraceShade);
   extern __shared__ float sL[];  // FP8: [3][N] staged radiance, then [3][N / 32] block factors
   __shared__ float red[TB];
   __shared__ uint16_t lst[4096];
   __shared__ uint32_t cnt[3], cur[3];
   shade_probe<PREC, TB>(sc, g, f, probe_org, hits, shadow, atlas, rad, rad_scale, probe_base, blockIdx.x, sL,
                         red, lst, cnt, cur);
+  if (threadIdx.x < 64) clock_end(clk);
 }
 
 // The probes of many updates in one launch (the request loop's fused stage): block
@@ -1246,36 +1257,36 @@ static void shade_launch(const SceneK& sc, const GridK& g, const FrameK& f, cons
                          const ane_hit* hits,
                          const uint8_t* shadow,
                          const float4* a4, int precision, void* rad, float* rad_scale,
-                         int num_probes, int probe_base, hipStream_t s)
+                         int num_probes, int probe_base, const ClockArg& clk, hipStream_t s)
 {
   if (precision == ANE_PRECISION_FP32)
     hipLaunchKernelGGL((k_shade<ANE_PRECISION_FP32, TB>), dim3(num_probes), dim3(TB), 0, s, sc, g, f,
-                       probe_org, hits, shadow, a4, rad, rad_scale, probe_base);
+                       probe_org, hits, shadow, a4, rad, rad_scale, probe_base, clk);
   else if (precision == ANE_PRECISION_FP16)
     hipLaunchKernelGGL((k_shade<ANE_PRECISION_FP16, TB>), dim3(num_probes), dim3(TB), 0, s, sc, g, f,
-                       probe_org, hits, shadow, a4, rad, rad_scale, probe_base);
+                       probe_org, hits, shadow, a4, rad, rad_scale, probe_base, clk);
   else if (precision == ANE_PRECISION_BF16)
     hipLaunchKernelGGL((k_shade<ANE_PRECISION_BF16, TB>), dim3(num_probes), dim3(TB), 0, s, sc, g, f,
-                       probe_org, hits, shadow, a4, rad, rad_scale, probe_base);
+                       probe_org, hits, shadow, a4, rad, rad_scale, probe_base, clk);
   else
     hipLaunchKernelGGL((k_shade<ANE_PRECISION_FP8, TB>), dim3(num_probes), dim3(TB),
                        fp8_shade_smem(g.rays), s, sc, g, f, probe_org, hits, shadow, a4, rad,
-                       rad_scale, probe_base);
+                       rad_scale, probe_base, clk);
 }
 
 void launch_shade(const SceneK& sc, const GridK& g, const FrameK& f, const float4* probe_org,
                   const ane_hit* hits,
                   const uint8_t* shadow, const float* atlas, int precision, void* rad,
-                  float* rad_scale, int num_probes, int probe_base, hipStream_t s)
+                  float* rad_scale, int num_probes, int probe_base, const ClockArg& clk, hipStream_t s)
 {
   if (num_probes <= 0) return;
   const float4* a4 = reinterpret_cast<const float4*>(atlas);
   if (g.rays >= 512)
     shade_launch<ANE_SHADE_TB>(sc, g, f, probe_org, hits, shadow, a4, precision, rad, rad_scale,
-                               num_probes, probe_base, s);
+                               num_probes, probe_base, clk, s);
   else
     shade_launch<256>(sc, g, f, probe_org, hits, shadow, a4, precision, rad, rad_scale,
-                      num_probes, probe_base, s);
+                      num_probes, probe_base, clk, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -14,8 +14,10 @@
 namespace ane {
 
 __global__ __launch_bounds__(256) void k_translate(int W, int H, int plane_h, int sx, int sz,
-                                                   const float4* src, float4* dst)
+                                                   const float4* src, float4* dst, ClockArg clk)
 {
+  clock_begin(clk, 0);
+  if (blockIdx.x == 0 && threadIdx.x < 64) clock_fold(clk);
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (int64_t)W * H) return;
   const int Y = (int)(i / W), X = (int)(i - (int64_t)Y * W);
@@ -26,15 +28,17 @@ __global__ __launch_bounds__(256) void k_translate(int W, int H, int plane_h, in
   int64_t s = i;
   if (in_x && in_y) s = (int64_t)(Y + 10 * sz) * W + (X + 10 * sx);
   dst[i] = src[s];
+  clock_end(clk);
 }
 
-void launch_translate(const GridK& g, const float4* src, float4* dst, int dx, int dz, hipStream_t s)
+void launch_translate(const GridK& g, const float4* src, float4* dst, int dx, int dz, const ClockArg& clk,
+                      hipStream_t s)
 {
   const int64_t n = (int64_t)g.atlas_w * g.atlas_h;
   const int sx = dx > 0 ? 1 : (dx < 0 ? -1 : 0);
   const int sz = dz > 0 ? 1 : (dz < 0 ? -1 : 0);
   hipLaunchKernelGGL(k_translate, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g.atlas_w,
-                     g.atlas_h, 10 * g.nz, sx, sz, src, dst);
+                     g.atlas_h, 10 * g.nz, sx, sz, src, dst, clk);
 }
 
 // ---------------------------------------------------------------------------

@@ -169,8 +169,10 @@ typedef struct ane_scene_info {
 #define ANE_NODES_QUANTIZED_MIN_TRIS 2000000
 
 typedef struct ane_ddgi_stats {
-  /* device time per stage from hipEvent pairs, ms: the last call and the mean
-   * over all calls since the last ane_ddgi_stats_reset.  Stage order:
+  /* device time per stage from clock stamps of its kernels, ms: the last call and
+   * the mean over all calls since the last ane_ddgi_stats_reset (calls captured into
+   * a graph are not counted).  A stage ends where the next one of its call begins,
+   * the last one with its kernel.  Stage order:
    * setup, trace (primary rays and, in the same launch, the shadow ray of
    * every hit unless a sun grid serves them), sun grid (the build of the shadow
    * rays' candidate lists, only in the updates that build one: a new scene
