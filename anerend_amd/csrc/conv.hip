@@ -12,10 +12,11 @@
 // drop-in path), BF16 / FP16 (v_mfma_f32_16x16x32_bf16 / _f16) or FP8-e4m3
 // (v_mfma_f32_16x16x32_fp8_fp8), FP32 accumulate; FP8 carries a per-texel weight
 // scale and an FP32 radiance scale per probe, channel and 32 rays.
-//   k_conv_stream  a whole update: 64 probes per block, the weights in LDS, each
+//   k_conv_stream  large updates: 64 probes per block, the weights in LDS, each
 //                  wave streams its 16 probes over all rays
-//   k_conv_mfma    16 probes per block, 4 waves splitting the rays: weights too
-//                  large for LDS (FP32 beyond 640 rays, 16-bit beyond 1280)
+//   k_conv_mfma    16 probes per block, 4 waves splitting the rays: up to 8,192 probes
+//                  (up to 2,048 with the row tiles split over blocks), and weights too
+//                  large for LDS (FP32 beyond 608 rays, 16-bit beyond 1216)
 //   k_conv_jobs    the same blocks over the updates of a serving batch
 //   k_conv_fp32    FP32 register-tiled kernel for ray counts that are not a
 //                  multiple of 32
@@ -126,10 +127,11 @@ __global__ __launch_bounds__(256) void k_conv_fp32(GridK g, const float* rad, co
 
 // ---------------------------------------------------------------------------
 // MFMA convolution (FP32, BF16, FP8 operands, FP32 accumulate).
-// Block = 16 probes (one MFMA column tile) x 64 texels x 3 channels, 4 waves.
+// Block = 16 probes (one MFMA column tile) x RT row tiles of 16 texels x 3 channels,
+// 4 waves (RT = 4 covers the probe's 64 texels).
 // The 4 waves split the rays: wave w takes the 32-ray steps s = w, w + 4, ...,
 // loading the weight (A) and radiance (B) fragments of CH steps at a time, and
-// accumulates 4 row tiles x 3 channels.
+// accumulates RT row tiles x 3 channels.
 // The partial sums meet in LDS; then all 256 threads run the hysteresis
 // epilogue with consecutive threads on consecutive texels of a tile row (each
 // probe's row is 128 contiguous bytes of the atlas).
@@ -215,14 +217,16 @@ static constexpr int kPartStride = 17;  // texel stride of the LDS partials (pro
 
 // LDS of the partial sums: waves 2 and 3 hand theirs to waves 0 and 1, which
 // add them and leave two partials for the epilogue (26 KB, 6 blocks per CU)
-typedef float ConvPart[2][3][64 * kPartStride];
+template <int RT>
+using ConvPart = float[2][3][16 * RT * kPartStride];
 
-// One block's 16 probes (see above); blk is the block's index within its update.
-template <int PREC>
+// One block's 16 probes and RT of the 4 row tiles (see above); blk is the block's index
+// within its update (the row tiles of the same probes are neighbours).
+template <int PREC, int RT>
 __device__ __forceinline__ void conv_block(const GridK& g, const void* rad, const float* rad_scale,
                                            const void* wq, const float* wscale, const float* wsum,
                                            float4* atlas, int nprobes, int probe_base, int32_t bake, int blk,
-                                           ConvPart& part)
+                                           ConvPart<RT>& part)
 {
   using F = ConvFrag<PREC>;
   constexpr int EB = F::EB, CH = F::CH;
@@ -230,19 +234,20 @@ __device__ __forceinline__ void conv_block(const GridK& g, const void* rad, cons
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, kq = lane >> 4;
-  const int p0 = blk * kConvProbes;
+  const int p0 = blk / (4 / RT) * kConvProbes;
+  const int rt0 = blk % (4 / RT) * RT;  // the block's first row tile
   const bool pvalid = p0 + col < nprobes;
   const uint8_t* radp = (const uint8_t*)rad + (int64_t)(pvalid ? p0 + col : 0) * 3 * n * EB;
   // FP8: the scale of each (channel, 32-ray step) of this lane's probe
   const float* rsp = rad_scale + (int64_t)(pvalid ? p0 + col : 0) * 3 * S;
   const uint8_t* wp = (const uint8_t*)wq;
-  f32x4 acc[4][3];
+  f32x4 acc[RT][3];
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int c = 0; c < 3; ++c) acc[rt][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   for (int s0 = wave; s0 < S; s0 += kConvWaves * CH) {
-    F a[CH][4], b[CH][3];
+    F a[CH][RT], b[CH][3];
     float bs[CH][3];
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
@@ -253,8 +258,8 @@ __device__ __forceinline__ void conv_block(const GridK& g, const void* rad, cons
         for (int c = 0; c < 3; ++c) bs[j][c] = (s < S && pvalid) ? rsp[c * S + s] : 0.0f;
       }
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        if (s < S) a[j][rt].load(wp + ((int64_t)(rt * 16 + col) * n + k) * EB);
+      for (int rt = 0; rt < RT; ++rt) {
+        if (s < S) a[j][rt].load(wp + ((int64_t)((rt0 + rt) * 16 + col) * n + k) * EB);
         else a[j][rt].zero();
       }
 #pragma unroll
@@ -266,7 +271,7 @@ __device__ __forceinline__ void conv_block(const GridK& g, const void* rad, cons
 #pragma unroll
     for (int j = 0; j < CH; ++j)
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
+      for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
           if (PREC == ANE_PRECISION_FP8) {
@@ -282,7 +287,7 @@ __device__ __forceinline__ void conv_block(const GridK& g, const void* rad, cons
   // 0, 1 add them to their own and store the pair sums
   if (wave >= 2) {
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = rt * 16 + 4 * kq + i;
@@ -293,7 +298,7 @@ __device__ __forceinline__ void conv_block(const GridK& g, const void* rad, cons
   __syncthreads();
   if (wave < 2) {
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = rt * 16 + 4 * kq + i;
@@ -307,14 +312,14 @@ __device__ __forceinline__ void conv_block(const GridK& g, const void* rad, cons
   __syncthreads();
   const float h = g.hysteresis;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < RT; ++j) {
     const int item = tid + 256 * j;  // (ty, probe, tx), tx fastest
     const int tx = item & 7, p = (item >> 3) & 15, ty = item >> 7;
     if (p0 + p >= nprobes) continue;
-    const int t = ty * 8 + tx;
+    const int tl = ty * 8 + tx, t = 16 * rt0 + tl;
     float r[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) r[c] = part[0][c][t * kPartStride + p] + part[1][c][t * kPartStride + p];
+    for (int c = 0; c < 3; ++c) r[c] = part[0][c][tl * kPartStride + p] + part[1][c][tl * kPartStride + p];
     // per-texel weight scale (FP8 dequantization) or weight-sum correction (BF16)
     const float sc = (PREC == ANE_PRECISION_FP8) ? wscale[t]
                      : (PREC == ANE_PRECISION_BF16 || PREC == ANE_PRECISION_FP16) ? wscale[64 + t] : 1.0f;
@@ -324,7 +329,7 @@ __device__ __forceinline__ void conv_block(const GridK& g, const void* rad, cons
   }
 }
 
-template <int PREC>
+template <int PREC, int RT>
 __global__ __launch_bounds__(64 * kConvWaves) void k_conv_mfma(GridK g, const void* rad,
                                                               const float* rad_scale, const void* wq,
                                                               const float* wscale, const float* wsum,
@@ -332,18 +337,18 @@ __global__ __launch_bounds__(64 * kConvWaves) void k_conv_mfma(GridK g, const vo
                                                               int probe_base, int32_t bake, ClockArg clk)
 {
   clock_begin(clk, 0);
-  __shared__ ConvPart part;
-  conv_block<PREC>(g, rad, rad_scale, wq, wscale, wsum, atlas, nprobes, probe_base, bake, blockIdx.x, part);
+  __shared__ ConvPart<RT> part;
+  conv_block<PREC, RT>(g, rad, rad_scale, wq, wscale, wsum, atlas, nprobes, probe_base, bake, blockIdx.x, part);
   clock_end(clk);
   if (blockIdx.x == 0 && threadIdx.x >= 64 * (kConvWaves - 1)) clock_fold(clk);
 }
 
 // The convolutions of many updates in one launch (the request loop's fused
 // stage): block b runs block b - block_begin of the last job whose block_begin <= b.
-template <int PREC>
+template <int PREC, int RT>
 __global__ __launch_bounds__(64 * kConvWaves) void k_conv_jobs(const ConvJob* jobs, int njobs)
 {
-  __shared__ ConvPart part;
+  __shared__ ConvPart<RT> part;
   const int b = blockIdx.x;
   int lo = 0, hi = njobs - 1;
   while (lo < hi) {
@@ -352,7 +357,7 @@ __global__ __launch_bounds__(64 * kConvWaves) void k_conv_jobs(const ConvJob* jo
     else hi = mid - 1;
   }
   const ConvJob& j = jobs[lo];
-  conv_block<PREC>(j.g, j.rad, j.rad_scale, j.wq, j.wscale, j.wsum, j.atlas, j.nprobes, j.probe_base, j.bake,
+  conv_block<PREC, RT>(j.g, j.rad, j.rad_scale, j.wq, j.wscale, j.wsum, j.atlas, j.nprobes, j.probe_base, j.bake,
                    b - j.block_begin, part);
 }
 
@@ -374,9 +379,6 @@ __global__ __launch_bounds__(64 * kConvWaves) void k_conv_jobs(const ConvJob* jo
 // rt*16 + 4kq + i, i = 0..3, 4 consecutive texels (64 contiguous atlas bytes)
 // of tile row 2rt + kq/2 of probe col; its per-texel factors come from LDS.
 // ---------------------------------------------------------------------------
-#ifndef ANE_CONV_STREAM
-#define ANE_CONV_STREAM 1
-#endif
 // Radiance ring depth in 32-ray steps, per operand size (a sweep of 1, 2, 4 and 8:
 // deeper rings hold more registers; these were the fastest on the production shape).
 #ifndef ANE_CONV_DEPTH16
@@ -594,9 +596,16 @@ static size_t conv_stream_lds(int precision, int rays)
   return (size_t)64 * rays * conv_operand_bytes(precision) + kStreamFactorBytes;
 }
 
-bool conv_stream_fits(int precision, int rays)
+// Above kStreamMinProbes probes, when the weights of all rays fit LDS.  A streaming block
+// works its 64 probes off in one chain of all rays per wave, a split-ray block its 16 in a
+// quarter of it: with few blocks per CU the chain is the launch.  FP32, 512 rays, split-ray
+// against streaming: 1,024 probes 12.5 / 32.9 us, 4,096 14.1 / 33.5, 8,192 25.7 / 33.5,
+// 16,384 47.7 / 37.1; 16-bit 6.2 / 10.3, 6.4 / 10.7, 10.7 / 12.1, 18.4 / 16.4 us.
+static constexpr int kStreamMinProbes = 8192;
+bool conv_stream_fits(int precision, int rays, int num_probes)
 {
-  return ANE_CONV_STREAM && rays > 0 && rays % 32 == 0 && conv_stream_lds(precision, rays) <= (size_t)kStreamLdsMax;
+  return num_probes > kStreamMinProbes && rays > 0 && rays % 32 == 0 &&
+         conv_stream_lds(precision, rays) <= (size_t)kStreamLdsMax;
 }
 
 // The ring depth: the largest power of two up to the precision's depth that
@@ -665,7 +674,7 @@ static void launch_conv_stream_any(int precision, int S, bool jobs, const GridK&
 
 int conv_job_blocks(int precision, int rays, int num_probes)
 {
-  const int per = conv_stream_fits(precision, rays) ? kStreamProbes : kConvProbes;
+  const int per = conv_stream_fits(precision, rays, num_probes) ? kStreamProbes : kConvProbes;
   return (num_probes + per - 1) / per;
 }
 
@@ -681,13 +690,33 @@ void launch_conv_jobs(int precision, const ConvJob* jobs, int njobs, int total_b
   }
   const dim3 grid((unsigned)total_blocks), block(64 * kConvWaves);
   if (precision == ANE_PRECISION_FP32)
-    hipLaunchKernelGGL(k_conv_jobs<ANE_PRECISION_FP32>, grid, block, 0, s, jobs, njobs);
+    hipLaunchKernelGGL((k_conv_jobs<ANE_PRECISION_FP32, 4>), grid, block, 0, s, jobs, njobs);
   else if (precision == ANE_PRECISION_FP16)
-    hipLaunchKernelGGL(k_conv_jobs<ANE_PRECISION_FP16>, grid, block, 0, s, jobs, njobs);
+    hipLaunchKernelGGL((k_conv_jobs<ANE_PRECISION_FP16, 4>), grid, block, 0, s, jobs, njobs);
   else if (precision == ANE_PRECISION_BF16)
-    hipLaunchKernelGGL(k_conv_jobs<ANE_PRECISION_BF16>, grid, block, 0, s, jobs, njobs);
+    hipLaunchKernelGGL((k_conv_jobs<ANE_PRECISION_BF16, 4>), grid, block, 0, s, jobs, njobs);
   else
-    hipLaunchKernelGGL(k_conv_jobs<ANE_PRECISION_FP8>, grid, block, 0, s, jobs, njobs);
+    hipLaunchKernelGGL((k_conv_jobs<ANE_PRECISION_FP8, 4>), grid, block, 0, s, jobs, njobs);
+}
+
+// Row tiles per block: the fewest whose blocks still find a CU each (the sums of a texel
+// are the same either way).  1 / 2 / 4 row tiles, FP32, 512 rays: 1,024 probes 5.8 / 7.7 /
+// 12.5 us, 2,048 probes 11.1 / 8.4 / 12.5, 4,096 probes 18.6 / 14.3 / 13.9; 16-bit 3.2 / 4.3 /
+// 6.2, 6.4 / 4.3 / 6.2, 12.3 / 7.9 / 6.4 us.
+static constexpr int kConvCus = 256;
+template <int PREC>
+static void launch_conv_mfma(const GridK& g, const void* rad, const float* rad_scale, const void* wq,
+                             const float* wscale, const float* wsum, float4* atlas, int num_probes, int probe_base,
+                             bool bake, const ClockArg& clk, hipStream_t s)
+{
+  const int blocks = (num_probes + kConvProbes - 1) / kConvProbes;
+#define ANE_CONV(RT)                                                                                                   \
+  hipLaunchKernelGGL((k_conv_mfma<PREC, RT>), dim3((unsigned)(blocks * (4 / RT))), dim3(64 * kConvWaves), 0, s, g, rad, \
+                     rad_scale, wq, wscale, wsum, atlas, num_probes, probe_base, (int32_t)bake, clk)
+  if (4 * blocks <= kConvCus) ANE_CONV(1);
+  else if (2 * blocks <= kConvCus) ANE_CONV(2);
+  else ANE_CONV(4);
+#undef ANE_CONV
 }
 
 void launch_convolve(const GridK& g, const FrameK& f, int precision, const void* rad,
@@ -698,37 +727,28 @@ void launch_convolve(const GridK& g, const FrameK& f, int precision, const void*
   (void)f;
   if (num_probes <= 0) return;
   float4* a4 = reinterpret_cast<float4*>(atlas);
-  const unsigned blocks = (unsigned)((num_probes + kConvProbes - 1) / kConvProbes);
-  if (conv_stream_fits(precision, g.rays)) {
-    const void* wq = precision == ANE_PRECISION_FP32 ? (const void*)w32
-                     : precision == ANE_PRECISION_FP8 ? (const void*)wfp8 : (const void*)wbf16;
+  const void* wq = precision == ANE_PRECISION_FP32 ? (const void*)w32
+                   : precision == ANE_PRECISION_FP8 ? (const void*)wfp8 : (const void*)wbf16;
+  if (conv_stream_fits(precision, g.rays, num_probes)) {
     const int blocks = (num_probes + kStreamProbes - 1) / kStreamProbes;
     launch_conv_stream_any(precision, g.rays / 32, false, g, rad, rad_scale, wq, wfp8_scale, wsum, a4, num_probes,
                            probe_base, bake, nullptr, 0, blocks, conv_stream_lds(precision, g.rays), clk, s);
-    return;
-  }
-  if (precision == ANE_PRECISION_FP32) {
-    if (g.rays % 32 != 0) {  // the register-tiled kernel takes any ray count
-      const unsigned b32 = (unsigned)((num_probes + kPB - 1) / kPB);
-      hipLaunchKernelGGL(k_conv_fp32, dim3(b32), dim3(256), 0, s, g, (const float*)rad, w32, wsum,
-                         a4, num_probes, probe_base, (int32_t)bake, clk);
-      return;
-    }
-    hipLaunchKernelGGL(k_conv_mfma<ANE_PRECISION_FP32>, dim3(blocks), dim3(64 * kConvWaves), 0, s, g, rad,
-                       rad_scale, (const void*)w32, wfp8_scale, wsum, a4, num_probes, probe_base,
-                       (int32_t)bake, clk);
-  } else if (precision == ANE_PRECISION_FP16) {
-    hipLaunchKernelGGL(k_conv_mfma<ANE_PRECISION_FP16>, dim3(blocks), dim3(64 * kConvWaves), 0, s, g,
-                       rad, rad_scale, (const void*)wbf16, wfp8_scale, wsum, a4,
-                       num_probes, probe_base, (int32_t)bake, clk);
-  } else if (precision == ANE_PRECISION_BF16) {
-    hipLaunchKernelGGL(k_conv_mfma<ANE_PRECISION_BF16>, dim3(blocks), dim3(64 * kConvWaves), 0, s, g,
-                       rad, rad_scale, (const void*)wbf16, wfp8_scale, wsum, a4,
-                       num_probes, probe_base, (int32_t)bake, clk);
-  } else {
-    hipLaunchKernelGGL(k_conv_mfma<ANE_PRECISION_FP8>, dim3(blocks), dim3(64 * kConvWaves), 0, s, g,
-                       rad, rad_scale, (const void*)wfp8, wfp8_scale, wsum, a4, num_probes,
+  } else if (g.rays % 32 != 0) {  // FP32 only; the register-tiled kernel takes any ray count
+    const unsigned b32 = (unsigned)((num_probes + kPB - 1) / kPB);
+    hipLaunchKernelGGL(k_conv_fp32, dim3(b32), dim3(256), 0, s, g, (const float*)rad, w32, wsum, a4, num_probes,
                        probe_base, (int32_t)bake, clk);
+  } else if (precision == ANE_PRECISION_FP32) {
+    launch_conv_mfma<ANE_PRECISION_FP32>(g, rad, rad_scale, wq, wfp8_scale, wsum, a4, num_probes, probe_base, bake,
+                                         clk, s);
+  } else if (precision == ANE_PRECISION_FP16) {
+    launch_conv_mfma<ANE_PRECISION_FP16>(g, rad, rad_scale, wq, wfp8_scale, wsum, a4, num_probes, probe_base, bake,
+                                         clk, s);
+  } else if (precision == ANE_PRECISION_BF16) {
+    launch_conv_mfma<ANE_PRECISION_BF16>(g, rad, rad_scale, wq, wfp8_scale, wsum, a4, num_probes, probe_base, bake,
+                                         clk, s);
+  } else {
+    launch_conv_mfma<ANE_PRECISION_FP8>(g, rad, rad_scale, wq, wfp8_scale, wsum, a4, num_probes, probe_base, bake,
+                                        clk, s);
   }
 }
 

@@ -273,10 +273,10 @@ struct ConvJob {
 // max_rays: the largest ray count among the jobs (FP8 stages a probe in LDS)
 void launch_shade_jobs(int precision, const ShadeJob* jobs, int njobs, int total_blocks, int max_rays,
                        hipStream_t s);
-// Whether a convolution of this precision and ray count takes the streaming
-// kernel (its weights fit LDS); the request loop launches such jobs apart from
+// Whether a convolution of this precision, ray count and probe count takes the
+// streaming kernel; the request loop launches such jobs apart from
 // the others so that every update runs the kernel its own launch would.
-bool conv_stream_fits(int precision, int rays);
+bool conv_stream_fits(int precision, int rays, int num_probes);
 int conv_job_blocks(int precision, int rays, int num_probes);
 // stream: every job fits the streaming kernel; max_rays: their largest ray
 // count (LDS size); rays_gcd: the greatest common divisor of their ray counts

@@ -176,7 +176,7 @@ void ane_serve::launch_fused(std::vector<Launch>& batch, int slot,
       for (size_t i = 0; i < batch.size(); ++i) {
         if (prec[i] != p) continue;
         const int rays = cj[i].g.rays;
-        if ((ane::conv_stream_fits(p, rays) ? 0 : 1) != kind) continue;
+        if ((ane::conv_stream_fits(p, rays, cj[i].nprobes) ? 0 : 1) != kind) continue;
         sj[i].block_begin = grp[p].shade_blocks;
         cj[i].block_begin = grp[p].conv_blocks[kind];
         grp[p].shade_blocks += cj[i].nprobes;
