@@ -288,6 +288,9 @@ struct SunGridCache {
     cap = (uint32_t)capl;
     return ANE_OK;
   }
+  // 1 / 0: the current build is known on the host to be in use / left out, -1: not known
+  // yet (the launches of a call then decide on the device)
+  int known_valid() const { return built.set && known == built ? last_valid : -1; }
   // *use: the grid for (scene, version, dir) is current after the call.  A
   // direction with a zero (or non-finite) component never gets one: its rays
   // can lie exactly in a box face, where the traversal's slab test (zero
@@ -296,10 +299,13 @@ struct SunGridCache {
   // from the traversal's there.
   // clk, stage: the stage stamp of a build
   // rays: the rays of the request (the eager-build rule)
+  // *valid (nullable): known_valid() when *use
   int update(const SceneK& view, int32_t ntri, const void* scene, uint64_t version, const float* dir3,
-             int64_t rays, hipStream_t st, bool* use, const ClockArg& clk = ClockArg{}, int stage = 0)
+             int64_t rays, hipStream_t st, bool* use, const ClockArg& clk = ClockArg{}, int stage = 0,
+             int* valid = nullptr)
   {
     *use = false;
+    if (valid) *valid = -1;
     for (int k = 0; k < 3; ++k)
       if (!(dir3[k] != 0.0f) || !std::isfinite(dir3[k])) return ANE_OK;
     Key k;
@@ -307,14 +313,15 @@ struct SunGridCache {
     k.version = version;
     std::memcpy(k.dir, dir3, sizeof(k.dir));
     k.set = true;
-    if (built == k) {
-      *use = true;
-      return ANE_OK;
-    }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     ANE_CHECK_HIP(hipStreamIsCapturing(st, &cs));
     const bool capturing = cs != hipStreamCaptureStatusNone;
     if (!capturing) poll();  // no event queries under capture
+    if (built == k) {
+      *use = true;
+      if (valid) *valid = capturing ? -1 : known_valid();  // a graph keeps both ways: the grid may change before a replay
+      return ANE_OK;
+    }
     const bool eager = known.set && known.scene == scene && known.version == version && last_valid == 1 &&
                        rays >= (int64_t)ANE_SUNGRID_EAGER_RAYS * ntri;
     if (!ANE_SUNGRID_EAGER && !eager && !(seen == k)) {
@@ -412,9 +419,10 @@ struct ane_scene {
   float* d_sh_orig = nullptr;
   float* d_sh_dir = nullptr;
   ane_hit* d_sh_hits = nullptr;
-  uint32_t* d_sh_work = nullptr;
-  unsigned long long* d_sh_stats = nullptr;
-  uint32_t* d_sh_ov = nullptr;
+  uint32_t* d_sh_work = nullptr;             // claim counters, then (in the same buffer):
+  unsigned long long* d_sh_stats = nullptr;  // [2] work counters
+  uint32_t* d_sh_ov = nullptr;               // fault flag
+  bool sh_traced = false;                    // the last pass launched a traversal (d_sh_ov is its)
   int32_t* d_sh_spill = nullptr;
   int64_t sh_spill_words = 0;
   // point-light shadow workspace (grows to the most lights seen); the sum's
@@ -448,7 +456,7 @@ static void scene_free(ane_scene* s)
   dfree(s->d_info); dfree(s->d_topo); dfree(s->d_cross); dfree(s->d_cross_kids); dfree(s->d_top); dfree(s->d_ndepth); dfree(s->d_units);
   dfree(s->d_unit_root); dfree(s->d_uheight); dfree(s->d_stray); dfree(s->d_uscratch);
   dfree(s->d_sh_orig); dfree(s->d_sh_dir); dfree(s->d_sh_hits); dfree(s->d_sh_work);
-  dfree(s->d_sh_stats); dfree(s->d_sh_ov); dfree(s->d_sh_spill);
+  dfree(s->d_sh_spill);
   dfree(s->d_lt_lights); dfree(s->d_lt_orig); dfree(s->d_lt_dir); dfree(s->d_lt_tmax); dfree(s->d_lt_hits);
   dfree(s->d_lt_dist); dfree(s->d_lt_dirs); dfree(s->d_lt_wt); dfree(s->d_lt_idx); dfree(s->d_lt_order); dfree(s->d_lt_work);
   dfree(s->d_lt_stats);
@@ -922,14 +930,14 @@ struct ane_ddgi_ctx {
   ane_ddgi_stats stats{};
   int64_t bytes = 0;
   hipGraphExec_t gexec = nullptr;  // the last captured update (request loop)
-  // mirror-reflection workspace, sized on first use: [0] reflection rays,
-  // [1] their shadow rays
+  // mirror-reflection workspace in slot order (launch_mirror_rays), sized on first use:
+  // [0] reflection rays, [1] their shadow rays
   float* d_mr_orig[2] = {nullptr, nullptr};
   float* d_mr_dir[2] = {nullptr, nullptr};
   ane_hit* d_mr_hits[2] = {nullptr, nullptr};
-  uint32_t* d_mr_work = nullptr;             // [2] ray counters
-  unsigned long long* d_mr_stats = nullptr;  // [4]
-  uint32_t* d_mr_ov = nullptr;
+  uint32_t* d_mr_work = nullptr;             // claim counters, then (in the same buffer):
+  unsigned long long* d_mr_stats = nullptr;  // [4] work counters
+  uint32_t* d_mr_ov = nullptr;               // fault flag
   int32_t* d_mr_spill = nullptr;
   int64_t mr_px = 0, mr_spill_words = 0;
 };
@@ -946,7 +954,7 @@ static void ctx_free(ane_ddgi_ctx* c)
   c->sgc.destroy();
   if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
   for (int k = 0; k < 2; ++k) { dfree(c->d_mr_orig[k]); dfree(c->d_mr_dir[k]); dfree(c->d_mr_hits[k]); }
-  dfree(c->d_mr_work); dfree(c->d_mr_stats); dfree(c->d_mr_ov); dfree(c->d_mr_spill);
+  dfree(c->d_mr_work); dfree(c->d_mr_spill);
   dfree(c->d_clock);
 }
 
@@ -1593,23 +1601,23 @@ extern "C" int ane_ddgi_mirror_reflections(ane_ddgi_ctx* c, const ane_scene* s, 
   full.layer_count = c->g.ny;
   ANE_TRY(frame_to_k(c, &full, &fk));
   hipStream_t st = S(stream);
-  if (n > c->mr_px) {
+  const int64_t slots = pixel_slot_count(width, height);
+  if (slots > c->mr_px) {
     ANE_CHECK_HIP(hipStreamSynchronize(st));
     for (int k = 0; k < 2; ++k) { dfree(c->d_mr_orig[k]); dfree(c->d_mr_dir[k]); dfree(c->d_mr_hits[k]); }
     c->mr_px = 0;
     for (int k = 0; k < 2; ++k) {
-      ANE_TRY(dalloc(&c->d_mr_orig[k], 3 * n, nullptr));
-      ANE_TRY(dalloc(&c->d_mr_dir[k], 3 * n, nullptr));
-      ANE_TRY(dalloc(&c->d_mr_hits[k], n, nullptr));
+      ANE_TRY(dalloc(&c->d_mr_orig[k], 3 * slots, nullptr));
+      ANE_TRY(dalloc(&c->d_mr_dir[k], 3 * slots, nullptr));
+      ANE_TRY(dalloc(&c->d_mr_hits[k], slots, nullptr));
     }
-    c->mr_px = n;
+    c->mr_px = slots;
   }
-  if (!c->d_mr_work || !c->d_mr_stats || !c->d_mr_ov) {  // all three, or redo them
-    dfree(c->d_mr_work); dfree(c->d_mr_stats); dfree(c->d_mr_ov);
-    ANE_TRY(dalloc(&c->d_mr_work, 2 * kTraceWorkWords, nullptr));
-    ANE_TRY(dalloc(&c->d_mr_stats, 4, nullptr));
-    ANE_TRY(dalloc(&c->d_mr_ov, 1, nullptr));
-  }
+  // claim counters of the two traversals, 4 work counters (64-bit), the fault flag
+  constexpr int kMrWords = 2 * kTraceWorkWords + 9;
+  if (!c->d_mr_work) ANE_TRY(dalloc(&c->d_mr_work, kMrWords, nullptr));
+  c->d_mr_stats = reinterpret_cast<unsigned long long*>(c->d_mr_work + 2 * kTraceWorkWords);
+  c->d_mr_ov = c->d_mr_work + 2 * kTraceWorkWords + 8;
   const int64_t lanes = trace_lanes_per_launch();
   const int64_t sd = s->depth - trace_stack_lds() + 1 > 0 ? s->depth - trace_stack_lds() + 1 : 0;
   if (sd * lanes > c->mr_spill_words) {
@@ -1619,18 +1627,16 @@ extern "C" int ane_ddgi_mirror_reflections(ane_ddgi_ctx* c, const ane_scene* s, 
     ANE_TRY(dalloc(&c->d_mr_spill, sd * lanes, nullptr));
     c->mr_spill_words = sd * lanes;
   }
-  fill_u32(c->d_mr_work, 0u, 2 * kTraceWorkWords, st);
-  fill_u32(reinterpret_cast<uint32_t*>(c->d_mr_stats), 0u, 8, st);
-  fill_u32(c->d_mr_ov, 0u, 1, st);
   // mirror_reflections.rgen:57-79: reflection rays over [0.1, 50], closest hit
-  launch_mirror_rays(depth, normal4, width, height, ivp16, f->camera_pos, c->d_mr_orig[0], c->d_mr_dir[0], st);
+  launch_mirror_rays(depth, normal4, width, height, ivp16, f->camera_pos, c->d_mr_orig[0], c->d_mr_dir[0],
+                     c->d_mr_work, kMrWords, st);
   TraceArgs a{};
   a.sc = s->view;
   a.g.rays = 1;
   a.overflow = c->d_mr_ov;
   a.spill = c->d_mr_spill;
   a.spill_depth = (int32_t)sd;
-  a.nrays = (int32_t)n;
+  a.nrays = (int32_t)slots;
   a.t_min = 0.1f;
   a.t_max = 50.0f;
   a.hits = c->d_mr_hits[0];
@@ -1642,26 +1648,31 @@ extern "C" int ane_ddgi_mirror_reflections(ane_ddgi_ctx* c, const ane_scene* s, 
   // mirror_reflections.rchit:44-66: shadow rays from the hits, any hit over [0.1, 50]
   const f3 sun = normalize(mk(-fk.light_dir[0], -fk.light_dir[1], -fk.light_dir[2]));
   const float sun3[3] = {sun.x, sun.y, sun.z};
-  launch_mirror_shadow_rays(s->view, c->d_mr_hits[0], n, sun3, c->d_mr_orig[1], c->d_mr_dir[1], st);
+  // through the sun grid once it is current, else (or while its validity is not known
+  // here: decided by a device flag) by traversal
   const uint32_t* skip = nullptr;
+  int valid = 0;
   if (!counters4 && sun_grid_wanted(c)) {
     bool use = false;
-    ANE_TRY(c->sgc.update(s->view, s->ntri, s, s->version, sun3, n, st, &use));
-    if (use) {
-      launch_anyhit_grid(c->d_mr_orig[1], c->d_mr_dir[1], n, c->sgc.view(), s->view, 0.1f, 50.0f, c->d_mr_hits[1],
-                         st);
+    ANE_TRY(c->sgc.update(s->view, s->ntri, s, s->version, sun3, n, st, &use, ClockArg{}, 0, &valid));
+    if (!use) valid = 0;
+    if (valid != 0) {
+      launch_mirror_shadow_grid(s->view, c->d_mr_hits[0], slots, sun3, c->sgc.view(), 0.1f, 50.0f, c->d_mr_hits[1], st);
       skip = c->sgc.valid_flag();
     }
   }
-  a.skip_if_set = skip;
-  a.hits = c->d_mr_hits[1];
-  a.work = c->d_mr_work + kTraceWorkWords;
-  a.stats = c->d_mr_stats + 2;
-  a.ray_orig = c->d_mr_orig[1];
-  a.ray_dir = c->d_mr_dir[1];
-  launch_trace(a, true, true, counters4 != nullptr, st);
+  if (valid != 1) {
+    launch_mirror_shadow_rays(s->view, c->d_mr_hits[0], slots, sun3, c->d_mr_orig[1], c->d_mr_dir[1], st, skip);
+    a.skip_if_set = skip;
+    a.hits = c->d_mr_hits[1];
+    a.work = c->d_mr_work + kTraceWorkWords;
+    a.stats = c->d_mr_stats + 2;
+    a.ray_orig = c->d_mr_orig[1];
+    a.ray_dir = c->d_mr_dir[1];
+    launch_trace(a, true, true, counters4 != nullptr, st);
+  }
   launch_mirror_shade(s->view, c->g, fk, c->d_atlas[c->cur], depth, c->d_mr_orig[0], c->d_mr_hits[0],
-                      c->d_mr_hits[1], n, out_rgba, st);
+                      c->d_mr_hits[1], width, height, out_rgba, st);
   ANE_CHECK_HIP(hipGetLastError());
   if (counters4) {
     unsigned long long c4[4] = {0, 0, 0, 0};
@@ -1896,6 +1907,27 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
   for (int k = 0; k < 3; ++k)
     if (!std::isfinite(light3[k])) return fail(ANE_ERR_INVALID_ARG, "non-finite light direction");
   hipStream_t st = S(stream);
+  // without counters the rays go through the scene's grid along -light_dir once it is
+  // current; while its validity is not known here, the traversal launches follow and do
+  // nothing when it is (device flag)
+  const uint32_t* skip = nullptr;
+  s->sh_traced = true;
+  if (!counters2) {
+    const float dir[3] = {-light3[0], -light3[1], -light3[2]};
+    bool use = false;
+    int valid = -1;
+    ANE_TRY(s->sgc.update(s->view, s->ntri, s, s->version, dir, (int64_t)width * height, st, &use, ClockArg{}, 0,
+                          &valid));
+    if (use && valid != 0) {
+      launch_shadow_mask_grid(depth, width, height, ivp16, light3, s->sgc.view(), s->view, out_vis, st);
+      if (valid == 1) {
+        s->sh_traced = false;
+        ANE_CHECK_HIP(hipGetLastError());
+        return ANE_OK;
+      }
+      skip = s->sgc.valid_flag();
+    }
+  }
   if (n > s->shadow_px) {
     ANE_CHECK_HIP(hipStreamSynchronize(st));
     dfree(s->d_sh_orig); dfree(s->d_sh_dir); dfree(s->d_sh_hits);
@@ -1905,12 +1937,11 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
     ANE_TRY(dalloc(&s->d_sh_hits, n, nullptr));
     s->shadow_px = n;
   }
-  if (!s->d_sh_work || !s->d_sh_stats || !s->d_sh_ov) {  // all three, or redo them
-    dfree(s->d_sh_work); dfree(s->d_sh_stats); dfree(s->d_sh_ov);
-    ANE_TRY(dalloc(&s->d_sh_work, kTraceWorkWords, nullptr));
-    ANE_TRY(dalloc(&s->d_sh_stats, 2, nullptr));
-    ANE_TRY(dalloc(&s->d_sh_ov, 1, nullptr));
-  }
+  // claim counters, 2 work counters (64-bit), the fault flag
+  constexpr int kShWords = kTraceWorkWords + 5;
+  if (!s->d_sh_work) ANE_TRY(dalloc(&s->d_sh_work, kShWords, nullptr));
+  s->d_sh_stats = reinterpret_cast<unsigned long long*>(s->d_sh_work + kTraceWorkWords);
+  s->d_sh_ov = s->d_sh_work + kTraceWorkWords + 4;
   const int64_t lanes = trace_lanes_per_launch();
   const int64_t sd = s->depth - trace_stack_lds() + 1 > 0 ? s->depth - trace_stack_lds() + 1 : 0;
   if (sd * lanes > s->sh_spill_words) {
@@ -1920,22 +1951,7 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
     ANE_TRY(dalloc(&s->d_sh_spill, sd * lanes, nullptr));
     s->sh_spill_words = sd * lanes;
   }
-  // without counters the rays go through the scene's grid along -light_dir once it
-  // is current; the traversal launches below then do nothing (device flag)
-  const uint32_t* skip = nullptr;
-  if (!counters2) {
-    const float dir[3] = {-light3[0], -light3[1], -light3[2]};
-    bool use = false;
-    ANE_TRY(s->sgc.update(s->view, s->ntri, s, s->version, dir, (int64_t)width * height, st, &use));
-    if (use) {
-      launch_shadow_mask_grid(depth, width, height, ivp16, light3, s->sgc.view(), s->view, out_vis, st);
-      skip = s->sgc.valid_flag();
-    }
-  }
-  launch_shadow_rays(depth, width, height, ivp16, light3, s->d_sh_orig, s->d_sh_dir, st, skip);
-  fill_u32(s->d_sh_work, 0u, kTraceWorkWords, st);
-  fill_u32(reinterpret_cast<uint32_t*>(s->d_sh_stats), 0u, 4, st);
-  fill_u32(s->d_sh_ov, 0u, 1, st);
+  launch_shadow_rays(depth, width, height, ivp16, light3, s->d_sh_orig, s->d_sh_dir, s->d_sh_work, kShWords, st, skip);
   TraceArgs a{};
   a.sc = s->view;
   a.g.rays = 1;
@@ -1972,7 +1988,7 @@ extern "C" int ane_scene_check(ane_scene* s, void* stream)
   if (!s) return fail(ANE_ERR_INVALID_ARG, "NULL scene");
   uint32_t v[2] = {0, 0};
   ANE_CHECK_HIP(hipStreamSynchronize(S(stream)));
-  if (s->d_sh_ov) ANE_CHECK_HIP(hipMemcpy(&v[0], s->d_sh_ov, 4, hipMemcpyDeviceToHost));
+  if (s->d_sh_ov && s->sh_traced) ANE_CHECK_HIP(hipMemcpy(&v[0], s->d_sh_ov, 4, hipMemcpyDeviceToHost));
   if (s->d_lt_ov) ANE_CHECK_HIP(hipMemcpy(&v[1], s->d_lt_ov, 4, hipMemcpyDeviceToHost));
   if (s->d_sh_ov) ANE_CHECK_HIP(hipMemset(s->d_sh_ov, 0, 4));
   if (s->d_lt_ov) ANE_CHECK_HIP(hipMemset(s->d_lt_ov, 0, 4));

@@ -161,37 +161,12 @@ __host__ __device__ __forceinline__ int sun_cell(float v, float o, float inv, in
 }
 void sun_grid_setup(SunGridParams& g, const float* dir3, int gx, int gy);
 
-// Any hit of the ray r (origin o, the grid's direction) among the triangles of
-// its cell: the watertight test in list order, the first hit ends it.
-__device__ __forceinline__ bool grid_any_hit(const SunGridK& sg, const SunGridParams& g, const float4* tris,
-                                             int32_t ntri, const RayPre& r, f3 o, float tmin, float tmax,
-                                             ane_hit* h)
-{
-  const float X = comp(o, g.kx) - g.sx * comp(o, g.kz);
-  const float Y = comp(o, g.ky) - g.sy * comp(o, g.kz);
-  const int64_t cell = (int64_t)sun_cell(Y, g.y0, g.ich, g.gy) * g.gx + sun_cell(X, g.x0, g.icw, g.gx);
-  const uint32_t b = sg.start[cell], e = sg.start[cell + 1];
-  for (uint32_t k = b; k < e; ++k) {
-    const uint32_t p = sg.list[k];
-    if (p >= (uint32_t)ntri) continue;
-    const float4 v0 = tris[3 * (int64_t)p], v1 = tris[3 * (int64_t)p + 1], v2 = tris[3 * (int64_t)p + 2];
-    float t, u, v;
-    if (tri_test(r, mk(v0.x, v0.y, v0.z), mk(v1.x, v1.y, v1.z), mk(v2.x, v2.y, v2.z), tmin, tmax, t, u, v)) {
-      h->tri = __float_as_int(v0.w);
-      h->t = t;
-      h->u = u;
-      h->v = v;
-      return true;
-    }
-  }
-  return false;
-}
-// rays sharing the grid's direction (zero or non-finite direction: no ray); kernels
-// do nothing unless the grid is valid
+// slots of the tile order of a W x H image (at least its pixels)
+int64_t pixel_slot_count(int W, int H);
+// the shadow mask through the grid of its rays' direction (zero or non-finite
+// direction: no ray); does nothing unless the grid is valid
 void launch_shadow_mask_grid(const float* depth, int W, int H, const float* ivp16, const float* light3,
                              const SunGridK& sg, const SceneK& sc, float* vis, hipStream_t s);
-void launch_anyhit_grid(const float* orig, const float* dirs, int64_t n, const SunGridK& sg, const SceneK& sc,
-                        float tmin, float tmax, ane_hit* hits, hipStream_t s);
 // est: [sun_grid_scratch_words(ntri)] build scratch (partial sums of the candidate
 // estimate, per-block cell counts)
 int64_t sun_grid_scratch_words(int32_t ntri);
@@ -330,7 +305,8 @@ void launch_gi_lookup(const GridK& g, const FrameK& f, const float* atlas, const
 
 // RT hard shadows: per-pixel rays (orig, dirs: W*H*3 floats) and visibility
 void launch_shadow_rays(const float* depth, int W, int H, const float* ivp16, const float* light3,
-                        float* orig, float* dirs, hipStream_t s, const uint32_t* skip_if_set = nullptr);
+                        float* orig, float* dirs, uint32_t* clear, int nclear, hipStream_t s,
+                        const uint32_t* skip_if_set = nullptr);
 // point-light shadow moments: lights = n x 8 floats {x, y, z, range, r, g, b, enabled};
 // 1024 rays per light; lw / lidx [kmax][64 texels] = each texel's (weight, ray) pairs
 // with weight above 0.001 in the summation order, padded with weight 0
@@ -344,14 +320,18 @@ void launch_light_moments(const float* lights, int n, const float* dist, const f
                           const int32_t* lidx, int kmax, float* mom, hipStream_t s);
 void launch_shadow_resolve(const float* depth, const ane_hit* hits, int64_t n, float* vis, hipStream_t s,
                            const uint32_t* skip_if_set = nullptr);
-// mirror reflections: reflection rays, the shadow rays of their hits, shading
+// mirror reflections: reflection rays in slot order (pixel_slot_count(W, H) of them), the
+// shadow rays of their hits for the traversal or through a sun grid, shading.  clear:
+// [nclear] words set to 0 before the launches that follow.
 void launch_mirror_rays(const float* depth, const float* normal4, int W, int H, const float* ivp16,
-                        const float* cam3, float* orig, float* dirs, hipStream_t s);
+                        const float* cam3, float* orig, float* dirs, uint32_t* clear, int nclear, hipStream_t s);
 void launch_mirror_shadow_rays(const SceneK& sc, const ane_hit* hits, int64_t n, const float* sun3, float* orig,
-                               float* dirs, hipStream_t s);
+                               float* dirs, hipStream_t s, const uint32_t* skip_if_set);
+void launch_mirror_shadow_grid(const SceneK& sc, const ane_hit* hits, int64_t n, const float* sun3,
+                               const SunGridK& sg, float tmin, float tmax, ane_hit* shadow_hits, hipStream_t s);
 void launch_mirror_shade(const SceneK& sc, const GridK& g, const FrameK& f, const float* atlas,
                          const float* depth, const float* orig, const ane_hit* hits, const ane_hit* shadow_hits,
-                         int64_t n, float* out, hipStream_t s);
+                         int W, int H, float* out, hipStream_t s);
 
 // translate.hip
 void launch_translate(const GridK& g, const float4* src, float4* dst, int dx, int dz, const ClockArg& clk,
