@@ -433,15 +433,14 @@ struct ane_scene {
   float* d_lt_dir = nullptr;
   float* d_lt_tmax = nullptr;
   ane_hit* d_lt_hits = nullptr;
-  float* d_lt_dist = nullptr;
   float* d_lt_dirs = nullptr;
   float* d_lt_wt = nullptr;       // [lt_kmax][64] weights of each texel's rays, summation order
   int32_t* d_lt_idx = nullptr;    // [lt_kmax][64] their ray indices (lt_kmax 0: not set up yet)
   uint32_t* d_lt_order = nullptr; // [1024] ray traced in each slot (direction-coherent order)
   int32_t lt_kmax = 0;
-  uint32_t* d_lt_work = nullptr;
-  unsigned long long* d_lt_stats = nullptr;
-  uint32_t* d_lt_ov = nullptr;
+  uint32_t* d_lt_work = nullptr;             // claim counters, then (in the same buffer):
+  unsigned long long* d_lt_stats = nullptr;  // [2] work counters
+  uint32_t* d_lt_ov = nullptr;               // fault flag
   int32_t* d_lt_spill = nullptr;
   int64_t lt_spill_words = 0;
 };
@@ -458,9 +457,8 @@ static void scene_free(ane_scene* s)
   dfree(s->d_sh_orig); dfree(s->d_sh_dir); dfree(s->d_sh_hits); dfree(s->d_sh_work);
   dfree(s->d_sh_spill);
   dfree(s->d_lt_lights); dfree(s->d_lt_orig); dfree(s->d_lt_dir); dfree(s->d_lt_tmax); dfree(s->d_lt_hits);
-  dfree(s->d_lt_dist); dfree(s->d_lt_dirs); dfree(s->d_lt_wt); dfree(s->d_lt_idx); dfree(s->d_lt_order); dfree(s->d_lt_work);
-  dfree(s->d_lt_stats);
-  dfree(s->d_lt_ov); dfree(s->d_lt_spill);
+  dfree(s->d_lt_dirs); dfree(s->d_lt_wt); dfree(s->d_lt_idx); dfree(s->d_lt_order); dfree(s->d_lt_work);
+  dfree(s->d_lt_spill);
   s->sgc.destroy();
   if (s->ev0) (void)hipEventDestroy(s->ev0);
   if (s->ev1) (void)hipEventDestroy(s->ev1);
@@ -2015,9 +2013,10 @@ extern "C" int ane_scene_light_shadows(ane_scene* s, const ane_light* lights, in
   }
   hipStream_t st = S(stream);
   const int64_t m = (int64_t)num_lights * kLightRays;
+  constexpr int kLtWords = kTraceWorkWords + 5;  // claim counters, 2 work counters (64-bit), the fault flag
   if (s->lt_kmax == 0) {  // set last: a setup that failed part-way is redone from scratch
     dfree(s->d_lt_order); dfree(s->d_lt_dirs); dfree(s->d_lt_wt); dfree(s->d_lt_idx);
-    dfree(s->d_lt_work); dfree(s->d_lt_stats); dfree(s->d_lt_ov);
+    dfree(s->d_lt_work);
     std::vector<float> dirs((size_t)kLightRays * 3), wt((size_t)kLightRays * 64);
     fibonacci_dirs(kLightRays, dirs.data());  // worldDirFromFibonacciIndex, light_shadow.rgen:27-38
     light_weights(dirs.data(), wt.data());
@@ -2049,22 +2048,21 @@ extern "C" int ane_scene_light_shadows(ane_scene* s, const ane_light* lights, in
     ANE_CHECK_HIP(hipMemcpy(s->d_lt_dirs, dirs.data(), sizeof(float) * dirs.size(), hipMemcpyHostToDevice));
     ANE_CHECK_HIP(hipMemcpy(s->d_lt_wt, lw.data(), sizeof(float) * lw.size(), hipMemcpyHostToDevice));
     ANE_CHECK_HIP(hipMemcpy(s->d_lt_idx, li.data(), sizeof(int32_t) * li.size(), hipMemcpyHostToDevice));
-    ANE_TRY(dalloc(&s->d_lt_work, kTraceWorkWords, nullptr));
-    ANE_TRY(dalloc(&s->d_lt_stats, 2, nullptr));
-    ANE_TRY(dalloc(&s->d_lt_ov, 1, nullptr));
+    ANE_TRY(dalloc(&s->d_lt_work, kLtWords, nullptr));
+    s->d_lt_stats = reinterpret_cast<unsigned long long*>(s->d_lt_work + kTraceWorkWords);
+    s->d_lt_ov = s->d_lt_work + kTraceWorkWords + 4;
     s->lt_kmax = kmax;
   }
   if (num_lights > s->lt_cap) {
     ANE_CHECK_HIP(hipStreamSynchronize(st));
     dfree(s->d_lt_lights); dfree(s->d_lt_orig); dfree(s->d_lt_dir); dfree(s->d_lt_tmax);
-    dfree(s->d_lt_hits); dfree(s->d_lt_dist);
+    dfree(s->d_lt_hits);
     s->lt_cap = 0;
     ANE_TRY(dalloc(&s->d_lt_lights, 8 * (int64_t)num_lights, nullptr));
     ANE_TRY(dalloc(&s->d_lt_orig, 3 * m, nullptr));
     ANE_TRY(dalloc(&s->d_lt_dir, 3 * m, nullptr));
     ANE_TRY(dalloc(&s->d_lt_tmax, m, nullptr));
     ANE_TRY(dalloc(&s->d_lt_hits, m, nullptr));
-    ANE_TRY(dalloc(&s->d_lt_dist, m, nullptr));
     s->lt_cap = num_lights;
   }
   const int64_t lanes = trace_lanes_per_launch();
@@ -2080,10 +2078,7 @@ extern "C" int ane_scene_light_shadows(ane_scene* s, const ane_light* lights, in
   ANE_CHECK_HIP(hipMemcpyAsync(s->d_lt_lights, lights, sizeof(ane_light) * (size_t)num_lights,
                                hipMemcpyHostToDevice, st));
   launch_light_rays(s->d_lt_lights, num_lights, s->d_lt_dirs, s->d_lt_order, s->d_lt_orig, s->d_lt_dir,
-                    s->d_lt_tmax, st);
-  fill_u32(s->d_lt_work, 0u, kTraceWorkWords, st);
-  fill_u32(reinterpret_cast<uint32_t*>(s->d_lt_stats), 0u, 4, st);
-  fill_u32(s->d_lt_ov, 0u, 1, st);
+                    s->d_lt_tmax, s->d_lt_work, kLtWords, st);
   TraceArgs a{};
   a.sc = s->view;
   a.g.rays = 1;
@@ -2100,9 +2095,8 @@ extern "C" int ane_scene_light_shadows(ane_scene* s, const ane_light* lights, in
   a.t_max = 0.0f;          // per ray: the light's range (rgen:66)
   a.ray_tmax = s->d_lt_tmax;
   launch_trace(a, false, true, counters2 != nullptr, st);  // closest hit: rchit reports gl_HitTEXT
-  launch_light_dist(s->d_lt_lights, num_lights, s->d_lt_order, s->d_lt_hits, s->d_lt_dist, dist_img, st);
-  launch_light_moments(s->d_lt_lights, num_lights, s->d_lt_dist, s->d_lt_wt, s->d_lt_idx, s->lt_kmax,
-                       moments_img, st);
+  launch_light_moments(s->d_lt_lights, num_lights, s->d_lt_order, s->d_lt_hits, s->d_lt_wt, s->d_lt_idx, s->lt_kmax,
+                       dist_img, moments_img, st);
   ANE_CHECK_HIP(hipGetLastError());
   if (counters2) {
     unsigned long long c2[2] = {0, 0};

@@ -312,12 +312,11 @@ void launch_shadow_rays(const float* depth, int W, int H, const float* ivp16, co
 // with weight above 0.001 in the summation order, padded with weight 0
 static constexpr int kLightRays = 1024;
 // order[j]: the ray traced in slot j of each light (a permutation of 0..1023)
+// clear: [nclear] words set to 0 before the launches that follow
 void launch_light_rays(const float* lights, int n, const float* dirs, const uint32_t* order, float* orig,
-                       float* rdir, float* tmax, hipStream_t s);
-void launch_light_dist(const float* lights, int n, const uint32_t* order, const ane_hit* hits, float* dist,
-                       float* dist_img, hipStream_t s);
-void launch_light_moments(const float* lights, int n, const float* dist, const float* lw,
-                          const int32_t* lidx, int kmax, float* mom, hipStream_t s);
+                       float* rdir, float* tmax, uint32_t* clear, int nclear, hipStream_t s);
+void launch_light_moments(const float* lights, int n, const uint32_t* order, const ane_hit* hits, const float* lw,
+                          const int32_t* lidx, int kmax, float* dist_img, float* mom, hipStream_t s);
 void launch_shadow_resolve(const float* depth, const ane_hit* hits, int64_t n, float* vis, hipStream_t s,
                            const uint32_t* skip_if_set = nullptr);
 // mirror reflections: reflection rays in slot order (pixel_slot_count(W, H) of them), the

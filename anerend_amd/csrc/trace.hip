@@ -1432,10 +1432,13 @@ static constexpr int kLightSide = 32;  // LIGHT_DIR_DIST_PIX_SIZE: ray y * 32 + 
 // Fibonacci direction r over [0.1, range]; a disabled light (color.w < 0.5) casts
 // no ray (zero direction).  Slot j of a light traces ray order[j], so that the
 // lanes of a wave follow neighbouring directions.
+// clear: [nclear] words the traversal that follows counts in.
 __global__ __launch_bounds__(256) void k_light_rays(const float* lights, int n, const float* dirs,
                                                     const uint32_t* order, float* orig, float* rdir,
-                                                    float* tmax)
+                                                    float* tmax, uint32_t* clear, int nclear)
 {
+  if (blockIdx.x == 0)
+    for (int k = threadIdx.x; k < nclear; k += blockDim.x) clear[k] = 0u;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (int64_t)n * kLightRays) return;
   const int l = (int)(i / kLightRays), r = (int)order[i % kLightRays];
@@ -1449,46 +1452,55 @@ __global__ __launch_bounds__(256) void k_light_rays(const float* lights, int n, 
   tmax[i] = L[3];
 }
 
-// light_shadow.rchit:15-18 (hit distance), light_shadow.rmiss:12-15 (the range),
-// light_shadow.rgen:54-58 (disabled light: 0), stored at rgen:43-49, 84
-__global__ __launch_bounds__(256) void k_light_dist(const float* lights, int n, const uint32_t* order,
-                                                    const ane_hit* hits, float* dist, float* dist_img)
-{
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)n * kLightRays) return;
-  const int l = (int)(i / kLightRays), r = (int)order[i % kLightRays];
-  const float* L = lights + 8 * (int64_t)l;
-  const float d = L[7] < 0.5f ? 0.0f : (hits[i].tri >= 0 ? hits[i].t : L[3]);
-  dist[(int64_t)l * kLightRays + r] = d;
-  if (dist_img)
-    dist_img[(int64_t)(r / kLightSide) * kLightSide * n + (int64_t)kLightSide * l + r % kLightSide] = d;
-}
-
-// light_shadow_sum.comp:16-71: one thread per texel of one light's 8x8 tile.  The
-// shader visits the 1024 rays x outer, y inner and adds those whose weight
-// pow(max(0, dot(dir, octDir)), 50) is above 0.001 (63-69 of them per texel).
+// The distances of one light, light_shadow.rchit:15-18 (the hit), light_shadow.rmiss:12-15
+// (the range), light_shadow.rgen:54-58 (0 for a disabled light), kept in LDS and stored to
+// the distance image (rgen:43-49, 84), then light_shadow_sum.comp:16-71: one thread per texel
+// of the light's 8x8 tile.  The shader visits the 1024 rays x outer, y inner and adds those
+// whose weight pow(max(0, dot(dir, octDir)), 50) is above 0.001 (63-69 of them per texel).
 // lw / lidx [k][texel] list exactly those (weight, ray) pairs of each texel in that
 // order, padded with weight 0, so the sums are the shader's, operation for
 // operation, whatever the launch shape.  Texel (tx, ty) of light l lands at
 // (10 l + 1 + tx, ty) of the RG32F image; the border columns are not written.
-__global__ __launch_bounds__(64) void k_light_moments(const float* lights, int n, const float* dist,
-                                                      const float* lw, const int32_t* lidx, int kmax,
-                                                      float* mom)
+// A light's sums are one serial chain per texel; with few lights the launch is as long as
+// the round trips to the table, so kLightPre pairs are read ahead of their sums and the other
+// waves store the image meanwhile (64 lights: 24 + 5 us in two kernels with 8 pairs ahead).
+static constexpr int kLightPre = 24;
+__global__ __launch_bounds__(256) void k_light_moments(const float* lights, int n, const uint32_t* order,
+                                                       const ane_hit* hits, const float* lw, const int32_t* lidx,
+                                                       int kmax, float* dist_img, float* mom)
 {
   __shared__ float ds[kLightRays];
   const int l = blockIdx.x, t = threadIdx.x;
-  for (int k = t; k < kLightRays; k += 64) ds[k] = dist[(int64_t)l * kLightRays + k];
+  const float range = lights[8 * (int64_t)l + 3];
+  const bool off = lights[8 * (int64_t)l + 7] < 0.5f;  // sum.comp:35
+  const ane_hit* h = hits + (int64_t)l * kLightRays;
+  for (int k = t; k < kLightRays; k += 256) ds[order[k]] = off ? 0.0f : (h[k].tri >= 0 ? h[k].t : range);
   __syncthreads();
+  if (t >= 64) {
+    if (dist_img)
+      for (int r = t - 64; r < kLightRays; r += 192)
+        dist_img[(int64_t)(r / kLightSide) * kLightSide * n + (int64_t)kLightSide * l + r % kLightSide] = ds[r];
+    return;
+  }
   float ar = 0.0f, ag = 0.0f, aw = 0.0f;
-  if (!(lights[8 * (int64_t)l + 7] < 0.5f)) {  // sum.comp:35
-#pragma unroll 8
-    for (int k = 0; k < kmax; ++k) {
-      const float w = lw[k * 64 + t];
-      if (w > 0.001f) {
-        const float d = ds[lidx[k * 64 + t]];
-        ar += w * d;
-        ag += w * d * d;
-        aw += w;
+  if (!off) {
+    for (int k0 = 0; k0 < kmax; k0 += kLightPre) {
+      float w[kLightPre];
+      int32_t r[kLightPre];
+#pragma unroll
+      for (int k = 0; k < kLightPre; ++k) {
+        const int q = k0 + k < kmax ? k0 + k : kmax - 1;
+        w[k] = lw[q * 64 + t];
+        r[k] = lidx[q * 64 + t];
+      }
+#pragma unroll
+      for (int k = 0; k < kLightPre; ++k) {
+        if (k0 + k < kmax && w[k] > 0.001f) {
+          const float d = ds[r[k]];
+          ar += w[k] * d;
+          ag += w[k] * d * d;
+          aw += w[k];
+        }
       }
     }
     if (aw > 1e-6f) {
@@ -1502,29 +1514,20 @@ __global__ __launch_bounds__(64) void k_light_moments(const float* lights, int n
 }
 
 void launch_light_rays(const float* lights, int n, const float* dirs, const uint32_t* order, float* orig,
-                       float* rdir, float* tmax, hipStream_t s)
+                       float* rdir, float* tmax, uint32_t* clear, int nclear, hipStream_t s)
 {
   const int64_t m = (int64_t)n * kLightRays;
   if (m <= 0) return;
   hipLaunchKernelGGL(k_light_rays, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, lights, n, dirs,
-                     order, orig, rdir, tmax);
+                     order, orig, rdir, tmax, clear, nclear);
 }
 
-void launch_light_dist(const float* lights, int n, const uint32_t* order, const ane_hit* hits, float* dist,
-                       float* dist_img, hipStream_t s)
-{
-  const int64_t m = (int64_t)n * kLightRays;
-  if (m <= 0) return;
-  hipLaunchKernelGGL(k_light_dist, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, lights, n, order,
-                     hits, dist, dist_img);
-}
-
-void launch_light_moments(const float* lights, int n, const float* dist, const float* lw,
-                          const int32_t* lidx, int kmax, float* mom, hipStream_t s)
+void launch_light_moments(const float* lights, int n, const uint32_t* order, const ane_hit* hits, const float* lw,
+                          const int32_t* lidx, int kmax, float* dist_img, float* mom, hipStream_t s)
 {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_light_moments, dim3((unsigned)n), dim3(64), 0, s, lights, n, dist, lw, lidx, kmax,
-                     mom);
+  hipLaunchKernelGGL(k_light_moments, dim3((unsigned)n), dim3(256), 0, s, lights, n, order, hits, lw, lidx, kmax,
+                     dist_img, mom);
 }
 
 void launch_shadow_rays(const float* depth, int W, int H, const float* ivp16, const float* light3,
