@@ -9,6 +9,7 @@
 #include <mutex>
 #include <string>
 #include <algorithm>
+#include <atomic>
 #include <utility>
 #include <vector>
 
@@ -177,11 +178,11 @@ using namespace ane;
 // for any-hit rays that all share it, and the key they were built for.  A key
 // is first only remembered; the second request with it builds the grid on the
 // request's stream, so a direction or scene that changes with every call keeps
-// the traversal and never pays a build.  One exception: when a grid of the same
-// scene version (another direction) was built and found valid, and the request
-// has at least ANE_SUNGRID_EAGER_RAYS rays per triangle (a build costs about as
-// much as the traversal of 5 probe rays per triangle saves), the first request
-// with a new direction builds: a sun that moves every frame over a static scene.
+// the traversal and never pays a build.  One exception, a sun that moves every frame
+// over a static scene: a new direction builds at once when a grid of the same scene
+// version was found in use and the request has ANE_SUNGRID_EAGER_RAYS rays per triangle,
+// or when the request before had the same scene version, no grid of it was found out of
+// use and the rays pay for the build by themselves (sun_grid_pays).
 // ===========================================================================
 #ifndef ANE_SUNGRID_DENSITY
 #define ANE_SUNGRID_DENSITY 1.0  // cells per triangle
@@ -193,8 +194,14 @@ using namespace ane;
 #define ANE_SUNGRID_EAGER 0  // 1: build on the first request with a key
 #endif
 #ifndef ANE_SUNGRID_EAGER_RAYS
-#define ANE_SUNGRID_EAGER_RAYS 6  // rays per triangle from which a new direction alone builds at once
+#define ANE_SUNGRID_EAGER_RAYS 6  // rays per triangle from which a new direction builds at once over a known-valid scene
 #endif
+// Rays from which a moving direction builds at once also before a build was found in use:
+// about 2.5 per triangle, what a build costs against what it saves (one FP16 layer range of
+// terrain1m with a moving sun, traversed / built: 2.1 rays per triangle 636 / 654 us, 3.2
+// 844 / 795 us, 8.5 1850 / 1499 us), above its launches (13k triangles: 131k rays 184 / 216
+// us, 524k 260 / 269 us, 1.05M 353 / 330 us).
+static bool sun_grid_pays(int64_t rays, int32_t ntri) { return 2 * rays >= 5 * (int64_t)ntri + 1200000; }
 
 struct SunGridCache {
   SunGridParams* params = nullptr;
@@ -265,6 +272,19 @@ struct SunGridCache {
       known = pend;
     }
   }
+  // reads the flag of the build of k back, unless an earlier read-back is still on its way
+  // (recorded again in every frame its event would never complete for a host that runs ahead)
+  int read_back(const Key& k, hipStream_t st)
+  {
+    if (pending) return ANE_OK;
+    if (!h_valid) ANE_CHECK_HIP(hipHostMalloc((void**)&h_valid, sizeof(uint32_t), hipHostMallocDefault));
+    if (!ev) ANE_CHECK_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    ANE_CHECK_HIP(hipMemcpyAsync(h_valid, &params->valid, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    ANE_CHECK_HIP(hipEventRecord(ev, st));
+    pend = k;
+    pending = true;
+    return ANE_OK;
+  }
   // device buffers for a scene of ntri triangles: about ANE_SUNGRID_DENSITY cells
   // per triangle (at most 4096 x 4096), ANE_SUNGRID_CAPACITY entries per triangle
   int alloc(int32_t ntri)
@@ -319,15 +339,22 @@ struct SunGridCache {
     if (!capturing) poll();  // no event queries under capture
     if (built == k) {
       *use = true;
+      if (!capturing && !(known == k)) ANE_TRY(read_back(k, st));
       if (valid) *valid = capturing ? -1 : known_valid();  // a graph keeps both ways: the grid may change before a replay
       return ANE_OK;
     }
-    const bool eager = known.set && known.scene == scene && known.version == version && last_valid == 1 &&
-                       rays >= (int64_t)ANE_SUNGRID_EAGER_RAYS * ntri;
+    // a new direction over the scene version of a build that was found in use, or of the
+    // last request while no build of that version was found out of use
+    const bool judged = known.set && known.scene == scene && known.version == version;
+    const bool valid_scene = judged && last_valid == 1;
+    const bool moving = valid_scene || (!judged && seen.set && seen.scene == scene && seen.version == version);
+    const bool eager = (valid_scene && rays >= (int64_t)ANE_SUNGRID_EAGER_RAYS * ntri) ||
+                       (moving && sun_grid_pays(rays, ntri));
     if (!ANE_SUNGRID_EAGER && !eager && !(seen == k)) {
       seen = k;
       return ANE_OK;
     }
+    seen = k;
     ANE_TRY(alloc(ntri));
     SunGridParams p;
     sun_grid_setup(p, dir3, g, g);
@@ -335,14 +362,7 @@ struct SunGridCache {
     ANE_CHECK_HIP(hipGetLastError());
     built = k;
     ++builds;
-    if (!capturing) {
-      if (!h_valid) ANE_CHECK_HIP(hipHostMalloc((void**)&h_valid, sizeof(uint32_t), hipHostMallocDefault));
-      if (!ev) ANE_CHECK_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-      ANE_CHECK_HIP(hipMemcpyAsync(h_valid, &params->valid, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-      ANE_CHECK_HIP(hipEventRecord(ev, st));
-      pend = k;
-      pending = true;
-    }
+    if (!capturing) ANE_TRY(read_back(k, st));
     *use = true;
     return ANE_OK;
   }
@@ -470,6 +490,10 @@ static void scene_free(ane_scene* s)
   }
 }
 
+// Versions never repeat: a context's derived data is keyed by its scene's address and
+// version, and a new scene can lie where an old one was.
+static std::atomic<uint64_t> g_scene_version{0};
+
 static int validate_instances(const ane_scene* s, const ane_instance* inst, int32_t ninst)
 {
   for (int32_t k = 0; k < ninst; ++k) {
@@ -563,7 +587,7 @@ static int scene_apply_node_format(ane_scene* s, hipStream_t st, bool fitted = f
 // full LBVH build from the uploaded instances
 static int scene_build(ane_scene* s, hipStream_t st, bool write_inst)
 {
-  ++s->version;
+  s->version = ++g_scene_version;
   ANE_CHECK_HIP(hipEventRecord(s->ev0, st));
   const int n = s->ntri;
   launch_flatten(s->view, s->d_world, s->d_tri_inst, s->d_tri_rec, s->d_cpart, s->d_cbounds, write_inst, st);
@@ -609,7 +633,7 @@ static int scene_build(ane_scene* s, hipStream_t st, bool write_inst)
 
 static int scene_refit_dev(ane_scene* s, hipStream_t st)
 {
-  ++s->version;
+  s->version = ++g_scene_version;
   ANE_CHECK_HIP(hipEventRecord(s->ev0, st));
   const int n = s->ntri;
   // a refit keeps the Morton order: the fit makes the leaf-order triangles straight
