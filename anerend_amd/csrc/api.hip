@@ -401,7 +401,8 @@ struct ane_scene {
   uint32_t* d_cbounds = nullptr;
   uint32_t* d_cpart = nullptr;  // per-block centroid-bound partials of a build
   uint4* d_qnodes = nullptr;    // quantized traversal nodes (allocated when first used)
-  bool boxes_stale = false;     // the last fit left the 64-byte records' boxes out (quantized traversal)
+  uint4* d_hnodes = nullptr;    // grid nodes (closest-hit traversal)
+  GridFrame* d_hframe = nullptr;
   int32_t node_format = ANE_NODES_AUTO;
   uint32_t* d_scratch = nullptr;
   uint32_t* d_info = nullptr;   // fit plan read back at a build: level offsets, counts, tree depth
@@ -471,7 +472,7 @@ static void scene_free(ane_scene* s)
   dfree(s->d_inst); dfree(s->d_inv); dfree(s->d_tri_inst); dfree(s->d_tri_rec); dfree(s->d_inst_off);
   dfree(s->d_world); dfree(s->d_keys); dfree(s->d_keys2); dfree(s->d_ids); dfree(s->d_ids2);
   dfree(s->d_nodes); dfree(s->d_leaf_parent); dfree(s->d_tris);
-  dfree(s->d_node_box); dfree(s->d_cbounds); dfree(s->d_cpart); dfree(s->d_qnodes); dfree(s->d_scratch);
+  dfree(s->d_node_box); dfree(s->d_cbounds); dfree(s->d_cpart); dfree(s->d_qnodes); dfree(s->d_hnodes); dfree(s->d_hframe); dfree(s->d_scratch);
   dfree(s->d_info); dfree(s->d_topo); dfree(s->d_cross); dfree(s->d_cross_kids); dfree(s->d_top); dfree(s->d_ndepth); dfree(s->d_units);
   dfree(s->d_unit_root); dfree(s->d_uheight); dfree(s->d_stray); dfree(s->d_uscratch);
   dfree(s->d_sh_orig); dfree(s->d_sh_dir); dfree(s->d_sh_hits); dfree(s->d_sh_work);
@@ -557,23 +558,9 @@ static int scene_fit_qnodes(ane_scene* s, uint4** out)
   return ANE_OK;
 }
 
-// The 64-byte records' boxes, when the last fit left them out: a fit from the
-// current leaf-order triangles that writes them (the traversal of quantized
-// records does not read them; a change of node format and the BVH read-back do).
-static int scene_full_boxes(ane_scene* s, hipStream_t st)
-{
-  if (!s->boxes_stale) return ANE_OK;
-  launch_fit(s->d_tris, s->ntri, s->d_nodes, s->d_node_box, nullptr, s->d_topo, s->d_leaf_parent, s->d_units,
-             s->nunits, s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, nullptr, nullptr, nullptr, st, true);
-  ANE_CHECK_HIP(hipGetLastError());
-  s->boxes_stale = false;
-  return ANE_OK;
-}
-
 // fitted: the fit that just ran wrote the quantized records (scene_fit_qnodes)
 static int scene_apply_node_format(ane_scene* s, hipStream_t st, bool fitted = false)
 {
-  if (!fitted) ANE_TRY(scene_full_boxes(s, st));
   if (!scene_wants_qnodes(s)) {
     s->view.qnodes = nullptr;
     return ANE_OK;
@@ -612,8 +599,8 @@ static int scene_build(ane_scene* s, hipStream_t st, bool write_inst)
   uint4* qn = nullptr;
   ANE_TRY(scene_fit_qnodes(s, &qn));
   launch_fit(s->d_tris, n, s->d_nodes, s->d_node_box, qn, s->d_topo, s->d_leaf_parent, s->d_units, s->nunits,
-             s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, nullptr, nullptr, s->d_uheight, st, qn == nullptr);
-  s->boxes_stale = qn != nullptr;
+             s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, nullptr, nullptr, s->d_uheight, st);
+  launch_grid_nodes(s->d_nodes, n, s->d_hframe, s->d_hnodes, st);
   ANE_TRY(scene_apply_node_format(s, st, qn != nullptr));
   uint32_t* d_depth = s->d_info + 132;
   if (launch_tree_depth(s->d_topo, n, s->d_unit_root, s->d_uheight, s->nunits, s->d_top, s->d_uscratch,
@@ -622,8 +609,13 @@ static int scene_build(ane_scene* s, hipStream_t st, bool write_inst)
   ANE_CHECK_HIP(hipGetLastError());
   ANE_CHECK_HIP(hipEventRecord(s->ev1, st));
   uint32_t depth = 0;
-  if (n >= 2) ANE_CHECK_HIP(hipMemcpyAsync(&depth, d_depth, 4, hipMemcpyDeviceToHost, st));
+  GridFrame frame{};
+  if (n >= 2) {
+    ANE_CHECK_HIP(hipMemcpyAsync(&depth, d_depth, 4, hipMemcpyDeviceToHost, st));
+    ANE_CHECK_HIP(hipMemcpyAsync(&frame, s->d_hframe, sizeof(frame), hipMemcpyDeviceToHost, st));
+  }
   ANE_CHECK_HIP(hipStreamSynchronize(st));
+  s->view.hnodes = grid_frame_ok(frame) ? s->d_hnodes : nullptr;
   // the deepest internal nodes have two leaf children: leaf depth = number of internal levels
   s->depth = (int32_t)depth;
   ANE_CHECK_HIP(hipEventElapsedTime(&s->build_ms, s->ev0, s->ev1));
@@ -642,8 +634,8 @@ static int scene_refit_dev(ane_scene* s, hipStream_t st)
   uint4* qn = nullptr;
   ANE_TRY(scene_fit_qnodes(s, &qn));
   launch_fit(s->d_tris, n, s->d_nodes, s->d_node_box, qn, s->d_topo, s->d_leaf_parent, s->d_units, s->nunits,
-             s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, &view, s->d_ids, nullptr, st, qn == nullptr);
-  s->boxes_stale = qn != nullptr;
+             s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, &view, s->d_ids, nullptr, st);
+  launch_grid_nodes(s->d_nodes, n, s->d_hframe, s->d_hnodes, st);
   s->world_stale = true;
   ANE_TRY(scene_apply_node_format(s, st, qn != nullptr));
   ANE_CHECK_HIP(hipGetLastError());
@@ -719,6 +711,8 @@ extern "C" int ane_scene_create(const float* vertices, int64_t num_vertices, con
   ANE_A(d_ids, n);
   ANE_A(d_ids2, n);
   ANE_A(d_nodes, n > 1 ? n - 1 : 1);
+  ANE_A(d_hnodes, 2 * (n > 1 ? n - 1 : 1));
+  ANE_A(d_hframe, 1);
   ANE_A(d_leaf_parent, n);
   ANE_A(d_tris, n * 3);
   ANE_A(d_node_box, (n > 1 ? n - 1 : 1) * 6);
@@ -760,6 +754,7 @@ extern "C" int ane_scene_create(const float* vertices, int64_t num_vertices, con
   v.vertices = s->d_vertices; v.indices = s->d_indices; v.meshes = s->d_meshes; v.mats = s->d_mats;
   v.inst = s->d_inst; v.inv_xform = s->d_inv; v.tri_inst = s->d_tri_inst; v.tri_rec = s->d_tri_rec; v.inst_tri_off = s->d_inst_off;
   v.nodes = reinterpret_cast<const float4*>(s->d_nodes); v.tris = s->d_tris;
+  v.hnodes = s->d_hnodes; v.hframe = s->d_hframe;
   v.ntri = s->ntri; v.ninst = s->ninst;
   st = scene_build(s, sm, true);
   if (st) return bail(st);
@@ -864,9 +859,6 @@ extern "C" int ane_scene_debug_bvh(const ane_scene* s, uint64_t* keys, uint32_t*
 {
   if (!s) return fail(ANE_ERR_INVALID_ARG, "scene is NULL");
   const int64_t n = s->ntri;
-  // the boxes come from the 64-byte records, refitted first if the last fit left
-  // them out (derived data: the scene is unchanged otherwise)
-  if (boxes) ANE_TRY(scene_full_boxes(const_cast<ane_scene*>(s), nullptr));
   ANE_CHECK_HIP(hipDeviceSynchronize());
   if (keys) ANE_CHECK_HIP(hipMemcpy(keys, s->d_keys, 8 * n, hipMemcpyDeviceToHost));
   if (ids) ANE_CHECK_HIP(hipMemcpy(ids, s->d_ids, 4 * n, hipMemcpyDeviceToHost));

@@ -624,6 +624,87 @@ void launch_quantize_nodes(const NodeBuild* nodes, int n, uint4* q, hipStream_t 
   hipLaunchKernelGGL(k_quantize_nodes, dim3((unsigned)((n - 1 + 255) / 256)), dim3(256), 0, s, nodes, n, q);
 }
 
+// The frame of the grid nodes: the bounds of the root's two children.
+__global__ void k_grid_frame(const NodeBuild* nodes, GridFrame* f)
+{
+  const NodeBuild nd = nodes[0];
+  const float lo[3] = {fminf(nd.a.x, nd.b.x), fminf(nd.a.z, nd.b.z), fminf(nd.c.x, nd.c.z)};
+  const float hi[3] = {fmaxf(nd.a.y, nd.b.y), fmaxf(nd.a.w, nd.b.w), fmaxf(nd.c.y, nd.c.w)};
+  GridFrame g;
+  g.r = 0.0f;
+  bool finite = true;
+  for (int k = 0; k < 3; ++k) {
+    g.o[k] = lo[k];
+    // 65535 cells span the extent: the cell is rounded up twice
+    g.s[k] = fmaxf((hi[k] - lo[k]) / 65535.0f * 1.000001f, 1e-30f);
+    g.r = fmaxf(g.r, fmaxf(fabsf(lo[k]), fabsf(hi[k])));
+    finite = finite && __builtin_isfinite(lo[k]) && __builtin_isfinite(hi[k]);
+  }
+  if (!finite) g.r = __builtin_inff();
+  g.sum = 0.0f;
+  g.count = 0u;
+  *f = g;
+}
+
+// Grid nodes from the fitted 64-byte records, one thread per node.  Cell indices are
+// floor / ceil in binary64 (their 1e-16 is far inside the traversal's slab margin).  Every
+// kGridSample-th block adds the area growth of its child boxes to the frame's sums.
+static constexpr int kGridSample = 32;
+__device__ __forceinline__ void grid_box(const GridFrame& f, const float* lo, const float* hi, uint32_t* w, float& grow,
+                                         uint32_t& n)
+{
+  float e[3], q[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double a = floor(((double)lo[k] - (double)f.o[k]) / (double)f.s[k]);
+    const double b = ceil(((double)hi[k] - (double)f.o[k]) / (double)f.s[k]);
+    const uint32_t l = (uint32_t)fmin(fmax(a, 0.0), 65535.0), u = (uint32_t)fmin(fmax(b, 0.0), 65535.0);
+    w[k] = l | u << 16;
+    e[k] = hi[k] - lo[k];
+    q[k] = (float)(u - l) * f.s[k] + 2.0f * kSlabMargin * f.r;  // as the traversal sees it
+  }
+  const float area = e[0] * e[1] + e[1] * e[2] + e[2] * e[0];
+  if (area > 0.0f) {
+    grow += fminf((q[0] * q[1] + q[1] * q[2] + q[2] * q[0]) / area, 16.0f);
+    n += 1u;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_grid_nodes(const NodeBuild* nodes, int n, GridFrame* frame, uint4* q)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  float grow = 0.0f;
+  uint32_t cnt = 0u;
+  if (i < n - 1) {
+    const GridFrame f = *frame;
+    const NodeBuild nd = nodes[i];
+    const float l0[3] = {nd.a.x, nd.a.z, nd.c.x}, h0[3] = {nd.a.y, nd.a.w, nd.c.y};
+    const float l1[3] = {nd.b.x, nd.b.z, nd.c.z}, h1[3] = {nd.b.y, nd.b.w, nd.c.w};
+    uint32_t w[6];
+    grid_box(f, l0, h0, w, grow, cnt);
+    grid_box(f, l1, h1, w + 3, grow, cnt);
+    q[2 * (int64_t)i] = make_uint4(w[0], w[1], w[2], w[3]);
+    q[2 * (int64_t)i + 1] = make_uint4(w[4], w[5], (uint32_t)nd.d.x, (uint32_t)nd.d.y);
+  }
+  if (blockIdx.x % kGridSample != 0) return;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    grow += __shfl_xor(grow, d, 64);
+    cnt += __shfl_xor(cnt, d, 64);
+  }
+  if ((threadIdx.x & 63) == 0 && cnt) {
+    atomicAdd(&frame->sum, grow);
+    atomicAdd(&frame->count, cnt);
+  }
+}
+
+void launch_grid_nodes(const NodeBuild* nodes, int n, GridFrame* frame, uint4* q, hipStream_t s)
+{
+  if (n < 2) return;
+  hipLaunchKernelGGL(k_grid_frame, dim3(1), dim3(1), 0, s, nodes, frame);
+  hipLaunchKernelGGL(k_grid_nodes, dim3((unsigned)((n - 1 + 255) / 256)), dim3(256), 0, s, nodes, n, frame, q);
+}
+
 // Fit one internal node from its (already final) children: child boxes into
 // the traversal record (and its quantized record when qn is set), the union
 // into node_box.
@@ -686,7 +767,7 @@ template <bool FROM_REC>
 __global__ __launch_bounds__(kSpan) void k_fit_span(SceneK sc, const uint32_t* ids, float4* tris, NodeBuild* nodes,
                                                     float* node_box, uint4* qn, const int4* topo,
                                                     const int32_t* leaf_parent, const int2* units, int n,
-                                                    uint8_t* uheight, int full)
+                                                    uint8_t* uheight)
 {
   extern __shared__ int4 span_lds[];
   int4* nd = span_lds;                                       // [kSpan] topology of nodes s..
@@ -743,12 +824,10 @@ __global__ __launch_bounds__(kSpan) void k_fit_span(SceneK sc, const uint32_t* i
       float l0[3], h0[3], l1[3], h1[3];
       span_child_box(lb, ib, d.x, s, l0, h0);
       span_child_box(lb, ib, d.y, s, l1, h1);
-      if (full) {  // the 64-byte record's boxes (a scene that traverses quantized records skips them)
-        NodeBuild* q = &nodes[p];
-        q->a = make_float4(l0[0], h0[0], l0[1], h0[1]);
-        q->b = make_float4(l1[0], h1[0], l1[1], h1[1]);
-        q->c = make_float4(l0[2], h0[2], l1[2], h1[2]);
-      }
+      NodeBuild* q = &nodes[p];
+      q->a = make_float4(l0[0], h0[0], l0[1], h0[1]);
+      q->b = make_float4(l1[0], h1[0], l1[1], h1[1]);
+      q->c = make_float4(l0[2], h0[2], l1[2], h1[2]);
       float u[6];
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
@@ -1071,7 +1150,7 @@ int launch_tree_depth(const int4* topo, int n, const int32_t* unit_root, const u
 void launch_fit(float4* tris, int n, NodeBuild* nodes, float* node_box, uint4* qnodes, const int4* topo,
                 const int32_t* leaf_parent, const int2* units, int nunits, const int32_t* stray, int nstray,
                 const int32_t* cross, const int2* cross_kids, const std::vector<int32_t>& cross_begin, const SceneK* refit,
-                const uint32_t* ids, uint8_t* uheight, hipStream_t s, bool full_boxes)
+                const uint32_t* ids, uint8_t* uheight, hipStream_t s)
 {
   if (n < 2 || cross_begin.size() < 2) {
     if (refit && n == 1) launch_refit_tris(*refit, ids, n, tris, s);
@@ -1092,11 +1171,11 @@ void launch_fit(float4* tris, int n, NodeBuild* nodes, float* node_box, uint4* q
   if (nunits > 0) {
     if (refit)
       hipLaunchKernelGGL(k_fit_span<true>, dim3((unsigned)nunits), dim3(kSpan), kSpanLds, s, *refit, ids, tris,
-                         nodes, node_box, qnodes, topo, leaf_parent, units, n, uheight, full_boxes ? 1 : 0);
+                         nodes, node_box, qnodes, topo, leaf_parent, units, n, uheight);
     else
       hipLaunchKernelGGL(k_fit_span<false>, dim3((unsigned)nunits), dim3(kSpan), kSpanLds, s, none,
                          (const uint32_t*)nullptr, tris, nodes, node_box, qnodes, topo, leaf_parent, units, n,
-                         uheight, full_boxes ? 1 : 0);
+                         uheight);
   }
   // the crossing nodes, deepest level first: a launch per level below the top
   // ones, then the top levels in one workgroup

@@ -106,6 +106,8 @@ struct SceneK {
   const uint32_t* inst_tri_off; // [ninst + 1]
   const float4* nodes;          // [ntri - 1][4] traversal nodes
   const uint4* qnodes;          // [ntri - 1][2] quantized traversal nodes, or null (use nodes)
+  const uint4* hnodes;          // [ntri - 1][2] grid nodes of the closest-hit traversal
+  const struct GridFrame* hframe; // their frame
   const float4* tris;           // [ntri][3] sorted world triangles (v0.w = id bits)
   int32_t ntri;
   int32_t ninst;
@@ -133,6 +135,29 @@ struct NodeBuild {
 // Karras split), leaves (~position) where the leaf flag is set.
 ANE_HD float qnode_step(uint32_t ebyte) { return __builtin_bit_cast(float, (ebyte - 128u + 127u) << 23); }
 ANE_HD float qnode_bound(float o, uint32_t q, float step) { return o + (float)q * step; }
+
+// Grid node, 32 bytes (2 x uint4), for the closest-hit traversal: the bounds of both
+// children on a 2^16 grid over the scene's bounds, rounded outward:
+//   w0..w2 child 0 x, y, z: lower | upper << 16;  w3..w5 child 1;  w6 left, w7 right
+// (children as in NodeBuild).  A bound is o + q * s in the frame.  A node costs two
+// 16-byte loads per ray instead of four.
+struct GridFrame {
+  float o[3], s[3];   // lower corner and cell size (rounded up)
+  float r;            // largest coordinate magnitude of the bounds
+  float sum;          // sampled child boxes: the growth of their area by the rounding,
+  uint32_t count;     // summed, and their number
+};
+// Outward margin of the grid traversal's slabs, of the largest coordinate magnitude of
+// scene and ray origin.  In units of 2^-24 of it, the rounding of the slab constants and
+// products adds up to 10 and that of the triangle test (translation, shear, edge functions,
+// t) to about 26; this is 67.
+static constexpr float kSlabMargin = 4e-6f;
+// The grid is used while it is finite and boxes grow by at most half on average; a scene
+// whose detail is far finer than 2^-16 of its extent keeps its full nodes.
+ANE_HD bool grid_frame_ok(const GridFrame& f)
+{
+  return f.r < 1e18f && f.sum <= 1.5f * (float)f.count;
+}
 
 ANE_HD uint32_t mesh_of(uint32_t custom) { return (custom >> 10) & 0x3FFFu; }
 ANE_HD uint32_t mat_of(uint32_t custom) { return custom & 0x3FFu; }

@@ -54,13 +54,12 @@ int launch_tree_depth(const int4* topo, int n, const int32_t* unit_root, const u
 // uheight (nullable): the height of each treelet's root, by treelet.
 // qnodes (nullable): the quantized records are written too, from the same child
 // boxes (the bytes launch_quantize_nodes makes from the fitted nodes).
-// full_boxes false: the treelet nodes' boxes in the 64-byte records are left
-// as they were (a scene that traverses the quantized records; the top nodes'
-// are written either way).
 void launch_fit(float4* tris, int n, NodeBuild* nodes, float* node_box, uint4* qnodes, const int4* topo,
                 const int32_t* leaf_parent, const int2* units, int nunits, const int32_t* stray, int nstray,
                 const int32_t* cross, const int2* cross_kids, const std::vector<int32_t>& cross_begin, const SceneK* refit,
-                const uint32_t* ids, uint8_t* uheight, hipStream_t s, bool full_boxes = true);
+                const uint32_t* ids, uint8_t* uheight, hipStream_t s);
+// the frame and the grid nodes from the fitted 64-byte records
+void launch_grid_nodes(const NodeBuild* nodes, int n, GridFrame* frame, uint4* q, hipStream_t s);
 // cross_kids[k]: the children of crossing node cross[k], for the total crossing
 // nodes of the fit plan (once per build)
 void launch_cross_kids(const int32_t* cross, const int4* topo, int total, int2* kids, hipStream_t s);

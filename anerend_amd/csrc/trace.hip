@@ -15,6 +15,8 @@
 //                    (sungrid.hip).  Q = true reads the scene's quantized 32-byte nodes
 //                    (large scenes), else the 64-byte nodes; caller rays may carry a
 //                    per-ray t_max
+//   k_trace_closest  the traversal of the closest-hit rays that need no work counts:
+//                    the same hits from 32-byte grid nodes
 //   k_probe_shadow_grid  with a sun grid: the shadow rays of the probe hits against
 //                    the triangles of their cells, the candidates of a wave's 64 rays
 //                    spread over its lanes
@@ -100,6 +102,22 @@ static constexpr int kRefill = ANE_TRACE_REFILL;
 static constexpr int kLeafBatchProbe = ANE_TRACE_LEAFBATCH;
 static constexpr int kLeafBatchRays = ANE_TRACE_LEAFBATCH_RAYS;
 static constexpr int kShadeUnroll = ANE_SHADE_UNROLL;
+// closest-hit traversal of grid nodes, terrain1m / 4.04M-triangle update: 6 waves per SIMD
+// 1.179 / 12.98 ms against 1.143 / 13.02; leaf batches of 12 / 16 lanes 1.137 / 1.140 against
+// 1.143, but 701 / 716 us against 671 for the 65k rays over 246k triangles; 5 / 8 steps per
+// refill check 1.143 / 1.149 and 204 / 198 us against 198 for one probe layer
+#ifndef ANE_CLOSEST_WAVES
+#define ANE_CLOSEST_WAVES 7
+#endif
+#ifndef ANE_CLOSEST_LEAFBATCH
+#define ANE_CLOSEST_LEAFBATCH 8
+#endif
+#ifndef ANE_CLOSEST_LEAFBATCH_RAYS
+#define ANE_CLOSEST_LEAFBATCH_RAYS 1  // caller rays (4 / 8: 115 / 127 us against 109 for 64 lights)
+#endif
+#ifndef ANE_CLOSEST_STEPS
+#define ANE_CLOSEST_STEPS 7
+#endif
 
 bool trace_grid_supported() { return true; }
 
@@ -294,6 +312,44 @@ __device__ __forceinline__ f3 hit_geom_pos(const SceneK& sc, int32_t id, float u
   return xform_point(sc.inst[h.inst].transform, pos);
 }
 
+// The next chunk of a wave (lanes `im` wait for rays): claim i of counter k is chunk
+// (k + i) % K of the i-th group of K chunks; nrays when every ray was in a first chunk or
+// claimed (in 32 bits: a wave makes one claim past the end).  cend: the chunk's end.
+__device__ __forceinline__ uint32_t claim_chunk(const TraceArgs& a, uint32_t nrays, uint64_t im, int lane, uint32_t& cend)
+{
+  uint32_t base = nrays;
+  if (a.static_rays < nrays) {
+    constexpr uint32_t K = (uint32_t)kTraceCounters;
+    const uint32_t k = blockIdx.x & (K - 1u);
+    const int who = __ffsll((unsigned long long)im) - 1;
+    uint32_t i = 0u;
+    if (lane == who) i = atomicAdd(a.work + k * kTraceCounterStride, 1u);
+    i = (uint32_t)__builtin_amdgcn_readlane((int)i, who);
+    base = a.static_rays + (i * K + ((k + i) & (K - 1u))) * kChunk;
+    base = base < nrays ? base : nrays;
+  }
+  cend = base + kChunk < nrays ? base + kChunk : nrays;
+  return base;
+}
+
+// The two child boxes and the children of a quantized node (layout next to NodeBuild).
+__device__ __forceinline__ void decode_qnode(const uint4* nq, float4& na, float4& nb, float4& nc, int32_t& L, int32_t& R)
+{
+  const uint4 q0 = nq[0], q1 = nq[1];
+  const float ox = __uint_as_float(q0.x), oy = __uint_as_float(q0.y), oz = __uint_as_float(q0.z);
+  const float sx = qnode_step(q0.w & 0xFFu), sy = qnode_step((q0.w >> 8) & 0xFFu);
+  const float sz = qnode_step((q0.w >> 16) & 0xFFu);
+  na = make_float4(qnode_bound(ox, q1.x & 0xFFu, sx), qnode_bound(ox, q1.x >> 24, sx),
+                   qnode_bound(oy, (q1.x >> 8) & 0xFFu, sy), qnode_bound(oy, q1.y & 0xFFu, sy));
+  nb = make_float4(qnode_bound(ox, (q1.y >> 16) & 0xFFu, sx), qnode_bound(ox, (q1.z >> 8) & 0xFFu, sx),
+                   qnode_bound(oy, q1.y >> 24, sy), qnode_bound(oy, (q1.z >> 16) & 0xFFu, sy));
+  nc = make_float4(qnode_bound(oz, (q1.x >> 16) & 0xFFu, sz), qnode_bound(oz, (q1.y >> 8) & 0xFFu, sz),
+                   qnode_bound(oz, q1.z & 0xFFu, sz), qnode_bound(oz, q1.z >> 24, sz));
+  const int32_t g = (int32_t)q1.w;
+  L = (q0.w >> 24) & 1u ? ~g : g;
+  R = (q0.w >> 25) & 1u ? ~(g + 1) : g + 1;
+}
+
 // ---------------------------------------------------------------------------
 // traversal
 //   RAYS = false: probe rays.  A lane traces its primary ray (closest hit,
@@ -387,23 +443,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
     const uint64_t am = __ballot(ray >= 0);
     const uint32_t need = (uint32_t)__popcll(im);
     if (need != 0u && (am == 0ull || need >= (uint32_t)kRefill)) {
-      if (cbeg >= cend) {  // the next chunk: none when every ray was in a first chunk
-        uint32_t base = nrays;
-        if (a.static_rays < nrays) {
-          // claim i of counter k: chunk (k + i) % K of the i-th group of K chunks
-          // (in 32 bits: a wave makes one claim past the end)
-          constexpr uint32_t K = (uint32_t)kTraceCounters;
-          const uint32_t k = blockIdx.x & (K - 1u);
-          const int who = __ffsll((unsigned long long)im) - 1;
-          uint32_t i = 0u;
-          if (lane == who) i = atomicAdd(a.work + k * kTraceCounterStride, 1u);
-          i = (uint32_t)__builtin_amdgcn_readlane((int)i, who);
-          base = a.static_rays + (i * K + ((k + i) & (K - 1u))) * kChunk;
-          base = base < nrays ? base : nrays;
-        }
-        cbeg = base;
-        cend = base + kChunk < nrays ? base + kChunk : nrays;
-      }
+      if (cbeg >= cend) cbeg = claim_chunk(a, nrays, im, lane, cend);
       const uint32_t avail = cend > cbeg ? cend - cbeg : 0u;
       const uint32_t rank = (uint32_t)__popcll(im & lt);
       if (idle) {
@@ -470,21 +510,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
         float4 na, nb, nc;
         int32_t L, R;
         if (Q) {
-          // quantized node: decode the two child boxes (layout next to NodeBuild)
-          const uint4* nq = sc.qnodes + 2 * (int64_t)node;
-          const uint4 q0 = nq[0], q1 = nq[1];
-          const float ox = __uint_as_float(q0.x), oy = __uint_as_float(q0.y), oz = __uint_as_float(q0.z);
-          const float sx = qnode_step(q0.w & 0xFFu), sy = qnode_step((q0.w >> 8) & 0xFFu);
-          const float sz = qnode_step((q0.w >> 16) & 0xFFu);
-          na = make_float4(qnode_bound(ox, q1.x & 0xFFu, sx), qnode_bound(ox, q1.x >> 24, sx),
-                           qnode_bound(oy, (q1.x >> 8) & 0xFFu, sy), qnode_bound(oy, q1.y & 0xFFu, sy));
-          nb = make_float4(qnode_bound(ox, (q1.y >> 16) & 0xFFu, sx), qnode_bound(ox, (q1.z >> 8) & 0xFFu, sx),
-                           qnode_bound(oy, q1.y >> 24, sy), qnode_bound(oy, (q1.z >> 16) & 0xFFu, sy));
-          nc = make_float4(qnode_bound(oz, (q1.x >> 16) & 0xFFu, sz), qnode_bound(oz, (q1.y >> 8) & 0xFFu, sz),
-                           qnode_bound(oz, q1.z & 0xFFu, sz), qnode_bound(oz, q1.z >> 24, sz));
-          const int32_t g = (int32_t)q1.w;
-          L = (q0.w >> 24) & 1u ? ~g : g;
-          R = (q0.w >> 25) & 1u ? ~(g + 1) : g + 1;
+          decode_qnode(sc.qnodes + 2 * (int64_t)node, na, nb, nc, L, R);
         } else {
           const float4* nd = sc.nodes + 4 * (int64_t)node;
           na = nd[0];
@@ -590,6 +616,325 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
       atomicAdd(&a.stats[1], ct);
       atomicAdd(&a.stats[2], sn);
       atomicAdd(&a.stats[3], st);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// closest-hit traversal (probe rays, and caller rays asked for their closest hit)
+//   The hits are those of k_trace: the closest hit is the minimum of (t, triangle id)
+//   over all triangles, whatever boxes are visited, as long as no box around a hit is
+//   culled.  k_trace is bound by VALU issue and, right behind it, by the L1: a CU serves
+//   one access of a lane per clock, and a 64-byte node is four of them (terrain1m launch:
+//   452 M accesses in 489 M clocks of the CUs).  So:
+//   - Grid nodes (GridFrame): two accesses per node, 249 M for the launch.
+//   - A slab is one conversion and one fma: t = q * (s * inv) + c with c = (o - origin -+
+//     margin) * inv per ray; the bound pairs are rotated by the ray's signs so that near
+//     and far planes need no minimum and maximum.  The margin (kSlabMargin) makes the boxes
+//     a superset of the exact test's, and no 1 + 2 gamma(3) factor is needed.
+//   - A lane at a leaf keeps it in `node` until the next leaf batch and pops after it, so
+//     that one compare (node < lim) tells who goes on; the stack pointer is the LDS address
+//     of its ring, whose bottom entry ends the traversal; barycentrics and reciprocals lie
+//     in LDS, so that 7 waves per SIMD need no spills.
+//   terrain1m update 1.325 -> 1.143 ms, one of its layers 249 -> 198 us, 64 lights 129 ->
+//   102 us, 1080p mirror pass 474 -> 423 us; 385 M VALU instructions in 0.6 ms, which is
+//   VALU issue again.
+//   Rays whose products could leave the normal range (a direction component below 1e-29,
+//   huge coordinates) make their wave take the full (or quantized) nodes with the exact slab
+//   test of k_trace, which also keeps its decisions on rays that lie in a box face.  Scenes
+//   too fine for the grid at their last build, the counting variants, any-hit caller rays
+//   (their hit id is the first found) and launches with a step limit keep k_trace; a refit
+//   that outgrows the grid takes the exact slabs (1.37 ms).
+// ---------------------------------------------------------------------------
+static constexpr int64_t kFastMaxTris = (int64_t)1 << 25;  // 32-bit byte offsets of 64-byte nodes and 48-byte triangles
+
+__device__ __forceinline__ float uniform_f(float x)
+{
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+
+// The child boxes of a node in the scene's traversal layout under the exact slab test.
+__device__ __forceinline__ void exact_boxes(const SceneK& sc, int32_t node, const RayPre& r, float tmin, float tbest,
+                                            int32_t& L, int32_t& R, bool& b0, bool& b1, float& tn0, float& tn1)
+{
+  float4 na, nb, nc;
+  if (sc.qnodes) {
+    decode_qnode(sc.qnodes + 2 * (int64_t)node, na, nb, nc, L, R);
+  } else {
+    const float4* nd = sc.nodes + 4 * (int64_t)node;
+    na = nd[0];
+    nb = nd[1];
+    nc = nd[2];
+    const float4 nn = nd[3];
+    L = __float_as_int(nn.x);
+    R = __float_as_int(nn.y);
+  }
+  b0 = box_test(r, na.x, na.y, na.z, na.w, nc.x, nc.y, tmin, tbest, tn0);
+  b1 = box_test(r, nb.x, nb.y, nb.z, nb.w, nc.z, nc.w, tmin, tbest, tn1);
+}
+
+// min(x, y) of numbers, without the quieting of a y that the compiler cannot see through
+__device__ __forceinline__ float min_number(float x, float y)
+{
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+
+template <bool RAYS>
+__global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST_WAVES))) void k_trace_closest(TraceArgs a)
+{
+  constexpr int32_t kDone = 0x7FFFFFFF;  // the lane's traversal has ended (>= lim, not a leaf)
+  constexpr uint32_t kSlot = kTB * 4;    // bytes of one stack level of the block
+  constexpr uint32_t kRing = kSS * kSlot;
+  constexpr int kLeafBatch = RAYS ? ANE_CLOSEST_LEAFBATCH_RAYS : ANE_CLOSEST_LEAFBATCH;
+  constexpr int kSteps = ANE_CLOSEST_STEPS;  // traversal steps per refill check
+  const bool sgrid = !RAYS && a.sg.list != nullptr && a.sg.params->valid != 0u;
+  __shared__ int32_t stk[kSS * kTB];
+  // per lane, what only refills, hits and exact slabs touch (registers set the occupancy):
+  // the best hit's barycentrics and the reciprocal direction
+  __shared__ float cold[5][kTB];
+  if (RAYS && a.skip_if_set && *a.skip_if_set != 0u) return;  // a sun grid answered these rays
+  if (!RAYS) clock_begin(a.clk, kTraceRays);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const SceneK& sc = a.sc;
+  const float tmin = RAYS ? a.t_min : a.g.t_min;
+  const float tmax0 = RAYS ? a.t_max : a.g.t_max;
+  const int n = a.g.rays;
+  const uint32_t nrays = (uint32_t)a.nrays;
+  const int32_t root = (sc.ntri >= 2) ? 0 : (sc.ntri == 1 ? ~0 : kDone);
+  const uint32_t lim = sc.ntri >= 2 ? (uint32_t)sc.ntri - 1u : 0u;  // internal nodes
+  // refill checks a ray may live through: far above the visits of any valid hierarchy and
+  // the waits of its lane, so only a malformed one ends a ray here
+  const uint32_t patience = 2u * (uint32_t)sc.ntri + (1u << 22);
+  const char* const nbase = reinterpret_cast<const char*>(sc.hnodes);
+  const char* const tbase = reinterpret_cast<const char*>(sc.tris);
+  // the frame, in scalar registers (it is the same for every lane)
+  GridFrame fr{};
+  if (sc.ntri >= 2) fr = *sc.hframe;
+  const bool grid = __builtin_amdgcn_readfirstlane(grid_frame_ok(fr) ? 1 : 0) != 0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    fr.o[k] = uniform_f(fr.o[k]);
+    fr.s[k] = uniform_f(fr.s[k]);
+  }
+  fr.r = uniform_f(fr.r);
+
+  int32_t out = -1;  // output slot of the lane's ray, -1: idle
+  bool exhausted = false;
+  bool sph = false;    // the lane's ray is an any-hit (shadow) ray
+  bool exact = false;  // the lane's ray needs the exact slab test
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kTB / 64) + (tid >> 6))) * kChunk;
+  uint32_t cbeg = first < nrays ? first : nrays;
+  uint32_t cend = cbeg + kChunk < nrays ? cbeg + kChunk : nrays;
+  f3 ro = mk(0.0f, 0.0f, 0.0f), sh = ro;  // origin, watertight shear
+  int32_t kk = 0;                         // its axes kx | ky << 2 | kz << 4
+  f3 ci = ro, cn = ro, cf = ro;  // slab constants: per cell, of the near and of the far planes
+  uint32_t rx = 0u, ry = 0u, rz = 0u;  // rotation that puts a bound pair's near plane in the low half
+  float tbest = 0.0f;
+  int32_t bid = -1, node = kDone;
+  const uint32_t sp0 = (uint32_t)tid * 4u;
+  uint32_t sp = sp0;  // byte offset of the next stack entry, the ring's wrap not yet taken
+  uint32_t left_checks = 0u;
+
+  auto entry = [&](uint32_t p) -> int32_t& {
+    return *reinterpret_cast<int32_t*>(reinterpret_cast<char*>(stk) + (p & (kRing - 1u)));
+  };
+  auto spilled = [&](uint32_t p) -> int32_t& {
+    return a.spill[(int64_t)(p / kSlot - kSS) * a.total_lanes + (blockIdx.x * kTB + (sp0 >> 2))];
+  };
+  auto start = [&](const RayPre& r) {
+    ro = r.o;
+    sh = mk(r.sx, r.sy, r.sz);
+    kk = r.kx | (r.ky << 2) | (r.kz << 4);
+    cold[2][tid] = r.inv.x;
+    cold[3][tid] = r.inv.y;
+    cold[4][tid] = r.inv.z;
+    const float om = fmaxf(fabsf(ro.x), fmaxf(fabsf(ro.y), fabsf(ro.z)));
+    const float im = fmaxf(fabsf(r.inv.x), fmaxf(fabsf(r.inv.y), fabsf(r.inv.z)));
+    const float m = kSlabMargin * fmaxf(fr.r, om);
+    exact = !(im * fmaxf(fr.r + om + m, 1e8f) < 1e37f);
+    ci = mk(fr.s[0] * r.inv.x, fr.s[1] * r.inv.y, fr.s[2] * r.inv.z);
+    const f3 d = mk(fr.o[0] - ro.x, fr.o[1] - ro.y, fr.o[2] - ro.z);
+    // the near planes are the lower ones along a positive direction, each moved outward
+    const float mx = r.inv.x < 0.0f ? -m : m, my = r.inv.y < 0.0f ? -m : m, mz = r.inv.z < 0.0f ? -m : m;
+    cn = mk((d.x - mx) * r.inv.x, (d.y - my) * r.inv.y, (d.z - mz) * r.inv.z);
+    cf = mk((d.x + mx) * r.inv.x, (d.y + my) * r.inv.y, (d.z + mz) * r.inv.z);
+    rx = r.inv.x < 0.0f ? 16u : 0u;
+    ry = r.inv.y < 0.0f ? 16u : 0u;
+    rz = r.inv.z < 0.0f ? 16u : 0u;
+    bid = -1;
+    node = root;
+    entry(sp0) = kDone;  // the bottom of the stack ends the traversal
+    sp = sp0 + kSlot;
+    left_checks = patience;
+  };
+  auto pop = [&]() {
+    sp -= kSlot;
+    node = entry(sp);
+    if (sp >= kRing) entry(sp) = spilled(sp);
+  };
+  // one box: near and far distances from its three rotated bound pairs
+  auto box = [&](uint32_t wx, uint32_t wy, uint32_t wz, float& tn) -> bool {
+    wx = __builtin_amdgcn_alignbit(wx, wx, rx);
+    wy = __builtin_amdgcn_alignbit(wy, wy, ry);
+    wz = __builtin_amdgcn_alignbit(wz, wz, rz);
+    tn = fmaxf(fmaxf(fmaf((float)(wx & 0xFFFFu), ci.x, cn.x), fmaf((float)(wy & 0xFFFFu), ci.y, cn.y)),
+               fmaxf(fmaf((float)(wz & 0xFFFFu), ci.z, cn.z), tmin));
+    const float tf = fminf(fminf(fmaf((float)(wx >> 16), ci.x, cf.x), fmaf((float)(wy >> 16), ci.y, cf.y)),
+                           min_number(fmaf((float)(wz >> 16), ci.z, cf.z), tbest));
+    return tn <= tf;
+  };
+
+  for (;;) {
+    // ---- finish ended traversals; a probe ray that hit continues as its shadow ray ----
+    if (out >= 0) {
+      // a child index out of range or a ray without end (a malformed hierarchy) is a fault
+      const bool bad = node >= 0 ? ((uint32_t)node >= lim && node != kDone) : (uint32_t)~node >= (uint32_t)sc.ntri;
+      if (bad || --left_checks == 0u) {
+        *a.overflow = 1u;
+        node = kDone;
+      }
+      if (node == kDone) {
+        const float bu = cold[0][tid], bv = cold[1][tid];
+        if (RAYS || !sph) {
+          ane_hit h;
+          h.tri = bid;
+          h.t = (bid >= 0) ? tbest : 0.0f;
+          h.u = (bid >= 0) ? bu : 0.0f;
+          h.v = (bid >= 0) ? bv : 0.0f;
+          a.hits[out] = h;
+        }
+        if (!RAYS && !sph && bid >= 0 && !sgrid) {
+          // shadow ray from the hit position toward the sun (rchit:44-66), same lane
+          HitGeom hg;
+          const f3 p = hit_geom_pos(sc, bid, bu, bv, hg);
+          RayPre r;
+          load_dirpre(r, a.dirpre + 3 * n, p);
+          sph = true;
+          tbest = tmax0;
+          start(r);
+        } else {
+          if (!RAYS && !sgrid) a.shadow[out] = sph ? (uint8_t)(bid >= 0 ? 1 : 0) : (uint8_t)255;
+          out = -1;
+        }
+      }
+    }
+    // ---- refill idle lanes (between steps) ----
+    const bool idle = (out < 0) && !exhausted;
+    const uint64_t im = __ballot(idle);
+    const uint64_t am = __ballot(out >= 0);
+    const uint32_t need = (uint32_t)__popcll(im);
+    if (need != 0u && (am == 0ull || need >= (uint32_t)kRefill)) {
+      if (cbeg >= cend) cbeg = claim_chunk(a, nrays, im, lane, cend);
+      const uint32_t avail = cend > cbeg ? cend - cbeg : 0u;
+      const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(im >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)im, 0u));
+      if (idle) {
+        if (avail == 0u) {
+          exhausted = true;
+        } else if (rank < avail) {
+          const uint32_t gidx = cbeg + rank;
+          bool none = false;
+          RayPre r;
+          if (RAYS) {
+            out = (int32_t)gidx;
+            const f3 d = ld3(a.ray_dir + 3 * (int64_t)gidx);
+            none = (d.x == 0.0f && d.y == 0.0f && d.z == 0.0f) || !__builtin_isfinite(d.x) ||
+                   !__builtin_isfinite(d.y) || !__builtin_isfinite(d.z);
+            ray_setup(r, ld3(a.ray_orig + 3 * (int64_t)gidx), d);
+          } else {
+            // independent loads: processing-order ray setup, probe origin, output slot
+            const uint32_t ql = (uint32_t)(((uint64_t)gidx * a.div_magic) >> a.div_shift);
+            const uint32_t j = gidx - ql * (uint32_t)n;
+            const float4 po = a.probe_org[a.probe_base + (int)ql];
+            load_dirpre(r, a.dirpre + 3 * j, mk(po.x, po.y, po.z));
+            out = (int32_t)ql * n + (int)a.order[j];
+            sph = false;
+          }
+          tbest = tmax0;
+          if (RAYS && a.ray_tmax) tbest = a.ray_tmax[gidx];
+          start(r);
+          if (none) node = kDone;
+        }
+      }
+      cbeg += need < avail ? need : avail;
+    }
+    if (am == 0ull && __ballot(out >= 0) == 0ull) {
+      if (__ballot(!exhausted) == 0ull) break;
+      continue;
+    }
+    const bool slow = !grid || __ballot(exact && out >= 0) != 0ull;  // wave-uniform
+    // ---- traversal steps ----
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      if ((uint32_t)node < lim) {
+        int32_t L, Rc;
+        float tn0, tn1;
+        bool b0, b1;
+        if (!slow) {
+          const uint4* nq = reinterpret_cast<const uint4*>(nbase + (uint32_t)node * 32u);
+          const uint4 q0 = nq[0], q1 = nq[1];
+          L = (int32_t)q1.z;
+          Rc = (int32_t)q1.w;
+          b0 = box(q0.x, q0.y, q0.z, tn0);
+          b1 = box(q0.w, q1.x, q1.y, tn1);
+        } else {
+          RayPre r;
+          r.o = ro;
+          r.inv = mk(cold[2][tid], cold[3][tid], cold[4][tid]);
+          exact_boxes(sc, node, r, tmin, tbest, L, Rc, b0, b1, tn0, tn1);
+        }
+        const bool left = b0 && !(b1 && tn1 < tn0);
+        node = left ? L : Rc;
+        if (b0 && b1) {
+          // push the far child (LDS ring; the oldest entry spills when full)
+          bool room = true;
+          if (sp >= kRing) {
+            room = (int)(sp / kSlot) - kSS < a.spill_depth;
+            if (room) spilled(sp) = entry(sp);
+          }
+          if (room) {
+            entry(sp) = left ? Rc : L;
+            sp += kSlot;
+          } else {
+            *a.overflow = 1u;
+            node = kDone;
+          }
+        }
+        if (!(b0 || b1)) pop();
+      }
+      const uint64_t lm = __ballot(node < 0);
+      if (lm != 0ull) {
+        if (__popcll(lm) >= kLeafBatch || __ballot((uint32_t)node < lim) == 0ull) {
+          if (node < 0 && (uint32_t)~node < (uint32_t)sc.ntri) {
+            const float4* tv = reinterpret_cast<const float4*>(tbase + (uint32_t)~node * 48u);
+            const float4 v0 = tv[0], v1 = tv[1], v2 = tv[2];
+            RayPre r;
+            r.o = ro;
+            r.sx = sh.x;
+            r.sy = sh.y;
+            r.sz = sh.z;
+            r.kx = kk & 3;
+            r.ky = (kk >> 2) & 3;
+            r.kz = kk >> 4;
+            float t, tu, tw;
+            bool ended = false;
+            if (tri_test(r, mk(v0.x, v0.y, v0.z), mk(v1.x, v1.y, v1.z), mk(v2.x, v2.y, v2.z), tmin, tbest, t, tu, tw)) {
+              const int32_t id = __float_as_int(v0.w);
+              if (sph || t < tbest || (t == tbest && id < bid)) {
+                bid = id;
+                tbest = t;
+                cold[0][tid] = tu;
+                cold[1][tid] = tw;
+              }
+              ended = sph;  // any hit ends a shadow ray
+            }
+            pop();
+            if (ended) node = kDone;
+          }
+        }
+      }
     }
   }
 }
@@ -768,7 +1113,7 @@ int trace_lanes_per_launch()
   int dev = 0, cus = 0, per = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_trace<false, false, false, false>, kTB, 0);
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_trace_closest<false>, kTB, 0);
   if (cus <= 0) cus = 256;
   if (per <= 0) per = 8;
   g_lanes = cus * per * kTB;
@@ -792,7 +1137,11 @@ void launch_trace(const TraceArgs& a, bool any_hit, bool rays, bool count, hipSt
     if (b.sc.qnodes) hipLaunchKernelGGL((k_trace<S, R, C, true>), dim3(blocks), dim3(kTB), 0, s, b);  \
     else hipLaunchKernelGGL((k_trace<S, R, C, false>), dim3(blocks), dim3(kTB), 0, s, b);             \
   } while (0)
-  if (rays) {
+  const bool fast = !count && !(rays && any_hit) && a.step_limit == 0u && a.sc.hnodes && a.sc.ntri <= kFastMaxTris;
+  if (fast) {
+    if (rays) hipLaunchKernelGGL(k_trace_closest<true>, dim3(blocks), dim3(kTB), 0, s, b);
+    else hipLaunchKernelGGL(k_trace_closest<false>, dim3(blocks), dim3(kTB), 0, s, b);
+  } else if (rays) {
     if (any_hit) { if (count) ANE_TR(true, true, true); else ANE_TR(true, true, false); }
     else { if (count) ANE_TR(false, true, true); else ANE_TR(false, true, false); }
   } else {
