@@ -208,7 +208,7 @@ struct SunGridCache {
   uint32_t* acc = nullptr;    // [6][256] per-block bounds
   uint32_t* start = nullptr;  // [cells + 1] counts, scanned into starts
   uint32_t* cur = nullptr;    // [cells] scatter cursors
-  uint32_t* list = nullptr;   // [cap] candidates
+  uint2* list = nullptr;      // [cap] candidates
   uint32_t* scan = nullptr;   // scan scratch
   float* est = nullptr;       // build scratch, sun_grid_scratch_words(ntri)
   int64_t est_words = 0;

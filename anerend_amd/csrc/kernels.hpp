@@ -150,13 +150,22 @@ struct SunGridParams {
 struct SunGridK {
   const SunGridParams* params;  // device
   const uint32_t* start;        // [gx * gy + 1] first candidate of each cell
-  const uint32_t* list;         // candidates (sorted triangle positions); null: no grid
+  const uint2* list;            // candidates (sorted triangle position, sun_bounds in the cell); null: no grid
 };
 __host__ __device__ __forceinline__ int sun_cell(float v, float o, float inv, int n)
 {
   float f = floorf((v - o) * inv);
   f = fminf(fmaxf(f, 0.0f), (float)(n - 1));  // also NaN -> 0
   return (int)f;
+}
+// Where coordinate v lies in cell k of its row, in 256ths of a cell (clamped): with the
+// grid's margin on the triangles' side, a point within a triangle's projection lies within
+// the triangle's sun_bounds (the rounding here is below 1e-6 of the grid's cells, the
+// margin at least 1e-5 of them)
+__host__ __device__ __forceinline__ uint32_t sun_local(float v, float o, float inv, int k)
+{
+  const float f = floorf(((v - o) * inv - (float)k) * 256.0f);
+  return (uint32_t)fminf(fmaxf(f, 0.0f), 255.0f);
 }
 void sun_grid_setup(SunGridParams& g, const float* dir3, int gx, int gy);
 
@@ -170,7 +179,7 @@ void launch_shadow_mask_grid(const float* depth, int W, int H, const float* ivp1
 // estimate, per-block cell counts)
 int64_t sun_grid_scratch_words(int32_t ntri);
 void launch_sun_grid_build(const SceneK& sc, const SunGridParams& g, SunGridParams* d_params, uint32_t* acc,
-                           uint32_t* cnt, uint32_t* cur, uint32_t* list, uint32_t cap, uint32_t* scan_scratch,
+                           uint32_t* cnt, uint32_t* cur, uint2* list, uint32_t cap, uint32_t* scan_scratch,
                            float* est, const ClockArg& clk, int stage, hipStream_t s);
 // probe traces can take a sun grid (k_probe_shadow_grid runs their shadow rays)
 bool trace_grid_supported();

@@ -185,6 +185,18 @@ __device__ __forceinline__ bool sun_tri_overlaps_cell(const SunGridParams& g, co
   return true;
 }
 
+// The triangle's widened projected rectangle within cell (x, y), in 256ths of the cell:
+// x lower | upper << 8 | y lower << 16 | upper << 24
+__device__ __forceinline__ uint32_t sun_bounds(const SunGridParams& g, const CellRange& c, int x, int y)
+{
+  const float xl = fminf(fminf(c.px[0], c.px[1]), c.px[2]) - g.margin;
+  const float xh = fmaxf(fmaxf(c.px[0], c.px[1]), c.px[2]) + g.margin;
+  const float yl = fminf(fminf(c.py[0], c.py[1]), c.py[2]) - g.margin;
+  const float yh = fmaxf(fmaxf(c.py[0], c.py[1]), c.py[2]) + g.margin;
+  return sun_local(xl, g.x0, g.icw, x) | sun_local(xh, g.x0, g.icw, x) << 8 | sun_local(yl, g.y0, g.ich, y) << 16 |
+         sun_local(yh, g.y0, g.ich, y) << 24;
+}
+
 // Every (triangle, cell of its rectangle) pair of a wave's 64 triangles, spread
 // over the wave's lanes 64 at a time: f(ok, j, cj, x, y) runs in every lane of
 // the wave, round after round; ok says whether the lane has a pair in the round,
@@ -343,7 +355,7 @@ __global__ __launch_bounds__(256) void k_sun_cursor(const uint32_t* start, int64
 // cursor atomic per pair.  Both reserve from the same cursors, so the runs never
 // overlap.
 __global__ __launch_bounds__(256) void k_sun_scatter(const float4* tris, int32_t ntri, const SunGridParams* gp,
-                                                     const uint32_t* start, uint32_t* cur, uint32_t* list,
+                                                     const uint32_t* start, uint32_t* cur, uint2* list,
                                                      uint32_t cap, const uint16_t* tab, float* part)
 {
   __shared__ float ts[256], tk[256];  // per lane's triangle: the counts of its cells, and their number
@@ -383,7 +395,7 @@ __global__ __launch_bounds__(256) void k_sun_scatter(const float4* tris, int32_t
       const int64_t cell = (int64_t)y * g.gx + x;
       const int l = (y - win.y0) * win.w + (x - win.x0);
       const uint32_t k = win.n ? atomicAdd(&wcur[l], 1u) : atomicAdd(&cur[cell], 1u);
-      if (k < cap) list[k] = (uint32_t)(p0 + j);
+      if (k < cap) list[k] = make_uint2((uint32_t)(p0 + j), sun_bounds(g, cj, x, y));
       sc = win.n ? wtot[l] : (float)(start[cell + 1] - start[cell]);
       sk = 1.0f;
     }
@@ -467,7 +479,7 @@ void sun_grid_setup(SunGridParams& g, const float* dir3, int gx, int gy)
 }
 
 void launch_sun_grid_build(const SceneK& sc, const SunGridParams& g, SunGridParams* d_params, uint32_t* acc,
-                           uint32_t* cnt, uint32_t* cur, uint32_t* list, uint32_t cap, uint32_t* scan_scratch,
+                           uint32_t* cnt, uint32_t* cur, uint2* list, uint32_t cap, uint32_t* scan_scratch,
                            float* est, const ClockArg& clk, int stage, hipStream_t s)
 {
   const int64_t ncell = (int64_t)g.gx * g.gy;

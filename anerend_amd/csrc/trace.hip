@@ -955,23 +955,48 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
 // a hit).  Every shadow flag of the launch is written here (255: no hit).
 // ---------------------------------------------------------------------------
 #ifndef ANE_SHADOW_U
-#define ANE_SHADOW_U 2  // 1, 2, 4 and 8 swept: 238, 230, 250 and 383 µs on terrain1m
+#define ANE_SHADOW_U 3  // candidates per lane and round (1 / 2 / 4: 1.124 / 1.120 / 1.126 ms against 1.116 for the update)
 #endif
-static constexpr int kShadowU = ANE_SHADOW_U;  // candidates per lane and round
+static constexpr int kShadowU = ANE_SHADOW_U;
 
-// The candidates of a wave's 64 rays spread over its lanes: lane l's ray (origin
-// p, direction of r, list [b, b + c) of the sun grid) has its candidates tested
-// with the watertight any-hit test, 64 at a time, ray after ray and in list order
-// within a ray (kShadowU per lane and round, every load of a round issued before
-// any test).  key[l] (this wave's 64 LDS slots, set to 2 c + 1 by the caller)
-// ends as the earliest event of lane l's list in list order: 2 pos for a hit,
-// 2 pos + 1 for an entry out of range when STOP_ON_BAD (which also raises
-// *overflow; otherwise such entries are skipped).  Tests after a known event are
-// skipped.  All lanes of the wave must call it (shuffles).
+// The sun-grid cell of point p: its candidate list [b, b + c) and p's place in the cell
+// (x | y << 8, in 256ths).
+__device__ __forceinline__ void sun_lookup(const SunGridK& sg, const SunGridParams& g, f3 p, uint32_t& b, uint32_t& c,
+                                           uint32_t& q)
+{
+  const float X = comp(p, g.kx) - g.sx * comp(p, g.kz);
+  const float Y = comp(p, g.ky) - g.sy * comp(p, g.kz);
+  const int cx = sun_cell(X, g.x0, g.icw, g.gx), cy = sun_cell(Y, g.y0, g.ich, g.gy);
+  const uint32_t* st = sg.start + ((int64_t)cy * g.gx + cx);
+  b = st[0];
+  c = st[1] - b;
+  q = sun_local(X, g.x0, g.icw, cx) | sun_local(Y, g.y0, g.ich, cy) << 8;
+}
+
+// A wave's queue of candidates that passed the bounds check (LDS)
+struct SunQueue {
+  uint32_t id[64 * (kShadowU + 1)], pos[64 * (kShadowU + 1)];
+  uint8_t ray[64 * (kShadowU + 1)];
+};
+
+// The candidates of a wave's 64 rays spread over its lanes: lane l's ray (origin p,
+// place q in its cell, list [b, b + c) of the sun grid) has its candidates checked ray
+// after ray and in list order within a ray, kShadowU per lane and round.  A candidate
+// whose bounds in the cell (sun_bounds) miss the ray is done: its 8-byte entry was read
+// next to its neighbours' by the wave, and its 48-byte triangle, three L1 accesses of one
+// lane, is not.  The others queue up in LDS and take the watertight any-hit test (r: the
+// rays' direction) 64 at a time.  The probe shadow kernel of terrain1m, which ran the L1 at
+// 99% of one access per clock, went from 114 to 79 M accesses and the update from 1.143 to
+// 1.113 ms; the 1080p shadow mask from 53.1 to 50.9 us, its mirror pass 423 to 416 us.
+// key[l] (this wave's 64 LDS slots, set to 2 c + 1 by the caller) ends as the earliest
+// event of lane l's list in list order: 2 pos for a hit, 2 pos + 1 for an entry out of
+// range when STOP_ON_BAD (which also raises *overflow; otherwise such entries are
+// skipped).  Tests after a known event are skipped.  All lanes of the wave must call it
+// (shuffles).
 template <bool STOP_ON_BAD>
 __device__ __forceinline__ void grid_wave_events(const SunGridK& sg, const float4* tris, int32_t ntri, RayPre r,
-                                                 f3 p, uint32_t b, uint32_t c, float tmin, float tmax,
-                                                 uint32_t* key, uint32_t* overflow)
+                                                 f3 p, uint32_t q, uint32_t b, uint32_t c, float tmin, float tmax,
+                                                 uint32_t* key, SunQueue& queue, uint32_t* overflow)
 {
   const int lane = threadIdx.x & 63;
   uint32_t incl = c;
@@ -983,10 +1008,26 @@ __device__ __forceinline__ void grid_wave_events(const SunGridK& sg, const float
   const uint32_t total = __shfl(incl, 63, 64);
   const uint32_t excl = incl - c;
   constexpr int U = kShadowU;
+  uint32_t waiting = 0u;  // wave-uniform: queue entries
+  // the last (at most 64) entries of the queue
+  auto drain = [&]() {
+    const uint32_t m = waiting < 64u ? waiting : 64u;
+    waiting -= m;
+    const uint32_t k = waiting + ((uint32_t)lane < m ? (uint32_t)lane : 0u);
+    const int j = queue.ray[k];
+    const uint32_t id = queue.id[k], pos = queue.pos[k];
+    r.o = mk(__shfl(p.x, j, 64), __shfl(p.y, j, 64), __shfl(p.z, j, 64));
+    if ((uint32_t)lane < m && 2u * pos < key[j]) {
+      const float4 v0 = tris[3 * (int64_t)id], v1 = tris[3 * (int64_t)id + 1], v2 = tris[3 * (int64_t)id + 2];
+      float tt, uu, vv;
+      if (tri_test(r, mk(v0.x, v0.y, v0.z), mk(v1.x, v1.y, v1.z), mk(v2.x, v2.y, v2.z), tmin, tmax, tt, uu, vv))
+        atomicMin(&key[j], 2u * pos);
+    }
+  };
   for (uint32_t t0 = 0; t0 < total; t0 += 64u * U) {
-    uint32_t pos[U], e[U];
+    uint32_t pos[U], qj[U];
+    uint2 e[U];
     int jj[U];
-    f3 o[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t t = t0 + 64u * u + (uint32_t)lane;
@@ -999,37 +1040,37 @@ __device__ __forceinline__ void grid_wave_events(const SunGridK& sg, const float
         if (v <= tc) j += step;
       }
       const uint32_t ej = __shfl(excl, j, 64), bj = __shfl(b, j, 64);
-      o[u] = mk(__shfl(p.x, j, 64), __shfl(p.y, j, 64), __shfl(p.z, j, 64));
+      qj[u] = __shfl(q, j, 64);
       jj[u] = t < total ? j : -1;
       pos[u] = tc - ej;
       e[u] = sg.list[bj + pos[u]];
     }
-    float4 v0[U], v1[U], v2[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t q = e[u] < (uint32_t)ntri ? (int64_t)e[u] : 0;
-      v0[u] = tris[3 * q];
-      v1[u] = tris[3 * q + 1];
-      v2[u] = tris[3 * q + 2];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (jj[u] >= 0 && 2u * pos[u] < key[jj[u]]) {
-        if (e[u] >= (uint32_t)ntri) {
-          if (STOP_ON_BAD) {
-            *overflow = 1u;
-            atomicMin(&key[jj[u]], 2u * pos[u] + 1u);
-          }
-        } else {
-          float tt, uu, vv;
-          r.o = o[u];
-          if (tri_test(r, mk(v0[u].x, v0[u].y, v0[u].z), mk(v1[u].x, v1[u].y, v1[u].z),
-                       mk(v2[u].x, v2[u].y, v2[u].z), tmin, tmax, tt, uu, vv))
-            atomicMin(&key[jj[u]], 2u * pos[u]);
+      const uint32_t qx = qj[u] & 0xFFu, qy = qj[u] >> 8, w = e[u].y;
+      bool in = jj[u] >= 0 && qx >= (w & 0xFFu) && qx <= ((w >> 8) & 0xFFu) && qy >= ((w >> 16) & 0xFFu) && qy <= (w >> 24);
+      if (jj[u] >= 0 && e[u].x >= (uint32_t)ntri) {
+        if (STOP_ON_BAD) {
+          *overflow = 1u;
+          atomicMin(&key[jj[u]], 2u * pos[u] + 1u);
         }
+        in = false;
       }
+      if (in) in = 2u * pos[u] < key[jj[u]];
+      const uint64_t im = __ballot(in);
+      if (in) {
+        const uint32_t k = waiting + __builtin_amdgcn_mbcnt_hi((uint32_t)(im >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)im, 0u));
+        queue.id[k] = e[u].x;
+        queue.pos[k] = pos[u];
+        queue.ray[k] = (uint8_t)jj[u];
+      }
+      waiting += (uint32_t)__popcll(im);
     }
+    // at most 63 stay, so that the next round's fit
+    while (waiting >= 64u) drain();
   }
+  if (waiting) drain();
 }
 
 #ifndef ANE_SHADOW_TB
@@ -1041,6 +1082,7 @@ template <bool COUNT>
 __device__ __forceinline__ void probe_shadow_group(const TraceArgs& a, int64_t first)
 {
   __shared__ uint32_t key[kShadowTB];
+  __shared__ SunQueue queue[kShadowTB / 64];
   const SunGridParams* gq = a.sg.params;
   const int tid = threadIdx.x, lane = tid & 63, wb = tid & ~63;
   const int64_t i = first + tid;
@@ -1052,21 +1094,17 @@ __device__ __forceinline__ void probe_shadow_group(const TraceArgs& a, int64_t f
   if (in) h = a.hits[i];
   const bool has = in && h.tri >= 0;
   f3 p = mk(0.0f, 0.0f, 0.0f);
-  uint32_t b = 0u, c = 0u;
+  uint32_t b = 0u, c = 0u, q = 0u;
   if (has) {
     HitGeom hg;
     p = hit_geom_pos(sc, h.tri, h.u, h.v, hg);
-    const float X = comp(p, gq->kx) - gq->sx * comp(p, gq->kz);
-    const float Y = comp(p, gq->ky) - gq->sy * comp(p, gq->kz);
-    const int64_t cell =
-        (int64_t)sun_cell(Y, gq->y0, gq->ich, gq->gy) * gq->gx + sun_cell(X, gq->x0, gq->icw, gq->gx);
-    b = a.sg.start[cell];
-    c = a.sg.start[cell + 1] - b;
+    sun_lookup(a.sg, *gq, p, b, c, q);
   }
   key[tid] = 2u * c + 1u;
   RayPre r;
   load_dirpre(r, a.dirpre + 3 * a.g.rays, p);  // the sun direction's ray setup
-  grid_wave_events<true>(a.sg, sc.tris, sc.ntri, r, p, b, c, a.g.t_min, a.g.t_max, key + wb, a.overflow);
+  grid_wave_events<true>(a.sg, sc.tris, sc.ntri, r, p, q, b, c, a.g.t_min, a.g.t_max, key + wb, queue[tid >> 6],
+                         a.overflow);
   const uint32_t k = key[tid];
   if (in) a.shadow[i] = has ? (uint8_t)((k & 1u) ? 0 : 1) : (uint8_t)255;
   if (COUNT) {
@@ -1909,6 +1947,7 @@ __global__ __launch_bounds__(256) void k_shadow_mask_grid(const float* depth, in
                                                           SunGridK sg, SceneK sc, float* vis)
 {
   __shared__ uint32_t key[256];
+  __shared__ SunQueue queue[4];
   const SunGridParams g = *sg.params;
   if (!g.valid) return;
   const int tid = threadIdx.x;
@@ -1919,19 +1958,16 @@ __global__ __launch_bounds__(256) void k_shadow_mask_grid(const float* depth, in
   const float d = in ? depth[i] : 1.0f;
   const bool ray = in && d != 1.0f && dir_ok;
   f3 p = mk(0.0f, 0.0f, 0.0f);
-  uint32_t b = 0u, c = 0u;
+  uint32_t b = 0u, c = 0u, q = 0u;
   if (ray) {
     p = pixel_world_pos(i, W, H, d, ivp);
-    const float X = comp(p, g.kx) - g.sx * comp(p, g.kz);
-    const float Y = comp(p, g.ky) - g.sy * comp(p, g.kz);
-    const int64_t cell = (int64_t)sun_cell(Y, g.y0, g.ich, g.gy) * g.gx + sun_cell(X, g.x0, g.icw, g.gx);
-    b = sg.start[cell];
-    c = sg.start[cell + 1] - b;
+    sun_lookup(sg, g, p, b, c, q);
   }
   key[tid] = 2u * c + 1u;
   RayPre r;
   ray_setup(r, p, dir_ok ? dir : mk(0.0f, 0.0f, 1.0f));
-  grid_wave_events<false>(sg, sc.tris, sc.ntri, r, p, b, c, 0.1f, 50.0f, key + (tid & ~63), nullptr);
+  grid_wave_events<false>(sg, sc.tris, sc.ntri, r, p, q, b, c, 0.1f, 50.0f, key + (tid & ~63), queue[tid >> 6],
+                          nullptr);
   if (in) vis[i] = (ray && !(key[tid] & 1u)) ? 0.0f : 1.0f;  // shadow.rgen:66-67
 }
 
@@ -2011,6 +2047,7 @@ __global__ __launch_bounds__(256) void k_mirror_shadow_grid(SceneK sc, const ane
                                                             SunGridK sg, float tmin, float tmax, ane_hit* shadow_hits)
 {
   __shared__ uint32_t key[256];
+  __shared__ SunQueue queue[4];
   const SunGridParams g = *sg.params;
   if (!g.valid) return;
   const int tid = threadIdx.x;
@@ -2020,20 +2057,16 @@ __global__ __launch_bounds__(256) void k_mirror_shadow_grid(SceneK sc, const ane
   h.u = h.v = 0.0f;
   if (i < n) h = hits[i];
   f3 p = mk(0.0f, 0.0f, 0.0f);
-  uint32_t b = 0u, c = 0u;
+  uint32_t b = 0u, c = 0u, q = 0u;
   if (h.tri >= 0) {
     HitGeom hg;
     p = hit_geom_pos(sc, h.tri, h.u, h.v, hg);
-    const float X = comp(p, g.kx) - g.sx * comp(p, g.kz);
-    const float Y = comp(p, g.ky) - g.sy * comp(p, g.kz);
-    const int64_t cell = (int64_t)sun_cell(Y, g.y0, g.ich, g.gy) * g.gx + sun_cell(X, g.x0, g.icw, g.gx);
-    b = sg.start[cell];
-    c = sg.start[cell + 1] - b;
+    sun_lookup(sg, g, p, b, c, q);
   }
   key[tid] = 2u * c + 1u;
   RayPre r;
   ray_setup(r, p, sun);
-  grid_wave_events<false>(sg, sc.tris, sc.ntri, r, p, b, c, tmin, tmax, key + (tid & ~63), nullptr);
+  grid_wave_events<false>(sg, sc.tris, sc.ntri, r, p, q, b, c, tmin, tmax, key + (tid & ~63), queue[tid >> 6], nullptr);
   if (h.tri >= 0) shadow_hits[i].tri = (key[tid] & 1u) ? -1 : 0;
 }
 
