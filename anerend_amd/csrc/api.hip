@@ -711,7 +711,7 @@ extern "C" int ane_scene_create(const float* vertices, int64_t num_vertices, con
   ANE_A(d_ids, n);
   ANE_A(d_ids2, n);
   ANE_A(d_nodes, n > 1 ? n - 1 : 1);
-  ANE_A(d_hnodes, 2 * (n > 1 ? n - 1 : 1));
+  ANE_A(d_hnodes, 4 * (n > 1 ? n - 1 : 1));
   ANE_A(d_hframe, 1);
   ANE_A(d_leaf_parent, n);
   ANE_A(d_tris, n * 3);

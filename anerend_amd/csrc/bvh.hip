@@ -648,7 +648,7 @@ __global__ void k_grid_frame(const NodeBuild* nodes, GridFrame* f)
 
 // Grid nodes from the fitted 64-byte records, one thread per node.  Cell indices are
 // floor / ceil in binary64 (their 1e-16 is far inside the traversal's slab margin).  Every
-// kGridSample-th block adds the area growth of its child boxes to the frame's sums.
+// kGridSample-th block adds the area growth of its entries' boxes to the frame's sums.
 static constexpr int kGridSample = 32;
 __device__ __forceinline__ void grid_box(const GridFrame& f, const float* lo, const float* hi, uint32_t* w, float& grow,
                                          uint32_t& n)
@@ -670,6 +670,26 @@ __device__ __forceinline__ void grid_box(const GridFrame& f, const float* lo, co
   }
 }
 
+__device__ __forceinline__ uint32_t grid_index(int c) { return (uint32_t)(c < 0 ? ~c : c); }
+
+// the two entries of child c (its box lo, hi) of a grid node
+__device__ __forceinline__ void grid_child(const NodeBuild* nodes, const GridFrame& f, int c, const float* lo,
+                                           const float* hi, uint32_t* w, uint32_t& ref, float& grow, uint32_t& n)
+{
+  if (c >= 0) {
+    const NodeBuild nd = nodes[c];
+    const float l0[3] = {nd.a.x, nd.a.z, nd.c.x}, h0[3] = {nd.a.y, nd.a.w, nd.c.y};
+    const float l1[3] = {nd.b.x, nd.b.z, nd.c.z}, h1[3] = {nd.b.y, nd.b.w, nd.c.w};
+    grid_box(f, l0, h0, w, grow, n);
+    grid_box(f, l1, h1, w + 3, grow, n);
+    ref = grid_index(nd.d.x) | (nd.d.x < 0 ? kGridLeaf0 : 0u) | (nd.d.y < 0 ? kGridLeaf1 : 0u);
+  } else {
+    grid_box(f, lo, hi, w, grow, n);
+    w[3] = w[4] = w[5] = 0x0000FFFFu;
+    ref = grid_index(c) | kGridLeaf0 | kGridLeaf1;
+  }
+}
+
 __global__ __launch_bounds__(256) void k_grid_nodes(const NodeBuild* nodes, int n, GridFrame* frame, uint4* q)
 {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -680,11 +700,14 @@ __global__ __launch_bounds__(256) void k_grid_nodes(const NodeBuild* nodes, int 
     const NodeBuild nd = nodes[i];
     const float l0[3] = {nd.a.x, nd.a.z, nd.c.x}, h0[3] = {nd.a.y, nd.a.w, nd.c.y};
     const float l1[3] = {nd.b.x, nd.b.z, nd.c.z}, h1[3] = {nd.b.y, nd.b.w, nd.c.w};
-    uint32_t w[6];
-    grid_box(f, l0, h0, w, grow, cnt);
-    grid_box(f, l1, h1, w + 3, grow, cnt);
-    q[2 * (int64_t)i] = make_uint4(w[0], w[1], w[2], w[3]);
-    q[2 * (int64_t)i + 1] = make_uint4(w[4], w[5], (uint32_t)nd.d.x, (uint32_t)nd.d.y);
+    uint32_t w[12], rl, rr;
+    grid_child(nodes, f, nd.d.x, l0, h0, w, rl, grow, cnt);
+    grid_child(nodes, f, nd.d.y, l1, h1, w + 6, rr, grow, cnt);
+    uint4* o = q + 4 * (int64_t)i;
+    o[0] = make_uint4(w[0], w[1], w[2], w[3]);
+    o[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    o[2] = make_uint4(w[8], w[9], w[10], w[11]);
+    o[3] = make_uint4(rl, rr, grid_index(nd.d.x), 0u);
   }
   if (blockIdx.x % kGridSample != 0) return;
 #pragma unroll

@@ -106,7 +106,7 @@ struct SceneK {
   const uint32_t* inst_tri_off; // [ninst + 1]
   const float4* nodes;          // [ntri - 1][4] traversal nodes
   const uint4* qnodes;          // [ntri - 1][2] quantized traversal nodes, or null (use nodes)
-  const uint4* hnodes;          // [ntri - 1][2] grid nodes of the closest-hit traversal
+  const uint4* hnodes;          // [ntri - 1][4] grid nodes of the closest-hit traversal, null: not used
   const struct GridFrame* hframe; // their frame
   const float4* tris;           // [ntri][3] sorted world triangles (v0.w = id bits)
   int32_t ntri;
@@ -136,11 +136,17 @@ struct NodeBuild {
 ANE_HD float qnode_step(uint32_t ebyte) { return __builtin_bit_cast(float, (ebyte - 128u + 127u) << 23); }
 ANE_HD float qnode_bound(float o, uint32_t q, float step) { return o + (float)q * step; }
 
-// Grid node, 32 bytes (2 x uint4), for the closest-hit traversal: the bounds of both
-// children on a 2^16 grid over the scene's bounds, rounded outward:
-//   w0..w2 child 0 x, y, z: lower | upper << 16;  w3..w5 child 1;  w6 left, w7 right
-// (children as in NodeBuild).  A bound is o + q * s in the frame.  A node costs two
-// 16-byte loads per ray instead of four.
+// Grid node, 64 bytes (4 x uint4), for the closest-hit traversal: node i's grandchildren, two
+// levels of the hierarchy for one round trip.  Their bounds lie on a 2^16 grid over the
+// scene's bounds, rounded outward:
+//   words 0..11: entry e = 0..3 at 3 e, x, y, z: lower | upper << 16.  Entries 0, 1 are the
+//   left child's children, 2, 3 the right child's; a leaf child is its own first entry, and
+//   the second is empty (lower 65535, upper 0 on every axis).
+//   words 12, 13: the entries of a child as first index | kGridLeaf0 / kGridLeaf1: a node
+//   split at g has its children, nodes or leaves, at g and g + 1.  word 14: node i's own g,
+//   the index of its left child.
+// A bound is o + q * s in the frame.
+static constexpr uint32_t kGridLeaf0 = 1u << 31, kGridLeaf1 = 1u << 30, kGridIndex = (1u << 30) - 1u;
 struct GridFrame {
   float o[3], s[3];   // lower corner and cell size (rounded up)
   float r;            // largest coordinate magnitude of the bounds

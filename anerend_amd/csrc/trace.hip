@@ -16,7 +16,7 @@
 //                    (large scenes), else the 64-byte nodes; caller rays may carry a
 //                    per-ray t_max
 //   k_trace_closest  the traversal of the closest-hit rays that need no work counts:
-//                    the same hits from 32-byte grid nodes
+//                    the same hits from 64-byte grid nodes, two levels each
 //   k_probe_shadow_grid  with a sun grid: the shadow rays of the probe hits against
 //                    the triangles of their cells, the candidates of a wave's 64 rays
 //                    spread over its lanes
@@ -102,21 +102,13 @@ static constexpr int kRefill = ANE_TRACE_REFILL;
 static constexpr int kLeafBatchProbe = ANE_TRACE_LEAFBATCH;
 static constexpr int kLeafBatchRays = ANE_TRACE_LEAFBATCH_RAYS;
 static constexpr int kShadeUnroll = ANE_SHADE_UNROLL;
-// closest-hit traversal of grid nodes, terrain1m / 4.04M-triangle update: 6 waves per SIMD
-// 1.179 / 12.98 ms against 1.143 / 13.02; leaf batches of 12 / 16 lanes 1.137 / 1.140 against
-// 1.143, but 701 / 716 us against 671 for the 65k rays over 246k triangles; 5 / 8 steps per
-// refill check 1.143 / 1.149 and 204 / 198 us against 198 for one probe layer
+// closest-hit traversal of grid nodes: 6 waves per SIMD 1.111 ms against 1.089 for the
+// terrain1m update; leaf batches of 8 / 16 lanes 1.077 / 1.068 against 1.067
 #ifndef ANE_CLOSEST_WAVES
 #define ANE_CLOSEST_WAVES 7
 #endif
 #ifndef ANE_CLOSEST_LEAFBATCH
-#define ANE_CLOSEST_LEAFBATCH 8
-#endif
-#ifndef ANE_CLOSEST_LEAFBATCH_RAYS
-#define ANE_CLOSEST_LEAFBATCH_RAYS 1  // caller rays (4 / 8: 115 / 127 us against 109 for 64 lights)
-#endif
-#ifndef ANE_CLOSEST_STEPS
-#define ANE_CLOSEST_STEPS 7
+#define ANE_CLOSEST_LEAFBATCH 12
 #endif
 
 bool trace_grid_supported() { return true; }
@@ -627,7 +619,13 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
 //   culled.  k_trace is bound by VALU issue and, right behind it, by the L1: a CU serves
 //   one access of a lane per clock, and a 64-byte node is four of them (terrain1m launch:
 //   452 M accesses in 489 M clocks of the CUs).  So:
-//   - Grid nodes (GridFrame): two accesses per node, 249 M for the launch.
+//   - Grid nodes: a round trip takes a ray two levels down.  The far child of a step is
+//     pushed as one reference when both its entries are hit, so the stack needs no more
+//     than the two-way traversal's, and its record is tested against the hits found since.
+//     One level a step, in 32 bytes: 12.98 ms against 10.4 for the dynamic frame of the
+//     4.04M-triangle scene, whose nodes miss the L2; 102 us against 87 for 64 lights, 108
+//     against 101 for the update of a room, 404 against 382 for the 1080p mirror pass, 1.115
+//     against 1.067 ms for the terrain1m update.
 //   - A slab is one conversion and one fma: t = q * (s * inv) + c with c = (o - origin -+
 //     margin) * inv per ray; the bound pairs are rotated by the ray's signs so that near
 //     and far planes need no minimum and maximum.  The margin (kSlabMargin) makes the boxes
@@ -636,9 +634,15 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
 //     that one compare (node < lim) tells who goes on; the stack pointer is the LDS address
 //     of its ring, whose bottom entry ends the traversal; barycentrics and reciprocals lie
 //     in LDS, so that 7 waves per SIMD need no spills.
-//   terrain1m update 1.325 -> 1.143 ms, one of its layers 249 -> 198 us, 64 lights 129 ->
-//   102 us, 1080p mirror pass 474 -> 423 us; 385 M VALU instructions in 0.6 ms, which is
-//   VALU issue again.
+//   - While chunks are left to claim, a wave is kept full: leaves are tested 12 lanes at a
+//     time, and the steps end once kRefill lanes have nothing to do.  A wave that knows of
+//     no more chunks (all of a small launch, the end of a large one) waits on its longest
+//     ray, so a leaf is tested at once and 7 steps run between the checks: 1.067 ms for the
+//     terrain1m update and 101 / 178 us for a room's update and a terrain1m layer; batches
+//     and 7 steps throughout 1.162 ms and 108 / 193 us, 3 steps 1.108 and 112 / 201.
+//   k_trace took 1.325 ms for that update, 249 us for the layer, 129 for the lights, 474 for
+//   the mirror pass.  What bounds it is VALU issue for large launches, the chain of node
+//   reads for small ones and the L2's misses for scenes beyond it.
 //   Rays whose products could leave the normal range (a direction component below 1e-29,
 //   huge coordinates) make their wave take the full (or quantized) nodes with the exact slab
 //   test of k_trace, which also keeps its decisions on rays that lie in a box face.  Scenes
@@ -646,7 +650,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
 //   (their hit id is the first found) and launches with a step limit keep k_trace; a refit
 //   that outgrows the grid takes the exact slabs (1.37 ms).
 // ---------------------------------------------------------------------------
-static constexpr int64_t kFastMaxTris = (int64_t)1 << 25;  // 32-bit byte offsets of 64-byte nodes and 48-byte triangles
+static constexpr int64_t kFastMaxTris = (int64_t)1 << 25;  // 32-bit byte offsets of nodes and triangles
 
 __device__ __forceinline__ float uniform_f(float x)
 {
@@ -681,14 +685,19 @@ __device__ __forceinline__ float min_number(float x, float y)
   return r;
 }
 
+// node reference of entry e (0, 1) of a grid node's child word
+__device__ __forceinline__ int32_t grid_ref(uint32_t w, uint32_t e)
+{
+  return (int32_t)((w & kGridIndex) + e) ^ ((int32_t)(w << e) >> 31);
+}
+
 template <bool RAYS>
 __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST_WAVES))) void k_trace_closest(TraceArgs a)
 {
   constexpr int32_t kDone = 0x7FFFFFFF;  // the lane's traversal has ended (>= lim, not a leaf)
   constexpr uint32_t kSlot = kTB * 4;    // bytes of one stack level of the block
   constexpr uint32_t kRing = kSS * kSlot;
-  constexpr int kLeafBatch = RAYS ? ANE_CLOSEST_LEAFBATCH_RAYS : ANE_CLOSEST_LEAFBATCH;
-  constexpr int kSteps = ANE_CLOSEST_STEPS;  // traversal steps per refill check
+  constexpr float kMiss = 3.0e38f;  // beyond every entry distance a ray can have
   const bool sgrid = !RAYS && a.sg.list != nullptr && a.sg.params->valid != 0u;
   __shared__ int32_t stk[kSS * kTB];
   // per lane, what only refills, hits and exact slabs touch (registers set the occupancy):
@@ -720,6 +729,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
     fr.s[k] = uniform_f(fr.s[k]);
   }
   fr.r = uniform_f(fr.r);
+  const float ext = 65535.0f * fmaxf(fr.s[0], fmaxf(fr.s[1], fr.s[2]));
 
   int32_t out = -1;  // output slot of the lane's ray, -1: idle
   bool exhausted = false;
@@ -728,6 +738,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
   const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kTB / 64) + (tid >> 6))) * kChunk;
   uint32_t cbeg = first < nrays ? first : nrays;
   uint32_t cend = cbeg + kChunk < nrays ? cbeg + kChunk : nrays;
+  bool dry = nrays <= gridDim.x * (kTB / 64u) * kChunk;  // no chunk left to claim, as far as the wave knows
   f3 ro = mk(0.0f, 0.0f, 0.0f), sh = ro;  // origin, watertight shear
   int32_t kk = 0;                         // its axes kx | ky << 2 | kz << 4
   f3 ci = ro, cn = ro, cf = ro;  // slab constants: per cell, of the near and of the far planes
@@ -754,7 +765,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
     const float om = fmaxf(fabsf(ro.x), fmaxf(fabsf(ro.y), fabsf(ro.z)));
     const float im = fmaxf(fabsf(r.inv.x), fmaxf(fabsf(r.inv.y), fabsf(r.inv.z)));
     const float m = kSlabMargin * fmaxf(fr.r, om);
-    exact = !(im * fmaxf(fr.r + om + m, 1e8f) < 1e37f);
+    exact = !(im * fmaxf(fr.r + om + m, 1e8f) < 1e37f && 4.0f * m < ext);  // ext: empty entries miss
     ci = mk(fr.s[0] * r.inv.x, fr.s[1] * r.inv.y, fr.s[2] * r.inv.z);
     const f3 d = mk(fr.o[0] - ro.x, fr.o[1] - ro.y, fr.o[2] - ro.z);
     // the near planes are the lower ones along a positive direction, each moved outward
@@ -775,16 +786,29 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
     node = entry(sp);
     if (sp >= kRing) entry(sp) = spilled(sp);
   };
-  // one box: near and far distances from its three rotated bound pairs
-  auto box = [&](uint32_t wx, uint32_t wy, uint32_t wz, float& tn) -> bool {
+  // the far entries (LDS ring; the oldest one spills when it is full)
+  auto push = [&](int32_t ref) {
+    if (sp >= kRing) {
+      if ((int)(sp / kSlot) - kSS >= a.spill_depth) {
+        *a.overflow = 1u;
+        node = kDone;
+        return;
+      }
+      spilled(sp) = entry(sp);
+    }
+    entry(sp) = ref;
+    sp += kSlot;
+  };
+  // where the ray enters one box, from its three rotated bound pairs; kMiss if it does not
+  auto box = [&](uint32_t wx, uint32_t wy, uint32_t wz) -> float {
     wx = __builtin_amdgcn_alignbit(wx, wx, rx);
     wy = __builtin_amdgcn_alignbit(wy, wy, ry);
     wz = __builtin_amdgcn_alignbit(wz, wz, rz);
-    tn = fmaxf(fmaxf(fmaf((float)(wx & 0xFFFFu), ci.x, cn.x), fmaf((float)(wy & 0xFFFFu), ci.y, cn.y)),
-               fmaxf(fmaf((float)(wz & 0xFFFFu), ci.z, cn.z), tmin));
+    const float tn = fmaxf(fmaxf(fmaf((float)(wx & 0xFFFFu), ci.x, cn.x), fmaf((float)(wy & 0xFFFFu), ci.y, cn.y)),
+                           fmaxf(fmaf((float)(wz & 0xFFFFu), ci.z, cn.z), tmin));
     const float tf = fminf(fminf(fmaf((float)(wx >> 16), ci.x, cf.x), fmaf((float)(wy >> 16), ci.y, cf.y)),
                            min_number(fmaf((float)(wz >> 16), ci.z, cf.z), tbest));
-    return tn <= tf;
+    return tn <= tf ? tn : kMiss;
   };
 
   for (;;) {
@@ -829,6 +853,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
     if (need != 0u && (am == 0ull || need >= (uint32_t)kRefill)) {
       if (cbeg >= cend) cbeg = claim_chunk(a, nrays, im, lane, cend);
       const uint32_t avail = cend > cbeg ? cend - cbeg : 0u;
+      dry = dry || avail == 0u;
       const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(im >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)im, 0u));
       if (idle) {
         if (avail == 0u) {
@@ -865,48 +890,47 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
       continue;
     }
     const bool slow = !grid || __ballot(exact && out >= 0) != 0ull;  // wave-uniform
+    const int leaf_batch = RAYS || dry ? 1 : ANE_CLOSEST_LEAFBATCH;
     // ---- traversal steps ----
-#pragma unroll
-    for (int u = 0; u < kSteps; ++u) {
+    // (a chain of calls, for a loop with the early way out is not unrolled: 1.089 ms)
+    auto step = [&](bool goes_on) __attribute__((always_inline)) -> bool {
       if ((uint32_t)node < lim) {
-        int32_t L, Rc;
-        float tn0, tn1;
-        bool b0, b1;
         if (!slow) {
-          const uint4* nq = reinterpret_cast<const uint4*>(nbase + (uint32_t)node * 32u);
-          const uint4 q0 = nq[0], q1 = nq[1];
-          L = (int32_t)q1.z;
-          Rc = (int32_t)q1.w;
-          b0 = box(q0.x, q0.y, q0.z, tn0);
-          b1 = box(q0.w, q1.x, q1.y, tn1);
+          const uint4* nq = reinterpret_cast<const uint4*>(nbase + (uint32_t)node * 64u);
+          const uint4 q0 = nq[0], q1 = nq[1], q2 = nq[2], q3 = nq[3];
+          const float t0 = box(q0.x, q0.y, q0.z), t1 = box(q0.w, q1.x, q1.y);
+          const float t2 = box(q1.z, q1.w, q2.x), t3 = box(q2.y, q2.z, q2.w);
+          const float m0 = min_number(t0, t1), m1 = min_number(t2, t3);
+          // on to the nearest entry; its sibling and, below it, the far child are pushed:
+          // the far child as one reference when both its entries are hit
+          const bool sw = m1 < m0;
+          const float n0 = sw ? t2 : t0, n1 = sw ? t3 : t1, f0 = sw ? t0 : t2, f1 = sw ? t1 : t3;
+          const uint32_t nw = sw ? q3.y : q3.x, fw = sw ? q3.x : q3.y;
+          const uint32_t e = n1 < n0 ? 1u : 0u;
+          node = grid_ref(nw, e);
+          if (min_number(f0, f1) < kMiss) {
+            const bool h0 = f0 < kMiss, h1 = f1 < kMiss;
+            push(h0 && h1 ? (int32_t)(q3.z + (sw ? 0u : 1u)) : grid_ref(fw, h0 ? 0u : 1u));
+          }
+          if (fmaxf(n0, n1) < kMiss) push(grid_ref(nw, e ^ 1u));
+          if (!(min_number(m0, m1) < kMiss)) pop();
         } else {
+          int32_t L, Rc;
+          float tn0, tn1;
+          bool b0, b1;
           RayPre r;
           r.o = ro;
           r.inv = mk(cold[2][tid], cold[3][tid], cold[4][tid]);
           exact_boxes(sc, node, r, tmin, tbest, L, Rc, b0, b1, tn0, tn1);
+          const bool left = b0 && !(b1 && tn1 < tn0);
+          node = left ? L : Rc;
+          if (b0 && b1) push(left ? Rc : L);
+          if (!(b0 || b1)) pop();
         }
-        const bool left = b0 && !(b1 && tn1 < tn0);
-        node = left ? L : Rc;
-        if (b0 && b1) {
-          // push the far child (LDS ring; the oldest entry spills when full)
-          bool room = true;
-          if (sp >= kRing) {
-            room = (int)(sp / kSlot) - kSS < a.spill_depth;
-            if (room) spilled(sp) = entry(sp);
-          }
-          if (room) {
-            entry(sp) = left ? Rc : L;
-            sp += kSlot;
-          } else {
-            *a.overflow = 1u;
-            node = kDone;
-          }
-        }
-        if (!(b0 || b1)) pop();
       }
       const uint64_t lm = __ballot(node < 0);
       if (lm != 0ull) {
-        if (__popcll(lm) >= kLeafBatch || __ballot((uint32_t)node < lim) == 0ull) {
+        if (__popcll(lm) >= leaf_batch || __ballot((uint32_t)node < lim) == 0ull) {
           if (node < 0 && (uint32_t)~node < (uint32_t)sc.ntri) {
             const float4* tv = reinterpret_cast<const float4*>(tbase + (uint32_t)~node * 48u);
             const float4 v0 = tv[0], v1 = tv[1], v2 = tv[2];
@@ -935,7 +959,11 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
           }
         }
       }
-    }
+      // true: enough lanes have ended for a refill, and there is something to refill them with
+      return !goes_on && !dry && __popcll(__ballot(node == kDone)) >= kRefill;
+    };
+    (void)(step(true) || step(false) || step(false) || step(false) || step(false) ||
+           step(false) || step(true));
   }
 }
 
