@@ -634,11 +634,13 @@ __global__ void k_grid_frame(const NodeBuild* nodes, GridFrame* f)
   g.r = 0.0f;
   bool finite = true;
   for (int k = 0; k < 3; ++k) {
-    g.o[k] = lo[k];
-    // 65535 cells span the extent: the cell is rounded up twice
-    g.s[k] = fmaxf((hi[k] - lo[k]) / 65535.0f * 1.000001f, 1e-30f);
     g.r = fmaxf(g.r, fmaxf(fabsf(lo[k]), fabsf(hi[k])));
     finite = finite && __builtin_isfinite(lo[k]) && __builtin_isfinite(hi[k]);
+  }
+  for (int k = 0; k < 3; ++k) {
+    // the codes' values span 1.49997: the scale is rounded up, past the rounding of o too
+    g.s[k] = fmaxf((hi[k] - lo[k]) / 1.4999f + 2e-7f * g.r, 1e-30f);
+    g.o[k] = lo[k] - 0.5f * g.s[k];
   }
   if (!finite) g.r = __builtin_inff();
   g.sum = 0.0f;
@@ -646,22 +648,29 @@ __global__ void k_grid_frame(const NodeBuild* nodes, GridFrame* f)
   *f = g;
 }
 
-// Grid nodes from the fitted 64-byte records, one thread per node.  Cell indices are
-// floor / ceil in binary64 (their 1e-16 is far inside the traversal's slab margin).  Every
+// Grid nodes from the fitted 64-byte records, one thread per node.  Codes are floor / ceil in
+// binary64 (their 1e-16 is far inside the traversal's slab margin).  Every
 // kGridSample-th block adds the area growth of its entries' boxes to the frame's sums.
 static constexpr int kGridSample = 32;
+// the code of x, fractional: steps of 2^-16 up to the value 1 and of 2^-15 above it
+__device__ __forceinline__ double grid_code(float x, float o, float s)
+{
+  const double v = ((double)x - (double)o) / (double)s;
+  const double c = v < 1.0 ? (v - 0.5) * 65536.0 : 32768.0 + (v - 1.0) * 32768.0;
+  return fmin(fmax(c, 0.0), 65535.0);
+}
+
 __device__ __forceinline__ void grid_box(const GridFrame& f, const float* lo, const float* hi, uint32_t* w, float& grow,
                                          uint32_t& n)
 {
   float e[3], q[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const double a = floor(((double)lo[k] - (double)f.o[k]) / (double)f.s[k]);
-    const double b = ceil(((double)hi[k] - (double)f.o[k]) / (double)f.s[k]);
-    const uint32_t l = (uint32_t)fmin(fmax(a, 0.0), 65535.0), u = (uint32_t)fmin(fmax(b, 0.0), 65535.0);
+    const uint32_t l = (uint32_t)floor(grid_code(lo[k], f.o[k], f.s[k]));
+    const uint32_t u = (uint32_t)ceil(grid_code(hi[k], f.o[k], f.s[k]));
     w[k] = l | u << 16;
     e[k] = hi[k] - lo[k];
-    q[k] = (float)(u - l) * f.s[k] + 2.0f * kSlabMargin * f.r;  // as the traversal sees it
+    q[k] = (grid_value(u) - grid_value(l)) * f.s[k] + 2.0f * kSlabMargin * f.r;  // as the traversal sees it
   }
   const float area = e[0] * e[1] + e[1] * e[2] + e[2] * e[0];
   if (area > 0.0f) {

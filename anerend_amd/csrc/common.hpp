@@ -137,29 +137,31 @@ ANE_HD float qnode_step(uint32_t ebyte) { return __builtin_bit_cast(float, (ebyt
 ANE_HD float qnode_bound(float o, uint32_t q, float step) { return o + (float)q * step; }
 
 // Grid node, 64 bytes (4 x uint4), for the closest-hit traversal: node i's grandchildren, two
-// levels of the hierarchy for one round trip.  Their bounds lie on a 2^16 grid over the
-// scene's bounds, rounded outward:
+// levels of the hierarchy for one round trip.  Their bounds are 16-bit codes over the scene's
+// bounds, rounded outward; a code is the two middle bytes of the float 0x3F....00, which is
+// in [0.5, 2) and rises with the code, so that one byte permute unpacks it:
 //   words 0..11: entry e = 0..3 at 3 e, x, y, z: lower | upper << 16.  Entries 0, 1 are the
 //   left child's children, 2, 3 the right child's; a leaf child is its own first entry, and
 //   the second is empty (lower 65535, upper 0 on every axis).
 //   words 12, 13: the entries of a child as first index | kGridLeaf0 / kGridLeaf1: a node
 //   split at g has its children, nodes or leaves, at g and g + 1.  word 14: node i's own g,
 //   the index of its left child.
-// A bound is o + q * s in the frame.
+// A bound is o + grid_value(code) * s in the frame.
 static constexpr uint32_t kGridLeaf0 = 1u << 31, kGridLeaf1 = 1u << 30, kGridIndex = (1u << 30) - 1u;
 struct GridFrame {
-  float o[3], s[3];   // lower corner and cell size (rounded up)
+  float o[3], s[3];   // origin and scale: the bounds lie at 0.5 to 2 s from o
   float r;            // largest coordinate magnitude of the bounds
   float sum;          // sampled child boxes: the growth of their area by the rounding,
   uint32_t count;     // summed, and their number
 };
 // Outward margin of the grid traversal's slabs, of the largest coordinate magnitude of
-// scene and ray origin.  In units of 2^-24 of it, the rounding of the slab constants and
-// products adds up to 10 and that of the triangle test (translation, shear, edge functions,
-// t) to about 26; this is 67.
+// scene and ray origin.  In units of 2^-24 of it, the rounding of the frame, the slab
+// constants and the products adds up to 18 and that of the triangle test (translation,
+// shear, edge functions, t) to about 26; this is 67.
 static constexpr float kSlabMargin = 4e-6f;
 // The grid is used while it is finite and boxes grow by at most half on average; a scene
-// whose detail is far finer than 2^-16 of its extent keeps its full nodes.
+// whose detail is far finer than the codes' step (2^-15.6 to 2^-16.6 of its extent) keeps its full nodes.
+ANE_HD float grid_value(uint32_t code) { return __builtin_bit_cast(float, 0x3F000000u | code << 8); }
 ANE_HD bool grid_frame_ok(const GridFrame& f)
 {
   return f.r < 1e18f && f.sum <= 1.5f * (float)f.count;
