@@ -374,6 +374,13 @@ struct SunGridCache {
 // ===========================================================================
 // scene
 // ===========================================================================
+// What a build's kernels write for the host
+struct BuildInfo {
+  uint32_t plan[132];  // level offsets and counts of the fit plan
+  uint32_t depth;
+  GridFrame frame;
+};
+
 struct ane_scene {
   int device = 0;
   int64_t nvert = 0, nidx = 0;
@@ -405,7 +412,8 @@ struct ane_scene {
   GridFrame* d_hframe = nullptr;
   int32_t node_format = ANE_NODES_AUTO;
   uint32_t* d_scratch = nullptr;
-  uint32_t* d_info = nullptr;   // fit plan read back at a build: level offsets, counts, tree depth
+  uint32_t* d_depth = nullptr;  // tree depth of a build
+  BuildInfo* h_info = nullptr;  // what a build's kernels tell the host (coherent host memory)
   int4* d_topo = nullptr;       // children, parent and leaf-range end of every internal node
   int32_t* d_cross = nullptr;   // top nodes (more leaves than a fit treelet holds), by depth
   int2* d_cross_kids = nullptr; // their children, in the same order (cross_kids_cap entries)
@@ -473,7 +481,7 @@ static void scene_free(ane_scene* s)
   dfree(s->d_world); dfree(s->d_keys); dfree(s->d_keys2); dfree(s->d_ids); dfree(s->d_ids2);
   dfree(s->d_nodes); dfree(s->d_leaf_parent); dfree(s->d_tris);
   dfree(s->d_node_box); dfree(s->d_cbounds); dfree(s->d_cpart); dfree(s->d_qnodes); dfree(s->d_hnodes); dfree(s->d_hframe); dfree(s->d_scratch);
-  dfree(s->d_info); dfree(s->d_topo); dfree(s->d_cross); dfree(s->d_cross_kids); dfree(s->d_top); dfree(s->d_ndepth); dfree(s->d_units);
+  dfree(s->d_depth); dfree(s->d_topo); dfree(s->d_cross); dfree(s->d_cross_kids); dfree(s->d_top); dfree(s->d_ndepth); dfree(s->d_units);
   dfree(s->d_unit_root); dfree(s->d_uheight); dfree(s->d_stray); dfree(s->d_uscratch);
   dfree(s->d_sh_orig); dfree(s->d_sh_dir); dfree(s->d_sh_hits); dfree(s->d_sh_work);
   dfree(s->d_sh_spill);
@@ -481,6 +489,7 @@ static void scene_free(ane_scene* s)
   dfree(s->d_lt_dirs); dfree(s->d_lt_wt); dfree(s->d_lt_idx); dfree(s->d_lt_order); dfree(s->d_lt_work);
   dfree(s->d_lt_spill);
   s->sgc.destroy();
+  if (s->h_info) (void)hipHostFree(s->h_info);
   if (s->ev0) (void)hipEventDestroy(s->ev0);
   if (s->ev1) (void)hipEventDestroy(s->ev1);
   for (int k = 0; k < 2; ++k) {
@@ -511,14 +520,17 @@ static int validate_instances(const ane_scene* s, const ane_instance* inst, int3
   return ANE_OK;
 }
 
+// host memory that kernels read and write
+static constexpr unsigned kHostFlags = hipHostMallocMapped | hipHostMallocCoherent;
+
 static int upload_instances(ane_scene* s, const ane_instance* inst, hipStream_t st)
 {
   s->inst.assign(inst, inst + s->ninst);
   const size_t cap = (size_t)(s->ninst > 0 ? s->ninst : 1);
   const int k = s->up_slot;
   if (!s->h_inst[k]) {
-    ANE_CHECK_HIP(hipHostMalloc((void**)&s->h_inst[k], sizeof(ane_instance) * cap, hipHostMallocDefault));
-    ANE_CHECK_HIP(hipHostMalloc((void**)&s->h_inv[k], sizeof(float) * 12 * cap, hipHostMallocDefault));
+    ANE_CHECK_HIP(hipHostMalloc((void**)&s->h_inst[k], sizeof(ane_instance) * cap, kHostFlags));
+    ANE_CHECK_HIP(hipHostMalloc((void**)&s->h_inv[k], sizeof(float) * 12 * cap, kHostFlags));
     ANE_CHECK_HIP(hipEventCreateWithFlags(&s->ev_up[k], hipEventDisableTiming));
   }
   if (s->up_pending[k]) {
@@ -527,10 +539,9 @@ static int upload_instances(ane_scene* s, const ane_instance* inst, hipStream_t 
   }
   std::memcpy(s->h_inst[k], inst, sizeof(ane_instance) * s->ninst);
   for (int32_t i = 0; i < s->ninst; ++i) invert_3x4(inst[i].transform, s->h_inv[k] + 12 * i);
-  ANE_CHECK_HIP(hipMemcpyAsync(s->d_inst, s->h_inst[k], sizeof(ane_instance) * s->ninst,
-                               hipMemcpyHostToDevice, st));
-  ANE_CHECK_HIP(hipMemcpyAsync(s->d_inv, s->h_inv[k], sizeof(float) * 12 * s->ninst,
-                               hipMemcpyHostToDevice, st));
+  launch_upload(s->h_inst[k], s->d_inst, (int64_t)sizeof(ane_instance) * s->ninst, s->h_inv[k], s->d_inv,
+                (int64_t)sizeof(float) * 12 * s->ninst, st);
+  ANE_CHECK_HIP(hipGetLastError());
   ANE_CHECK_HIP(hipEventRecord(s->ev_up[k], st));
   s->up_pending[k] = true;
   s->up_slot = k ^ 1;
@@ -583,8 +594,8 @@ static int scene_build(ane_scene* s, hipStream_t st, bool write_inst)
   radix_sort_pairs(s->d_keys, s->d_ids, s->d_keys2, s->d_ids2, n, s->d_scratch, st);
   launch_karras(s->d_keys, n, s->d_nodes, s->d_leaf_parent, s->d_topo, st);
   launch_reorder(s->d_world, s->d_ids, n, s->d_tris, st);
-  if (launch_fit_plan(s->d_topo, s->d_leaf_parent, n, s->d_scratch, s->d_uscratch, s->d_info, s->d_ndepth,
-                      s->d_cross, s->d_top, s->d_units, s->d_unit_root, s->d_stray, &s->cross_begin, &s->nunits,
+  if (launch_fit_plan(s->d_topo, s->d_leaf_parent, n, s->d_scratch, s->d_uscratch, s->h_info->plan,
+                      s->d_depth, s->d_ndepth, s->d_cross, s->d_top, s->d_units, s->d_unit_root, s->d_stray, &s->cross_begin, &s->nunits,
                       &s->nstray, st) != 0)
     return fail(ANE_ERR_DEVICE, "LBVH fit plan failed");
   const int64_t ncross = s->cross_begin.empty() ? 0 : s->cross_begin.back();
@@ -602,20 +613,13 @@ static int scene_build(ane_scene* s, hipStream_t st, bool write_inst)
              s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, nullptr, nullptr, s->d_uheight, st);
   launch_grid_nodes(s->d_nodes, n, s->d_hframe, s->d_hnodes, st);
   ANE_TRY(scene_apply_node_format(s, st, qn != nullptr));
-  uint32_t* d_depth = s->d_info + 132;
-  if (launch_tree_depth(s->d_topo, n, s->d_unit_root, s->d_uheight, s->nunits, s->d_top, s->d_uscratch,
-                        s->d_ndepth, d_depth, st) != 0)
-    return fail(ANE_ERR_DEVICE, "LBVH depth failed");
+  launch_tree_depth(s->d_topo, n, s->d_unit_root, s->d_uheight, s->nunits, s->d_top, s->d_uscratch, s->d_ndepth,
+                    s->d_depth, s->d_hframe, &s->h_info->depth, &s->h_info->frame, st);
   ANE_CHECK_HIP(hipGetLastError());
   ANE_CHECK_HIP(hipEventRecord(s->ev1, st));
-  uint32_t depth = 0;
-  GridFrame frame{};
-  if (n >= 2) {
-    ANE_CHECK_HIP(hipMemcpyAsync(&depth, d_depth, 4, hipMemcpyDeviceToHost, st));
-    ANE_CHECK_HIP(hipMemcpyAsync(&frame, s->d_hframe, sizeof(frame), hipMemcpyDeviceToHost, st));
-  }
   ANE_CHECK_HIP(hipStreamSynchronize(st));
-  s->view.hnodes = grid_frame_ok(frame) ? s->d_hnodes : nullptr;
+  const uint32_t depth = n >= 2 ? s->h_info->depth : 0u;
+  s->view.hnodes = n < 2 || grid_frame_ok(s->h_info->frame) ? s->d_hnodes : nullptr;
   // the deepest internal nodes have two leaf children: leaf depth = number of internal levels
   s->depth = (int32_t)depth;
   ANE_CHECK_HIP(hipEventElapsedTime(&s->build_ms, s->ev0, s->ev1));
@@ -719,7 +723,7 @@ extern "C" int ane_scene_create(const float* vertices, int64_t num_vertices, con
   ANE_A(d_cbounds, 6);
   ANE_A(d_cpart, flatten_partial_words((int)n));
   ANE_A(d_scratch, radix_scratch_words(n > 0 ? n : 1));
-  ANE_A(d_info, 136);
+  ANE_A(d_depth, 1);
   ANE_A(d_topo, n > 1 ? n - 1 : 1);
   ANE_A(d_cross, n > 1 ? n - 1 : 1);
   ANE_A(d_top, n > 1 ? n - 1 : 1);
@@ -734,6 +738,8 @@ extern "C" int ane_scene_create(const float* vertices, int64_t num_vertices, con
   hipError_t e = hipSuccess;
   if ((e = hipEventCreate(&s->ev0)) != hipSuccess || (e = hipEventCreate(&s->ev1)) != hipSuccess)
     return bail(fail_hip(e, "hipEventCreate", __FILE__, __LINE__));
+  if ((e = hipHostMalloc((void**)&s->h_info, sizeof(BuildInfo), kHostFlags)) != hipSuccess)
+    return bail(fail_hip(e, "hipHostMalloc", __FILE__, __LINE__));
   if ((e = hipMemcpyAsync(s->d_vertices, vertices, sizeof(float) * 24 * num_vertices, hipMemcpyHostToDevice, sm)) ||
       (e = hipMemcpyAsync(s->d_indices, indices, sizeof(uint32_t) * num_indices, hipMemcpyHostToDevice, sm)) ||
       (e = hipMemcpyAsync(s->d_meshes, meshes, sizeof(ane_mesh) * num_meshes, hipMemcpyHostToDevice, sm)) ||

@@ -899,7 +899,20 @@ __global__ __launch_bounds__(kSpan) void k_fit_span(SceneK sc, const uint32_t* i
 
 // Treelet roots (flag[i], i < m), top nodes (tflag[i], i < m) and the leaves
 // hanging directly from a top node (sflag[k], k < n); the last slot of each stays
-// 0 so that the exclusive scans end in the totals.
+// 0 so that its exclusive scan ends in the total.  The three lie one after another in the
+// plan's scratch and are scanned at once (a launch of a few blocks takes as long as one of
+// none: three scans were nine of them, 40 us of the rebuild of 246k triangles): PlanScan
+// takes the sections' counts back out.
+struct PlanScan {
+  const uint32_t* g;  // exclusive scan of [n treelet roots][n + 1 strays][n top nodes]
+  int n;
+  __device__ uint32_t unit(int64_t k) const { return g[k]; }
+  __device__ uint32_t stray(int64_t k) const { return g[n + k] - g[n]; }
+  __device__ uint32_t top(int64_t k) const { return g[2 * (int64_t)n + 1 + k] - g[2 * (int64_t)n + 1]; }
+  __device__ uint32_t units() const { return unit(n - 1); }
+  __device__ uint32_t strays() const { return stray(n); }
+  __device__ uint32_t tops() const { return top(n - 1); }
+};
 __global__ __launch_bounds__(256) void k_unit_flags(const int4* topo, const int32_t* leaf_parent, int n,
                                                     uint32_t* flag, uint32_t* sflag, uint32_t* tflag)
 {
@@ -924,28 +937,31 @@ __global__ __launch_bounds__(256) void k_unit_flags(const int4* topo, const int3
   }
 }
 
-__global__ __launch_bounds__(256) void k_unit_scatter(const int4* topo, int n, const uint32_t* pos,
-                                                      const uint32_t* spos, const uint32_t* tpos, int2* units,
-                                                      int32_t* unit_root, int32_t* stray, int32_t* top)
+__global__ __launch_bounds__(256) void k_unit_scatter(const int4* topo, PlanScan p, int2* units, int32_t* unit_root,
+                                                      int32_t* stray, int32_t* top)
 {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n - 1) {
+  if (k < p.n - 1) {
     const int i = (int)k;
-    if (pos[k + 1] != pos[k]) {
+    const uint32_t u = p.unit(k), t = p.top(k);
+    if (p.unit(k + 1) != u) {
       const int j = topo[i].w;
-      units[pos[k]] = make_int2(min(i, j), max(i, j));
-      unit_root[pos[k]] = i;
+      units[u] = make_int2(min(i, j), max(i, j));
+      unit_root[u] = i;
     }
-    if (tpos[k + 1] != tpos[k]) top[tpos[k]] = i;
+    if (p.top(k + 1) != t) top[t] = i;
   }
-  if (k < n && spos[k + 1] != spos[k]) stray[spos[k]] = (int32_t)k;
+  if (k < p.n) {
+    const uint32_t v = p.stray(k);
+    if (p.stray(k + 1) != v) stray[v] = (int32_t)k;
+  }
 }
 
 // Depth of every top node (its ancestors are all top nodes): the walk to the root.
-__global__ __launch_bounds__(256) void k_top_depth(const int32_t* top, const uint32_t* ntop, const int4* topo,
+__global__ __launch_bounds__(256) void k_top_depth(const int32_t* top, PlanScan plan, const int4* topo,
                                                    uint8_t* ndepth)
 {
-  const uint32_t nt = *ntop;
+  const uint32_t nt = plan.tops();
   for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < nt; k += gridDim.x * blockDim.x) {
     const int i = top[k];
     int d = 0, p = topo[i].z;
@@ -959,13 +975,14 @@ __global__ __launch_bounds__(256) void k_top_depth(const int32_t* top, const uin
 
 // The top nodes in depth order (a counting sort in one workgroup; the order
 // within a level is immaterial): cross, and out[d] = the start of depth d in it
-// for d <= kMaxLevels, out[kMaxLevels + 1] = the number of depth levels.
-__global__ __launch_bounds__(1024) void k_top_sort(const int32_t* top, const uint32_t* ntop, const uint8_t* ndepth,
-                                                   int32_t* cross, uint32_t* out)
+// for d <= kMaxLevels, out[kMaxLevels + 1] = the number of depth levels, then the treelet
+// and stray-leaf counts.  out is host memory; *depth is cleared for k_tree_depth.
+__global__ __launch_bounds__(1024) void k_top_sort(const int32_t* top, PlanScan plan, const uint8_t* ndepth,
+                                                   int32_t* cross, uint32_t* out, uint32_t* depth)
 {
   __shared__ uint32_t cnt[kMaxLevels], cur[kMaxLevels];
   __shared__ uint32_t maxd;
-  const uint32_t nt = *ntop;
+  const uint32_t nt = plan.tops();
   if (threadIdx.x < kMaxLevels) cnt[threadIdx.x] = 0u;
   if (threadIdx.x == 0) maxd = 0u;
   __syncthreads();
@@ -984,6 +1001,9 @@ __global__ __launch_bounds__(1024) void k_top_sort(const int32_t* top, const uin
     }
     out[kMaxLevels] = run;
     out[kMaxLevels + 1] = maxd;
+    out[kMaxLevels + 2] = plan.units();
+    out[kMaxLevels + 3] = plan.strays();
+    *depth = 0u;
   }
   __syncthreads();
   for (uint32_t k = threadIdx.x; k < nt; k += blockDim.x) {
@@ -995,11 +1015,15 @@ __global__ __launch_bounds__(1024) void k_top_sort(const int32_t* top, const uin
 // Levels of the tree (internal nodes on the longest root-leaf path): over the
 // treelets, the depth of the root plus the treelet's height; over the top nodes,
 // their depth + 1.
+// (One atomic per block: one of every wave of 256 blocks took 14 us, the atomics' time.)
 __global__ __launch_bounds__(256) void k_tree_depth(const int32_t* unit_root, const uint8_t* uheight, int nunits,
-                                                    const int32_t* top, const uint32_t* ntop, const int4* topo,
+                                                    const int32_t* top, PlanScan plan, const int4* topo,
                                                     const uint8_t* ndepth, uint32_t* out)
 {
-  const uint32_t nt = *ntop;
+  __shared__ uint32_t deepest;
+  if (threadIdx.x == 0) deepest = 0u;
+  __syncthreads();
+  const uint32_t nt = plan.tops();
   uint32_t best = 0u;
   for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < (int64_t)nunits + nt;
        k += (int64_t)gridDim.x * blockDim.x) {
@@ -1010,7 +1034,16 @@ __global__ __launch_bounds__(256) void k_tree_depth(const int32_t* unit_root, co
       best = max(best, (uint32_t)ndepth[top[k - nunits]] + 1u);
     }
   }
-  atomicMax(out, best);
+  if (best) atomicMax(&deepest, best);
+  __syncthreads();
+  if (threadIdx.x == 0) atomicMax(out, deepest);
+}
+
+// What the host reads after a build, to host memory: the depth and the grid's frame.
+__global__ void k_build_info(const uint32_t* depth, const GridFrame* frame, uint32_t* out_depth, GridFrame* out_frame)
+{
+  *out_depth = *depth;
+  *out_frame = *frame;
 }
 
 // Refit: the leaf-order triangles of the leaves outside every treelet.
@@ -1129,54 +1162,60 @@ void launch_reorder(const float* world, const uint32_t* ids, int n, float4* tris
 }
 
 int launch_fit_plan(const int4* topo, const int32_t* leaf_parent, int n, uint32_t* scratch, uint32_t* uscratch,
-                    uint32_t* info, uint8_t* ndepth, int32_t* cross, int32_t* top, int2* units, int32_t* unit_root,
-                    int32_t* stray, std::vector<int32_t>* cross_begin, int* nunits, int* nstray, hipStream_t s)
+                    uint32_t* h_info, uint32_t* depth, uint8_t* ndepth, int32_t* cross, int32_t* top, int2* units,
+                    int32_t* unit_root, int32_t* stray, std::vector<int32_t>* cross_begin, int* nunits, int* nstray,
+                    hipStream_t s)
 {
   cross_begin->clear();
   *nunits = 0;
   *nstray = 0;
   if (n < 2) return 0;
-  const int64_t m = n - 1;
-  uint32_t* upos = uscratch;              // m + 1 words
-  uint32_t* spos = uscratch + n;          // n + 1 words
-  uint32_t* tpos = uscratch + 2 * n + 1;  // m + 1 words
   hipLaunchKernelGGL(k_unit_flags, dim3(blocks_for((int64_t)n + 1, 256)), dim3(256), 0, s, topo, leaf_parent, n,
-                     upos, spos, tpos);
-  exclusive_scan(upos, m + 1, scratch, s);
-  exclusive_scan(spos, (int64_t)n + 1, scratch, s);
-  exclusive_scan(tpos, m + 1, scratch, s);
-  hipLaunchKernelGGL(k_unit_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, s, topo, n, (const uint32_t*)upos,
-                     (const uint32_t*)spos, (const uint32_t*)tpos, units, unit_root, stray, top);
-  const uint32_t* ntop = tpos + m;
-  hipLaunchKernelGGL(k_top_depth, dim3(1024), dim3(256), 0, s, (const int32_t*)top, ntop, topo, ndepth);
-  hipLaunchKernelGGL(k_top_sort, dim3(1), dim3(1024), 0, s, (const int32_t*)top, ntop, (const uint8_t*)ndepth,
-                     cross, info);
-  // info: [0, kMaxLevels] top-level offsets, [kMaxLevels + 1] levels, then the treelet
-  // and stray-leaf counts
-  if (hipMemcpyAsync(info + kMaxLevels + 2, upos + m, 4, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-      hipMemcpyAsync(info + kMaxLevels + 3, spos + n, 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
-    return -1;
-  uint32_t h[kMaxLevels + 4];
-  if (hipMemcpyAsync(h, info, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess) return -1;
-  if (hipStreamSynchronize(s) != hipSuccess) return -1;
-  const int levels = (int)h[kMaxLevels + 1];
-  for (int d = 0; d <= levels && d <= kMaxLevels; ++d) cross_begin->push_back((int32_t)h[d]);
+                     uscratch, uscratch + n, uscratch + 2 * (int64_t)n + 1);
+  exclusive_scan(uscratch, 3 * (int64_t)n + 1, scratch, s);
+  const PlanScan plan{uscratch, n};
+  hipLaunchKernelGGL(k_unit_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, s, topo, plan, units, unit_root, stray,
+                     top);
+  hipLaunchKernelGGL(k_top_depth, dim3(1024), dim3(256), 0, s, (const int32_t*)top, plan, topo, ndepth);
+  hipLaunchKernelGGL(k_top_sort, dim3(1), dim3(1024), 0, s, (const int32_t*)top, plan, (const uint8_t*)ndepth, cross,
+                     h_info, depth);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) return -1;
+  const int levels = (int)h_info[kMaxLevels + 1];
+  for (int d = 0; d <= levels && d <= kMaxLevels; ++d) cross_begin->push_back((int32_t)h_info[d]);
   if (cross_begin->size() < 2) cross_begin->push_back(0);
-  *nunits = (int)h[kMaxLevels + 2];
-  *nstray = (int)h[kMaxLevels + 3];
+  *nunits = (int)h_info[kMaxLevels + 2];
+  *nstray = (int)h_info[kMaxLevels + 3];
   return 0;
 }
 
-int launch_tree_depth(const int4* topo, int n, const int32_t* unit_root, const uint8_t* uheight, int nunits,
-                      const int32_t* top, const uint32_t* uscratch, const uint8_t* ndepth, uint32_t* out,
-                      hipStream_t s)
+void launch_tree_depth(const int4* topo, int n, const int32_t* unit_root, const uint8_t* uheight, int nunits,
+                       const int32_t* top, const uint32_t* uscratch, const uint8_t* ndepth, uint32_t* depth,
+                       const GridFrame* frame, uint32_t* h_depth, GridFrame* h_frame, hipStream_t s)
 {
-  if (n < 2) return 0;
-  if (hipMemsetAsync(out, 0, 4, s) != hipSuccess) return -1;
-  const uint32_t* ntop = uscratch + 2 * n + 1 + (n - 1);
-  hipLaunchKernelGGL(k_tree_depth, dim3(256), dim3(256), 0, s, unit_root, uheight, nunits, top, ntop, topo, ndepth,
-                     out);
-  return 0;
+  if (n < 2) return;
+  hipLaunchKernelGGL(k_tree_depth, dim3(64), dim3(256), 0, s, unit_root, uheight, nunits, top, PlanScan{uscratch, n},
+                     topo, ndepth, depth);
+  hipLaunchKernelGGL(k_build_info, dim3(1), dim3(1), 0, s, (const uint32_t*)depth, frame, h_depth, h_frame);
+}
+
+// The instances and their inverse transforms from pinned host memory, read by the kernel
+// itself: two copies by the DMA engines put 50 us between the kernels before and after them
+// for 2,000 instances.
+__global__ __launch_bounds__(256) void k_upload(const uint4* a, uint4* da, int64_t na, const uint4* b, uint4* db,
+                                                int64_t nb)
+{
+  for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < na + nb; k += (int64_t)gridDim.x * 256) {
+    if (k < na) da[k] = a[k];
+    else db[k - na] = b[k - na];
+  }
+}
+
+void launch_upload(const void* a, void* da, int64_t a_bytes, const void* b, void* db, int64_t b_bytes, hipStream_t s)
+{
+  const int64_t na = a_bytes / 16, nb = b_bytes / 16;
+  if (na + nb <= 0) return;
+  hipLaunchKernelGGL(k_upload, dim3((unsigned)std::min<int64_t>((na + nb + 255) / 256, 1024)), dim3(256), 0, s,
+                     (const uint4*)a, (uint4*)da, na, (const uint4*)b, (uint4*)db, nb);
 }
 
 void launch_fit(float4* tris, int n, NodeBuild* nodes, float* node_box, uint4* qnodes, const int4* topo,

@@ -36,16 +36,22 @@ void launch_world_from_tris(const float4* tris, int n, float* world, hipStream_t
 // ranges and roots, the leaves directly under a top node, the top nodes in depth
 // order (cross) with the start of each depth level (cross_begin, one past the
 // last level at the end) and their depths (ndepth, by node).  scratch:
-// radix_scratch_words(n) words, uscratch: 3 n + 3 words, info: 136 words; cross,
-// top, units, unit_root: n - 1 entries, stray: n entries.
+// radix_scratch_words(n) words, uscratch: 3 n + 3 words, h_info: 132 words of coherent host
+// memory, depth: a device word that is cleared; cross, top, units, unit_root: n - 1
+// entries, stray: n entries.  Synchronizes the stream.
 int launch_fit_plan(const int4* topo, const int32_t* leaf_parent, int n, uint32_t* scratch, uint32_t* uscratch,
-                    uint32_t* info, uint8_t* ndepth, int32_t* cross, int32_t* top, int2* units, int32_t* unit_root,
-                    int32_t* stray, std::vector<int32_t>* cross_begin, int* nunits, int* nstray, hipStream_t s);
-// After a build's fit: the number of internal levels on the longest root-leaf path
-// into *out (device word), from the treelet heights and the top-node depths.
-int launch_tree_depth(const int4* topo, int n, const int32_t* unit_root, const uint8_t* uheight, int nunits,
-                      const int32_t* top, const uint32_t* uscratch, const uint8_t* ndepth, uint32_t* out,
-                      hipStream_t s);
+                    uint32_t* h_info, uint32_t* depth, uint8_t* ndepth, int32_t* cross, int32_t* top, int2* units,
+                    int32_t* unit_root, int32_t* stray, std::vector<int32_t>* cross_begin, int* nunits, int* nstray,
+                    hipStream_t s);
+// After a build's fit: the number of internal levels on the longest root-leaf path, from
+// the treelet heights and the top-node depths, and the grid's frame, into coherent host
+// memory (complete once the stream is synchronized; nothing for n < 2).  depth: the word
+// cleared by the plan.
+void launch_tree_depth(const int4* topo, int n, const int32_t* unit_root, const uint8_t* uheight, int nunits,
+                       const int32_t* top, const uint32_t* uscratch, const uint8_t* ndepth, uint32_t* depth,
+                       const GridFrame* frame, uint32_t* h_depth, GridFrame* h_frame, hipStream_t s);
+// two arrays of multiples of 16 bytes from mapped, coherent host memory to the device
+void launch_upload(const void* a, void* da, int64_t a_bytes, const void* b, void* db, int64_t b_bytes, hipStream_t s);
 // Bottom-up boxes: one launch for every treelet (LDS-local walks), then the top
 // nodes level by level (no inter-workgroup fences).
 // refit (refits): the leaf-order triangles are first made from the triangle
