@@ -298,15 +298,16 @@ void exclusive_scan(uint32_t* data, int64_t n, uint32_t* scratch, hipStream_t s)
 // ---------------------------------------------------------------------------
 // stable LSD radix sort of (uint64 key, uint32 value), 8-bit digits
 // ---------------------------------------------------------------------------
+template <int ITEMS>
 __global__ __launch_bounds__(kBlock) void k_radix_hist(const uint64_t* keys, int64_t n, int shift,
                                                       uint32_t* hist, int64_t ntiles)
 {
   __shared__ uint32_t h[256];
   h[threadIdx.x] = 0;
   __syncthreads();
-  int64_t base = (int64_t)blockIdx.x * kTile;
+  int64_t base = (int64_t)blockIdx.x * (ITEMS * kBlock);
 #pragma unroll
-  for (int i = 0; i < kItems; ++i) {
+  for (int i = 0; i < ITEMS; ++i) {
     int64_t idx = base + i * kBlock + threadIdx.x;
     if (idx < n) atomicAdd(&h[(uint32_t)(keys[idx] >> shift) & 255u], 1u);
   }
@@ -341,45 +342,45 @@ __global__ __launch_bounds__(kBlock) void k_radix_digit_scan(uint32_t* hist, int
 }
 
 // Stable scatter of one tile: digit d of tile t goes to (digits below d in all
-// tiles) + (digit d in the tiles before t) + (rank within the tile).  The tile is
-// first ordered by digit in LDS (ranks by ballots, as a stable counting sort), so
-// that consecutive threads write consecutive addresses of each digit's run.
+// tiles) + (digit d in the tiles before t) + (rank within the tile).  A wave ranks its own
+// run of 64 ITEMS keys, 64 at a time by ballots, against digit counters of its own, so that
+// the rounds need no barrier (with counters of the block and three barriers a round a rebuild
+// of 97k / 259k / 1.05M / 3.92M triangles took 358 / 393 / 590 / 1469 us, now 218 / 267 / 486 /
+// 1326).  The tile is then ordered by digit in LDS, so that consecutive
+// threads write consecutive addresses of each digit's run.
+template <int ITEMS>
 __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* kin, const uint32_t* vin,
                                                          uint64_t* kout, uint32_t* vout, int64_t n,
                                                          int shift, const uint32_t* offs,
                                                          const uint32_t* totals, int64_t ntiles)
 {
-  __shared__ uint32_t run[256];    // next tile-local position of each digit
-  __shared__ uint32_t gbase[256];  // global position of the tile's digit d, minus its local start
-  __shared__ uint32_t wcnt[kBlock / 64][256];
-  __shared__ uint64_t skey[kTile];
-  __shared__ uint32_t sval[kTile];
+  constexpr int kWaves = kBlock / 64;
+  constexpr int kKeys = ITEMS * kBlock;
+  __shared__ uint32_t wcnt[kWaves][256];  // a wave's digit counts, then its first tile-local position of each
+  __shared__ uint32_t gbase[256];         // global position of the tile's digit d, minus its local start
+  __shared__ uint64_t skey[kKeys];
+  __shared__ uint32_t sval[kKeys];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  const int64_t base = (int64_t)blockIdx.x * kTile;
-  const int tn = (int)min((int64_t)kTile, n - base);
-  uint64_t key[kItems];
-  uint32_t val[kItems];
-  run[threadIdx.x] = 0u;
-  __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * kKeys;
+  const int tn = (int)min((int64_t)kKeys, n - base);
+  const int64_t first = base + wave * (ITEMS * 64) + lane;
+  uint64_t key[ITEMS];
+  uint32_t val[ITEMS], loc[ITEMS];
 #pragma unroll
-  for (int r = 0; r < kItems; ++r) {
-    const int64_t idx = base + r * kBlock + threadIdx.x;
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t idx = first + r * 64;
     key[r] = idx < n ? kin[idx] : 0ull;
     val[r] = idx < n ? vin[idx] : 0u;
-    if (idx < n) atomicAdd(&run[(uint32_t)(key[r] >> shift) & 255u], 1u);
   }
-  __syncthreads();
-  uint32_t tot;
-  const uint32_t lstart = block_exclusive_scan(run[threadIdx.x], &tot);
-  const uint32_t below = block_exclusive_scan(totals[threadIdx.x], &tot);
-  gbase[threadIdx.x] = below + offs[(int64_t)threadIdx.x * ntiles + blockIdx.x] - lstart;
-  run[threadIdx.x] = lstart;
-  for (int r = 0; r < kItems; ++r) {
+  const uint32_t dig_total = totals[threadIdx.x], dig_off = offs[(int64_t)threadIdx.x * ntiles + blockIdx.x];
 #pragma unroll
-    for (int w = 0; w < kBlock / 64; ++w) wcnt[w][threadIdx.x] = 0;
-    __syncthreads();
-    const bool valid = base + r * kBlock + threadIdx.x < n;
+  for (int k = lane; k < 256; k += 64) wcnt[wave][k] = 0u;
+  volatile uint32_t* const cnt = wcnt[wave];  // this wave's alone until the barrier
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const bool valid = first + r * 64 < n;
     const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
     uint64_t mask = __ballot(valid);
 #pragma unroll
@@ -389,20 +390,32 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* kin, c
       mask &= bit ? bal : ~bal;
     }
     const uint32_t rank = (uint32_t)__popcll(mask & lt);
-    if (valid && rank == 0) wcnt[wave][d] = (uint32_t)__popcll(mask);
-    __syncthreads();
-    if (valid) {
-      uint32_t q = run[d];
-      for (int w = 0; w < wave; ++w) q += wcnt[w][d];
-      q += rank;
+    const uint32_t before = cnt[d];  // the LDS takes a wave's accesses in order
+    __builtin_amdgcn_wave_barrier();
+    loc[r] = before + rank;
+    if (valid && rank == 0) cnt[d] = before + (uint32_t)__popcll(mask);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  uint32_t c[kWaves], all = 0u, tot;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    c[w] = all;
+    all += wcnt[w][threadIdx.x];
+  }
+  const uint32_t lstart = block_exclusive_scan(all, &tot);
+  const uint32_t below = block_exclusive_scan(dig_total, &tot);
+  gbase[threadIdx.x] = below + dig_off - lstart;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) wcnt[w][threadIdx.x] = lstart + c[w];
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    if (first + r * 64 < n) {
+      const uint32_t q = wcnt[wave][(uint32_t)(key[r] >> shift) & 255u] + loc[r];
       skey[q] = key[r];
       sval[q] = val[r];
     }
-    __syncthreads();
-    uint32_t add = 0;
-#pragma unroll
-    for (int w = 0; w < kBlock / 64; ++w) add += wcnt[w][threadIdx.x];
-    run[threadIdx.x] += add;
   }
   __syncthreads();
   for (int q = threadIdx.x; q < tn; q += kBlock) {
@@ -415,19 +428,24 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* kin, c
   }
 }
 
+// Keys per thread of a tile: the larger the tile, the longer the runs that it writes; the
+// smaller, the shorter its chain and the more of the chip has one.  Rebuilds with 2 / 4 / 8:
+// 4k triangles 183 / 196 / 213 us, 97k 218 / 226 / 248, 180k 245 / 244 / 265, 524k 356 / 336 /
+// 340, 1.05M 559 / 501 / 486, 3.92M 1603 / 1426 / 1326.
+static int radix_items(int64_t n) { return n > 1 << 19 ? 8 : (n > 1 << 17 ? 4 : 2); }
+
+static int64_t radix_tiles(int64_t n) { return (n + radix_items(n) * kBlock - 1) / (radix_items(n) * kBlock); }
+
 int64_t radix_scratch_words(int64_t n)
 {
-  int64_t ntiles = (n + kTile - 1) / kTile;
-  return 256 * ntiles + 256;  // tile histograms, digit totals
+  return 256 * radix_tiles(n) + 256;  // tile histograms, digit totals
 }
 
-// Sorts (keys, vals) in place using (k2, v2) as ping-pong buffers (8 passes:
-// the result ends in keys/vals).  scratch: radix_scratch_words(n) words.
-void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* k2, uint32_t* v2, int64_t n,
-                      uint32_t* scratch, hipStream_t s)
+template <int ITEMS>
+static void radix_passes(uint64_t* keys, uint32_t* vals, uint64_t* k2, uint32_t* v2, int64_t n, uint32_t* scratch,
+                         hipStream_t s)
 {
-  if (n <= 1) return;
-  int64_t ntiles = (n + kTile - 1) / kTile;
+  const int64_t ntiles = radix_tiles(n);
   uint32_t* hist = scratch;
   uint32_t* totals = scratch + 256 * ntiles;
   uint64_t* ka = keys;
@@ -436,16 +454,28 @@ void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* k2, uint32_t* v2
   uint32_t* vb = v2;
   for (int pass = 0; pass < 8; ++pass) {
     int shift = 8 * pass;
-    hipLaunchKernelGGL(k_radix_hist, dim3((unsigned)ntiles), dim3(kBlock), 0, s, (const uint64_t*)ka,
+    hipLaunchKernelGGL(k_radix_hist<ITEMS>, dim3((unsigned)ntiles), dim3(kBlock), 0, s, (const uint64_t*)ka,
                        n, shift, hist, ntiles);
     hipLaunchKernelGGL(k_radix_digit_scan, dim3(256), dim3(kBlock), 0, s, hist, ntiles, totals);
-    hipLaunchKernelGGL(k_radix_scatter, dim3((unsigned)ntiles), dim3(kBlock), 0, s,
+    hipLaunchKernelGGL(k_radix_scatter<ITEMS>, dim3((unsigned)ntiles), dim3(kBlock), 0, s,
                        (const uint64_t*)ka, (const uint32_t*)va, kb, vb, n, shift,
                        (const uint32_t*)hist, (const uint32_t*)totals, ntiles);
     uint64_t* tk = ka; ka = kb; kb = tk;
     uint32_t* tv = va; va = vb; vb = tv;
   }
   // 8 passes: data is back in (keys, vals)
+}
+
+// Sorts (keys, vals) in place using (k2, v2) as ping-pong buffers (8 passes:
+// the result ends in keys/vals).  scratch: radix_scratch_words(n) words.
+void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* k2, uint32_t* v2, int64_t n,
+                      uint32_t* scratch, hipStream_t s)
+{
+  if (n <= 1) return;
+  const int items = radix_items(n);
+  if (items == 8) radix_passes<8>(keys, vals, k2, v2, n, scratch, s);
+  else if (items == 4) radix_passes<4>(keys, vals, k2, v2, n, scratch, s);
+  else radix_passes<2>(keys, vals, k2, v2, n, scratch, s);
 }
 
 // ---------------------------------------------------------------------------
