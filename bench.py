@@ -828,9 +828,10 @@ def main():
                 "traffic_source": "profiles/trace_terrain1m_traffic.md" if traffic else None,
                 "algorithmic_bytes": int(algo[dom]), "mean_ms": round(mean[dom], 4)}
         if ach > HBM_PEAK_GBS:
-            roof["note"] = ("algorithmic bytes above the HBM peak: the node and triangle reads are served "
-                            "by L2 and the Infinity Cache (traffic: the HBM bytes per launch); the kernel "
-                            "is bound by VALU issue")
+            roof["note"] = ("algorithmic bytes above the HBM peak: they are the counting traversal's, of one "
+                            "64-byte node per level; the timed kernel reads two levels per node, and L2 and "
+                            "the Infinity Cache serve it (traffic: the HBM bytes per launch); it is bound by "
+                            "VALU issue")
         if "shadow" in algo and mean.get("shadow", 0.0) > 0.0:
             sh = algo["shadow"] / (mean["shadow"] / 1000.0) / 1e9
             roof["shadow_kernel"] = {"achieved": round(sh, 1), "frac": round(sh / HBM_PEAK_GBS, 4),
