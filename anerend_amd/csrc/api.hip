@@ -227,6 +227,12 @@ struct SunGridCache {
     }
   } built, seen;
   uint64_t builds = 0;        // grids built so far
+  uint32_t id = 0;            // SunGridParams::id of `built`; another key takes the next one
+  // A graph the caller captured may hold a build and run it at any time, or never: `captured`
+  // is that the current build was only captured, `replayable` that some build was, so that
+  // the host never again knows which grid the device holds.
+  bool captured = false, replayable = false;
+  bool own_graph = false;     // the stream captures into a graph that runs once, right after the capture
   // the validity flag of a build, read back without blocking: copied to pinned
   // memory behind an event (not under stream capture) and taken once the event
   // has completed.  `known` is the build whose flag last_valid holds; a newer
@@ -235,6 +241,7 @@ struct SunGridCache {
   hipEvent_t ev = nullptr;
   bool pending = false;
   Key pend, known;
+  uint32_t pend_id = 0;
   int last_valid = -1;
 
   void release()
@@ -245,6 +252,7 @@ struct SunGridCache {
     est_words = 0;
     bytes = 0;
     built = Key{};
+    captured = false;
     pending = false;
     known = Key{};
     last_valid = -1;
@@ -267,8 +275,9 @@ struct SunGridCache {
       return;
     }
     pending = false;
-    if (q == hipSuccess) {
-      last_valid = *reinterpret_cast<volatile uint32_t*>(h_valid) ? 1 : 0;
+    const uint32_t v = *reinterpret_cast<volatile uint32_t*>(h_valid);
+    if (q == hipSuccess && (v == 0u || v == pend_id)) {  // else another build's
+      last_valid = v ? 1 : 0;
       known = pend;
     }
   }
@@ -282,6 +291,7 @@ struct SunGridCache {
     ANE_CHECK_HIP(hipMemcpyAsync(h_valid, &params->valid, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     ANE_CHECK_HIP(hipEventRecord(ev, st));
     pend = k;
+    pend_id = id;
     pending = true;
     return ANE_OK;
   }
@@ -297,6 +307,7 @@ struct SunGridCache {
     release();
     const int64_t ncell = (int64_t)gg * gg;
     ANE_TRY(dalloc(&params, 1, &bytes));
+    ANE_CHECK_HIP(hipMemset(params, 0, sizeof(*params)));  // no grid in use
     ANE_TRY(dalloc(&acc, 6 * 256, &bytes));
     ANE_TRY(dalloc(&start, ncell + 1, &bytes));
     ANE_TRY(dalloc(&cur, ncell, &bytes));
@@ -309,8 +320,8 @@ struct SunGridCache {
     return ANE_OK;
   }
   // 1 / 0: the current build is known on the host to be in use / left out, -1: not known
-  // yet (the launches of a call then decide on the device)
-  int known_valid() const { return built.set && known == built ? last_valid : -1; }
+  // (the launches of a call then decide on the device)
+  int known_valid() const { return !replayable && built.set && known == built ? last_valid : -1; }
   // *use: the grid for (scene, version, dir) is current after the call.  A
   // direction with a zero (or non-finite) component never gets one: its rays
   // can lie exactly in a box face, where the traversal's slab test (zero
@@ -336,10 +347,12 @@ struct SunGridCache {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     ANE_CHECK_HIP(hipStreamIsCapturing(st, &cs));
     const bool capturing = cs != hipStreamCaptureStatusNone;
+    const bool callers = capturing && !own_graph;  // a graph of the caller's
     if (!capturing) poll();  // no event queries under capture
-    if (built == k) {
+    const bool current = built == k;
+    if (current && (capturing || !captured)) {
       *use = true;
-      if (!capturing && !(known == k)) ANE_TRY(read_back(k, st));
+      if (!capturing && !replayable && !(known == k)) ANE_TRY(read_back(k, st));
       if (valid) *valid = capturing ? -1 : known_valid();  // a graph keeps both ways: the grid may change before a replay
       return ANE_OK;
     }
@@ -350,7 +363,7 @@ struct SunGridCache {
     const bool moving = valid_scene || (!judged && seen.set && seen.scene == scene && seen.version == version);
     const bool eager = (valid_scene && rays >= (int64_t)ANE_SUNGRID_EAGER_RAYS * ntri) ||
                        (moving && sun_grid_pays(rays, ntri));
-    if (!ANE_SUNGRID_EAGER && !eager && !(seen == k)) {
+    if (!ANE_SUNGRID_EAGER && !eager && !current && !(seen == k)) {
       seen = k;
       return ANE_OK;
     }
@@ -358,17 +371,21 @@ struct SunGridCache {
     ANE_TRY(alloc(ntri));
     SunGridParams p;
     sun_grid_setup(p, dir3, g, g);
+    if (!current) id = id == UINT32_MAX ? 1u : id + 1u;
+    p.id = id;
     launch_sun_grid_build(view, p, params, acc, start, cur, list, cap, scan, est, clk, stage, st);
     ANE_CHECK_HIP(hipGetLastError());
     built = k;
     ++builds;
-    if (!capturing) ANE_TRY(read_back(k, st));
+    captured = callers;
+    replayable = replayable || callers;
+    if (!capturing && !replayable) ANE_TRY(read_back(k, st));
     *use = true;
     return ANE_OK;
   }
-  SunGridK view() const { return SunGridK{params, start, list}; }
-  // device address of the validity flag (the traversal launches skip when it is set)
-  const uint32_t* valid_flag() const { return &params->valid; }
+  SunGridK view() const { return SunGridK{params, start, list, id}; }
+  // for the traversal launches that do nothing while the current build is in use
+  SunGridSkip skip() const { return SunGridSkip{&params->valid, id}; }
 };
 
 // ===========================================================================
@@ -1415,11 +1432,15 @@ int ddgi_update_graph(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame*
   if (e != hipSuccess) {
     return fail(ANE_ERR_DEVICE, "hipStreamBeginCapture: %s", hipGetErrorString(e));
   }
+  const uint64_t builds = c->sgc.builds;
+  c->sgc.own_graph = true;
   const int r = ane_ddgi_update(c, s, f, st);
+  c->sgc.own_graph = false;
   hipGraph_t g = nullptr;
   e = hipStreamEndCapture(st, &g);
   if (r != ANE_OK || e != hipSuccess || !g) {
     if (g) (void)hipGraphDestroy(g);
+    if (c->sgc.builds != builds) c->sgc.built = SunGridCache::Key{};  // its build did not run
     return r != ANE_OK ? r : fail(ANE_ERR_DEVICE, "hipStreamEndCapture: %s", hipGetErrorString(e));
   }
   if (c->gexec) {
@@ -1434,7 +1455,10 @@ int ddgi_update_graph(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame*
   if (!c->gexec) e = hipGraphInstantiate(&c->gexec, g, nullptr, nullptr, 0);
   if (e == hipSuccess) e = hipGraphLaunch(c->gexec, st);
   (void)hipGraphDestroy(g);
-  if (e != hipSuccess) return fail(ANE_ERR_DEVICE, "graph launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {
+    if (c->sgc.builds != builds) c->sgc.built = SunGridCache::Key{};
+    return fail(ANE_ERR_DEVICE, "graph launch: %s", hipGetErrorString(e));
+  }
   return ANE_OK;
 }
 }  // namespace ane
@@ -1670,7 +1694,7 @@ extern "C" int ane_ddgi_mirror_reflections(ane_ddgi_ctx* c, const ane_scene* s, 
   const float sun3[3] = {sun.x, sun.y, sun.z};
   // through the sun grid once it is current, else (or while its validity is not known
   // here: decided by a device flag) by traversal
-  const uint32_t* skip = nullptr;
+  SunGridSkip skip{};
   int valid = 0;
   if (!counters4 && sun_grid_wanted(c)) {
     bool use = false;
@@ -1678,12 +1702,12 @@ extern "C" int ane_ddgi_mirror_reflections(ane_ddgi_ctx* c, const ane_scene* s, 
     if (!use) valid = 0;
     if (valid != 0) {
       launch_mirror_shadow_grid(s->view, c->d_mr_hits[0], slots, sun3, c->sgc.view(), 0.1f, 50.0f, c->d_mr_hits[1], st);
-      skip = c->sgc.valid_flag();
+      skip = c->sgc.skip();
     }
   }
   if (valid != 1) {
     launch_mirror_shadow_rays(s->view, c->d_mr_hits[0], slots, sun3, c->d_mr_orig[1], c->d_mr_dir[1], st, skip);
-    a.skip_if_set = skip;
+    a.skip = skip;
     a.hits = c->d_mr_hits[1];
     a.work = c->d_mr_work + kTraceWorkWords;
     a.stats = c->d_mr_stats + 2;
@@ -1930,7 +1954,7 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
   // without counters the rays go through the scene's grid along -light_dir once it is
   // current; while its validity is not known here, the traversal launches follow and do
   // nothing when it is (device flag)
-  const uint32_t* skip = nullptr;
+  SunGridSkip skip{};
   s->sh_traced = true;
   if (!counters2) {
     const float dir[3] = {-light3[0], -light3[1], -light3[2]};
@@ -1945,7 +1969,7 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
         ANE_CHECK_HIP(hipGetLastError());
         return ANE_OK;
       }
-      skip = s->sgc.valid_flag();
+      skip = s->sgc.skip();
     }
   }
   if (n > s->shadow_px) {
@@ -1986,7 +2010,7 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
   a.ray_dir = s->d_sh_dir;
   a.t_min = 0.1f;  // shadow.rgen:66-67
   a.t_max = 50.0f;
-  a.skip_if_set = skip;
+  a.skip = skip;
   launch_trace(a, true, true, counters2 != nullptr, st);
   launch_shadow_resolve(depth, s->d_sh_hits, n, out_vis, st, skip);
   ANE_CHECK_HIP(hipGetLastError());

@@ -153,7 +153,8 @@ struct SunGridParams {
   float sx, sy, margin;    // shear of the direction; widening of the triangle rectangles
   int32_t kx, ky, kz;      // axis permutation (the watertight test's)
   int32_t gx, gy;          // cells
-  uint32_t valid;          // 0: the traversal takes the shadow rays
+  uint32_t id;             // of the build's scene version and direction (never 0)
+  uint32_t valid;          // id while the grid is in use, 0: the traversal takes the shadow rays
   float est;               // mean candidates of a ray from a triangle (over triangles)
   float max_est;           // above it the grid is not used (traversal is cheaper)
 };
@@ -161,7 +162,17 @@ struct SunGridK {
   const SunGridParams* params;  // device
   const uint32_t* start;        // [gx * gy + 1] first candidate of each cell
   const uint2* list;            // candidates (sorted triangle position, sun_bounds in the cell); null: no grid
+  uint32_t id;                  // the grid the launch was prepared for
 };
+// A launch may meet the grid of another direction or scene version than it was prepared
+// for: a graph that holds a build writes the grid again whenever it is replayed, unseen by
+// the host.  So the flag names the grid, and a launch uses, or skips for, its own alone.
+struct SunGridSkip {
+  const uint32_t* valid;  // null: never
+  uint32_t id;
+};
+__device__ __forceinline__ bool sun_grid_in_use(const SunGridK& sg) { return sg.params->valid == sg.id; }
+__device__ __forceinline__ bool sun_grid_answered(const SunGridSkip& k) { return k.valid && *k.valid == k.id; }
 __host__ __device__ __forceinline__ int sun_cell(float v, float o, float inv, int n)
 {
   float f = floorf((v - o) * inv);
@@ -182,7 +193,7 @@ void sun_grid_setup(SunGridParams& g, const float* dir3, int gx, int gy);
 // slots of the tile order of a W x H image (at least its pixels)
 int64_t pixel_slot_count(int W, int H);
 // the shadow mask through the grid of its rays' direction (zero or non-finite
-// direction: no ray); does nothing unless the grid is valid
+// direction: no ray); does nothing unless the grid is in use
 void launch_shadow_mask_grid(const float* depth, int W, int H, const float* ivp16, const float* light3,
                              const SunGridK& sg, const SceneK& sc, float* vis, hipStream_t s);
 // est: [sun_grid_scratch_words(ntri)] build scratch (partial sums of the candidate
@@ -232,7 +243,7 @@ struct TraceArgs {
   float t_min, t_max;
   const float* ray_tmax;   // caller rays: per-ray t_max (null: t_max for every ray)
   SunGridK sg;             // probe rays: candidates of the shadow rays (list null: traversal)
-  const uint32_t* skip_if_set; // caller rays: the launch does nothing when *skip_if_set != 0
+  SunGridSkip skip;        // caller rays: the launch does nothing when this grid is in use
   ClockArg clk;            // probe rays: stage stamps
 };
 
@@ -324,7 +335,7 @@ void launch_gi_lookup(const GridK& g, const FrameK& f, const float* atlas, const
 // RT hard shadows: per-pixel rays (orig, dirs: W*H*3 floats) and visibility
 void launch_shadow_rays(const float* depth, int W, int H, const float* ivp16, const float* light3,
                         float* orig, float* dirs, uint32_t* clear, int nclear, hipStream_t s,
-                        const uint32_t* skip_if_set = nullptr);
+                        const SunGridSkip& skip = SunGridSkip{});
 // point-light shadow moments: lights = n x 8 floats {x, y, z, range, r, g, b, enabled};
 // 1024 rays per light; lw / lidx [kmax][64 texels] = each texel's (weight, ray) pairs
 // with weight above 0.001 in the summation order, padded with weight 0
@@ -336,14 +347,14 @@ void launch_light_rays(const float* lights, int n, const float* dirs, const uint
 void launch_light_moments(const float* lights, int n, const uint32_t* order, const ane_hit* hits, const float* lw,
                           const int32_t* lidx, int kmax, float* dist_img, float* mom, hipStream_t s);
 void launch_shadow_resolve(const float* depth, const ane_hit* hits, int64_t n, float* vis, hipStream_t s,
-                           const uint32_t* skip_if_set = nullptr);
+                           const SunGridSkip& skip = SunGridSkip{});
 // mirror reflections: reflection rays in slot order (pixel_slot_count(W, H) of them), the
 // shadow rays of their hits for the traversal or through a sun grid, shading.  clear:
 // [nclear] words set to 0 before the launches that follow.
 void launch_mirror_rays(const float* depth, const float* normal4, int W, int H, const float* ivp16,
                         const float* cam3, float* orig, float* dirs, uint32_t* clear, int nclear, hipStream_t s);
 void launch_mirror_shadow_rays(const SceneK& sc, const ane_hit* hits, int64_t n, const float* sun3, float* orig,
-                               float* dirs, hipStream_t s, const uint32_t* skip_if_set);
+                               float* dirs, hipStream_t s, const SunGridSkip& skip);
 void launch_mirror_shadow_grid(const SceneK& sc, const ane_hit* hits, int64_t n, const float* sun3,
                                const SunGridK& sg, float tmin, float tmax, ane_hit* shadow_hits, hipStream_t s);
 void launch_mirror_shade(const SceneK& sc, const GridK& g, const FrameK& f, const float* atlas,

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kBoundBlocks) void k_sun_params(SunGridParams g, co
   r.y0 = y0;
   r.icw = (x1 > x0) ? (float)g.gx / (x1 - x0) : 0.0f;
   r.ich = (y1 > y0) ? (float)g.gy / (y1 - y0) : 0.0f;
-  r.valid = (acc[5] == 0u && isfinite(r.icw) && isfinite(r.ich)) ? 1u : 0u;
+  r.valid = (acc[5] == 0u && isfinite(r.icw) && isfinite(r.ich)) ? g.id : 0u;
   *out = r;
 }
 

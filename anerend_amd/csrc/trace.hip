@@ -370,9 +370,9 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_TRACE_W
   constexpr int kUnroll = Q ? ANE_TRACE_UNROLL_Q : ANE_TRACE_UNROLL;
   // with a sun grid in use, the probe shadow rays are k_probe_shadow_grid's
   // (launched after this kernel): the lanes here end at the primary hit
-  const bool sgrid = !RAYS && a.sg.list != nullptr && a.sg.params->valid != 0u;
+  const bool sgrid = !RAYS && a.sg.list != nullptr && sun_grid_in_use(a.sg);
   __shared__ int32_t stk[kSS][kTB];
-  if (RAYS && a.skip_if_set && *a.skip_if_set != 0u) return;  // a sun grid answered these rays
+  if (RAYS && sun_grid_answered(a.skip)) return;  // a sun grid answered these rays
   if (!RAYS) clock_begin(a.clk, kTraceRays);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -702,12 +702,12 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
   constexpr uint32_t kRing = kSS * kSlot;
   constexpr uint32_t kLower = 0x0401000Cu, kUpper = 0x0403020Cu;  // 0x3F, a bound pair's lower / upper code, 0
   constexpr float kMiss = 3.0e38f;  // beyond every entry distance a ray can have
-  const bool sgrid = !RAYS && a.sg.list != nullptr && a.sg.params->valid != 0u;
+  const bool sgrid = !RAYS && a.sg.list != nullptr && sun_grid_in_use(a.sg);
   __shared__ int32_t stk[kSS * kTB];
   // per lane, what only refills, hits and exact slabs touch (registers set the occupancy):
   // the best hit's barycentrics and the reciprocal direction
   __shared__ float cold[5][kTB];
-  if (RAYS && a.skip_if_set && *a.skip_if_set != 0u) return;  // a sun grid answered these rays
+  if (RAYS && sun_grid_answered(a.skip)) return;  // a sun grid answered these rays
   if (!RAYS) clock_begin(a.clk, kTraceRays);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1171,8 +1171,7 @@ template <bool COUNT>
 __global__ __launch_bounds__(kShadowTB) void k_probe_shadow_grid(TraceArgs a)
 {
   clock_begin(a.clk, kTraceShadow);
-  const SunGridParams* gq = a.sg.params;
-  if (gq->valid == 0u) return;  // no grid in use: the traversal ran the shadow rays
+  if (!sun_grid_in_use(a.sg)) return;  // no grid in use: the traversal ran the shadow rays
   probe_shadow_group<COUNT>(a, (int64_t)blockIdx.x * kShadowTB);
 }
 
@@ -1813,13 +1812,13 @@ int64_t pixel_slot_count(int W, int H) { return pixel_slots(W, H).n; }
 // clear: [nclear] words the traversal that follows counts in
 __global__ __launch_bounds__(256) void k_shadow_rays(const float* depth, int W, int H, Mat4 ivp, f3 dir,
                                                      float* orig, float* dirs, uint32_t* clear, int nclear,
-                                                     const uint32_t* skip_if_set)
+                                                     SunGridSkip skip)
 {
   if (blockIdx.x == 0)
     for (int k = threadIdx.x; k < nclear; k += blockDim.x) clear[k] = 0u;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (int64_t)W * H) return;
-  if (skip_if_set && *skip_if_set != 0u) return;
+  if (sun_grid_answered(skip)) return;
   const float d = depth[i];
   const f3 p = pixel_world_pos(i, W, H, d, ivp);
   orig[3 * i + 0] = p.x;
@@ -1833,11 +1832,11 @@ __global__ __launch_bounds__(256) void k_shadow_rays(const float* depth, int W, 
 }
 
 __global__ __launch_bounds__(256) void k_shadow_resolve(const float* depth, const ane_hit* hits, int64_t n,
-                                                        float* vis, const uint32_t* skip_if_set)
+                                                        float* vis, SunGridSkip skip)
 {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  if (skip_if_set && *skip_if_set != 0u) return;
+  if (sun_grid_answered(skip)) return;
   vis[i] = (depth[i] == 1.0f || hits[i].tri < 0) ? 1.0f : 0.0f;
 }
 
@@ -1952,7 +1951,7 @@ void launch_light_moments(const float* lights, int n, const uint32_t* order, con
 
 void launch_shadow_rays(const float* depth, int W, int H, const float* ivp16, const float* light3,
                         float* orig, float* dirs, uint32_t* clear, int nclear, hipStream_t s,
-                        const uint32_t* skip_if_set)
+                        const SunGridSkip& skip)
 {
   Mat4 m;
   for (int k = 0; k < 16; ++k) m.m[k] = ivp16[k];
@@ -1960,29 +1959,29 @@ void launch_shadow_rays(const float* depth, int W, int H, const float* ivp16, co
   const int64_t n = (int64_t)W * H;
   if (n <= 0) return;
   hipLaunchKernelGGL(k_shadow_rays, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, depth, W, H, m, dir,
-                     orig, dirs, clear, nclear, skip_if_set);
+                     orig, dirs, clear, nclear, skip);
 }
 
 void launch_shadow_resolve(const float* depth, const ane_hit* hits, int64_t n, float* vis, hipStream_t s,
-                           const uint32_t* skip_if_set)
+                           const SunGridSkip& skip)
 {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_shadow_resolve, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, depth, hits, n, vis,
-                     skip_if_set);
+                     skip);
 }
 
 // RT hard shadows through a sun grid built for the rays' direction: a thread per
 // pixel sets up its ray (the world position and ray setup of k_shadow_rays and the
 // trace) and looks up its cell; the candidates of a wave's 64 pixels are then
 // spread over its lanes (grid_wave_events), each in the watertight test: any hit
-// is the any-hit answer of the traversal.  Nothing unless the grid is valid.
+// is the any-hit answer of the traversal.  Nothing unless the grid is in use.
 __global__ __launch_bounds__(256) void k_shadow_mask_grid(const float* depth, int W, int H, Mat4 ivp, f3 dir,
                                                           SunGridK sg, SceneK sc, float* vis)
 {
   __shared__ uint32_t key[256];
   __shared__ SunQueue queue[4];
   const SunGridParams g = *sg.params;
-  if (!g.valid) return;
+  if (g.valid != sg.id) return;
   const int tid = threadIdx.x;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + tid;
   const bool in = i < (int64_t)W * H;
@@ -2052,11 +2051,11 @@ __global__ __launch_bounds__(256) void k_mirror_rays(const float* depth, const f
 
 // the shadow ray of every reflection hit (mirror_reflections.rchit:44-66), for the traversal
 __global__ __launch_bounds__(256) void k_mirror_shadow_rays(SceneK sc, const ane_hit* hits, int64_t n, f3 sun,
-                                                            float* orig, float* dirs, const uint32_t* skip_if_set)
+                                                            float* orig, float* dirs, SunGridSkip skip)
 {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  if (skip_if_set && *skip_if_set != 0u) return;
+  if (sun_grid_answered(skip)) return;
   const ane_hit h = hits[i];
   f3 p = mk(0.0f, 0.0f, 0.0f), d = mk(0.0f, 0.0f, 0.0f);
   if (h.tri >= 0) {
@@ -2075,14 +2074,14 @@ __global__ __launch_bounds__(256) void k_mirror_shadow_rays(SceneK sc, const ane
 // The same shadow rays through the sun grid, straight from the hits: the candidates of a
 // wave's 64 rays spread over its lanes, as for the probe shadow rays (one thread walking
 // its ray's list from staged rays: 95 + 15 us at 1080p, this kernel 47 us).  Writes
-// shadow_hits[i].tri, 0 (shadowed) or -1; nothing unless the grid is valid.
+// shadow_hits[i].tri, 0 (shadowed) or -1; nothing unless the grid is in use.
 __global__ __launch_bounds__(256) void k_mirror_shadow_grid(SceneK sc, const ane_hit* hits, int64_t n, f3 sun,
                                                             SunGridK sg, float tmin, float tmax, ane_hit* shadow_hits)
 {
   __shared__ uint32_t key[256];
   __shared__ SunQueue queue[4];
   const SunGridParams g = *sg.params;
-  if (!g.valid) return;
+  if (g.valid != sg.id) return;
   const int tid = threadIdx.x;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + tid;
   ane_hit h;
@@ -2143,11 +2142,11 @@ void launch_mirror_rays(const float* depth, const float* normal4, int W, int H, 
 }
 
 void launch_mirror_shadow_rays(const SceneK& sc, const ane_hit* hits, int64_t n, const float* sun3, float* orig,
-                               float* dirs, hipStream_t s, const uint32_t* skip_if_set)
+                               float* dirs, hipStream_t s, const SunGridSkip& skip)
 {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_mirror_shadow_rays, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, sc, hits, n,
-                     mk(sun3[0], sun3[1], sun3[2]), orig, dirs, skip_if_set);
+                     mk(sun3[0], sun3[1], sun3[2]), orig, dirs, skip);
 }
 
 void launch_mirror_shadow_grid(const SceneK& sc, const ane_hit* hits, int64_t n, const float* sun3,
