@@ -295,6 +295,11 @@ struct SunGridCache {
     pending = true;
     return ANE_OK;
   }
+  // judges the current build, whose launches were queued on st
+  int judge(hipStream_t st)
+  {
+    return built.set && !captured && !replayable && !(known == built) ? read_back(built, st) : ANE_OK;
+  }
   // device buffers for a scene of ntri triangles: about ANE_SUNGRID_DENSITY cells
   // per triangle (at most 4096 x 4096), ANE_SUNGRID_CAPACITY entries per triangle
   int alloc(int32_t ntri)
@@ -352,15 +357,18 @@ struct SunGridCache {
     const bool current = built == k;
     if (current && (capturing || !captured)) {
       *use = true;
-      if (!capturing && !replayable && !(known == k)) ANE_TRY(read_back(k, st));
+      if (!capturing) ANE_TRY(judge(st));
       if (valid) *valid = capturing ? -1 : known_valid();  // a graph keeps both ways: the grid may change before a replay
       return ANE_OK;
     }
     // a new direction over the scene version of a build that was found in use, or of the
-    // last request while no build of that version was found out of use
+    // last request while no build of that version was found out of use (not while a caller
+    // captures: a graph's builds are never judged, so that nothing would ever end them,
+    // and the buffers may not be there yet)
     const bool judged = known.set && known.scene == scene && known.version == version;
     const bool valid_scene = judged && last_valid == 1;
-    const bool moving = valid_scene || (!judged && seen.set && seen.scene == scene && seen.version == version);
+    const bool moving =
+        valid_scene || (!judged && !callers && seen.set && seen.scene == scene && seen.version == version);
     const bool eager = (valid_scene && rays >= (int64_t)ANE_SUNGRID_EAGER_RAYS * ntri) ||
                        (moving && sun_grid_pays(rays, ntri));
     if (!ANE_SUNGRID_EAGER && !eager && !current && !(seen == k)) {
@@ -379,7 +387,7 @@ struct SunGridCache {
     ++builds;
     captured = callers;
     replayable = replayable || callers;
-    if (!capturing && !replayable) ANE_TRY(read_back(k, st));
+    if (!capturing) ANE_TRY(judge(st));
     *use = true;
     return ANE_OK;
   }
@@ -1428,6 +1436,7 @@ int ddgi_update_graph(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame*
   ANE_TRY(ensure_spill(c, s->depth));
   if (sun_grid_wanted(c)) ANE_TRY(c->sgc.alloc(s->ntri));  // allocation outside the capture
   if (c->counting) return ane_ddgi_update(c, s, f, st);
+  c->sgc.poll();  // not possible under the capture
   hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) {
     return fail(ANE_ERR_DEVICE, "hipStreamBeginCapture: %s", hipGetErrorString(e));
@@ -1459,7 +1468,7 @@ int ddgi_update_graph(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame*
     if (c->sgc.builds != builds) c->sgc.built = SunGridCache::Key{};
     return fail(ANE_ERR_DEVICE, "graph launch: %s", hipGetErrorString(e));
   }
-  return ANE_OK;
+  return c->sgc.judge(st);
 }
 }  // namespace ane
 
