@@ -1960,27 +1960,8 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
   for (int k = 0; k < 3; ++k)
     if (!std::isfinite(light3[k])) return fail(ANE_ERR_INVALID_ARG, "non-finite light direction");
   hipStream_t st = S(stream);
-  // without counters the rays go through the scene's grid along -light_dir once it is
-  // current; while its validity is not known here, the traversal launches follow and do
-  // nothing when it is (device flag)
-  SunGridSkip skip{};
-  s->sh_traced = true;
-  if (!counters2) {
-    const float dir[3] = {-light3[0], -light3[1], -light3[2]};
-    bool use = false;
-    int valid = -1;
-    ANE_TRY(s->sgc.update(s->view, s->ntri, s, s->version, dir, (int64_t)width * height, st, &use, ClockArg{}, 0,
-                          &valid));
-    if (use && valid != 0) {
-      launch_shadow_mask_grid(depth, width, height, ivp16, light3, s->sgc.view(), s->view, out_vis, st);
-      if (valid == 1) {
-        s->sh_traced = false;
-        ANE_CHECK_HIP(hipGetLastError());
-        return ANE_OK;
-      }
-      skip = s->sgc.skip();
-    }
-  }
+  // the traversal's workspace, sized also by a pass that the grid answers alone: the same
+  // pass under capture queues both, and cannot allocate there
   if (n > s->shadow_px) {
     ANE_CHECK_HIP(hipStreamSynchronize(st));
     dfree(s->d_sh_orig); dfree(s->d_sh_dir); dfree(s->d_sh_hits);
@@ -2003,6 +1984,27 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
     s->sh_spill_words = 0;
     ANE_TRY(dalloc(&s->d_sh_spill, sd * lanes, nullptr));
     s->sh_spill_words = sd * lanes;
+  }
+  // without counters the rays go through the scene's grid along -light_dir once it is
+  // current; while its validity is not known here, the traversal launches follow and do
+  // nothing when it is (device flag)
+  SunGridSkip skip{};
+  s->sh_traced = true;
+  if (!counters2) {
+    const float dir[3] = {-light3[0], -light3[1], -light3[2]};
+    bool use = false;
+    int valid = -1;
+    ANE_TRY(s->sgc.update(s->view, s->ntri, s, s->version, dir, (int64_t)width * height, st, &use, ClockArg{}, 0,
+                          &valid));
+    if (use && valid != 0) {
+      launch_shadow_mask_grid(depth, width, height, ivp16, light3, s->sgc.view(), s->view, out_vis, st);
+      if (valid == 1) {
+        s->sh_traced = false;
+        ANE_CHECK_HIP(hipGetLastError());
+        return ANE_OK;
+      }
+      skip = s->sgc.skip();
+    }
   }
   launch_shadow_rays(depth, width, height, ivp16, light3, s->d_sh_orig, s->d_sh_dir, s->d_sh_work, kShWords, st, skip);
   TraceArgs a{};

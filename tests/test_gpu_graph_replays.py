@@ -135,3 +135,22 @@ def test_direct_calls_after_a_replayed_build(kind, other):
         assert np.array_equal(p.image(first.launch), want_other)
     for g in (first, second, third):
         g.close()
+
+
+@pytest.mark.parametrize("kind", ["mask", "mirror"])
+def test_a_pass_of_a_warm_size_is_captured(kind):
+    """The grid alone answers the direct calls of the larger size; its capture queues the
+    traversal too, in the workspace that those calls prepared."""
+    ds = native.DeviceScene(strip_scene())
+    small, large = Passes(kind, ds, 32, 24), Passes(kind, ds, 200, 130)
+    large.grid = small.grid
+    for _ in range(4):
+        small.direct(DOWN)
+    want = large.traversed(DOWN)
+    for _ in range(2):
+        assert np.array_equal(large.direct(DOWN), want)
+    g = Graph(lambda st: large.call(DOWN, st))
+    for _ in range(3):
+        assert np.array_equal(large.image(g.launch), want)
+        assert np.array_equal(large.direct(DOWN), want)
+    g.close()
