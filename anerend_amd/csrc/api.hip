@@ -476,7 +476,6 @@ struct ane_scene {
   uint32_t* d_sh_work = nullptr;             // claim counters, then (in the same buffer):
   unsigned long long* d_sh_stats = nullptr;  // [2] work counters
   uint32_t* d_sh_ov = nullptr;               // fault flag
-  bool sh_traced = false;                    // the last pass launched a traversal (d_sh_ov is its)
   int32_t* d_sh_spill = nullptr;
   int64_t sh_spill_words = 0;
   // point-light shadow workspace (grows to the most lights seen); the sum's
@@ -1973,7 +1972,10 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
   }
   // claim counters, 2 work counters (64-bit), the fault flag
   constexpr int kShWords = kTraceWorkWords + 5;
-  if (!s->d_sh_work) ANE_TRY(dalloc(&s->d_sh_work, kShWords, nullptr));
+  if (!s->d_sh_work) {
+    ANE_TRY(dalloc(&s->d_sh_work, kShWords, nullptr));
+    ANE_CHECK_HIP(hipMemset(s->d_sh_work, 0, kShWords * sizeof(uint32_t)));
+  }
   s->d_sh_stats = reinterpret_cast<unsigned long long*>(s->d_sh_work + kTraceWorkWords);
   s->d_sh_ov = s->d_sh_work + kTraceWorkWords + 4;
   const int64_t lanes = trace_lanes_per_launch();
@@ -1989,7 +1991,6 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
   // current; while its validity is not known here, the traversal launches follow and do
   // nothing when it is (device flag)
   SunGridSkip skip{};
-  s->sh_traced = true;
   if (!counters2) {
     const float dir[3] = {-light3[0], -light3[1], -light3[2]};
     bool use = false;
@@ -1997,9 +1998,8 @@ extern "C" int ane_scene_shadow_mask(ane_scene* s, const float* depth, int32_t w
     ANE_TRY(s->sgc.update(s->view, s->ntri, s, s->version, dir, (int64_t)width * height, st, &use, ClockArg{}, 0,
                           &valid));
     if (use && valid != 0) {
-      launch_shadow_mask_grid(depth, width, height, ivp16, light3, s->sgc.view(), s->view, out_vis, st);
+      launch_shadow_mask_grid(depth, width, height, ivp16, light3, s->sgc.view(), s->view, out_vis, s->d_sh_ov, st);
       if (valid == 1) {
-        s->sh_traced = false;
         ANE_CHECK_HIP(hipGetLastError());
         return ANE_OK;
       }
@@ -2043,7 +2043,7 @@ extern "C" int ane_scene_check(ane_scene* s, void* stream)
   if (!s) return fail(ANE_ERR_INVALID_ARG, "NULL scene");
   uint32_t v[2] = {0, 0};
   ANE_CHECK_HIP(hipStreamSynchronize(S(stream)));
-  if (s->d_sh_ov && s->sh_traced) ANE_CHECK_HIP(hipMemcpy(&v[0], s->d_sh_ov, 4, hipMemcpyDeviceToHost));
+  if (s->d_sh_ov) ANE_CHECK_HIP(hipMemcpy(&v[0], s->d_sh_ov, 4, hipMemcpyDeviceToHost));
   if (s->d_lt_ov) ANE_CHECK_HIP(hipMemcpy(&v[1], s->d_lt_ov, 4, hipMemcpyDeviceToHost));
   if (s->d_sh_ov) ANE_CHECK_HIP(hipMemset(s->d_sh_ov, 0, 4));
   if (s->d_lt_ov) ANE_CHECK_HIP(hipMemset(s->d_lt_ov, 0, 4));

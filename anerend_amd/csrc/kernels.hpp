@@ -193,9 +193,10 @@ void sun_grid_setup(SunGridParams& g, const float* dir3, int gx, int gy);
 // slots of the tile order of a W x H image (at least its pixels)
 int64_t pixel_slot_count(int W, int H);
 // the shadow mask through the grid of its rays' direction (zero or non-finite
-// direction: no ray); does nothing unless the grid is in use
+// direction: no ray), which has no fault: *fault is cleared.  Does nothing unless the grid
+// is in use.
 void launch_shadow_mask_grid(const float* depth, int W, int H, const float* ivp16, const float* light3,
-                             const SunGridK& sg, const SceneK& sc, float* vis, hipStream_t s);
+                             const SunGridK& sg, const SceneK& sc, float* vis, uint32_t* fault, hipStream_t s);
 // est: [sun_grid_scratch_words(ntri)] build scratch (partial sums of the candidate
 // estimate, per-block cell counts)
 int64_t sun_grid_scratch_words(int32_t ntri);

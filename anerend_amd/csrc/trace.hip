@@ -1976,7 +1976,7 @@ void launch_shadow_resolve(const float* depth, const ane_hit* hits, int64_t n, f
 // spread over its lanes (grid_wave_events), each in the watertight test: any hit
 // is the any-hit answer of the traversal.  Nothing unless the grid is in use.
 __global__ __launch_bounds__(256) void k_shadow_mask_grid(const float* depth, int W, int H, Mat4 ivp, f3 dir,
-                                                          SunGridK sg, SceneK sc, float* vis)
+                                                          SunGridK sg, SceneK sc, float* vis, uint32_t* fault)
 {
   __shared__ uint32_t key[256];
   __shared__ SunQueue queue[4];
@@ -1984,6 +1984,7 @@ __global__ __launch_bounds__(256) void k_shadow_mask_grid(const float* depth, in
   if (g.valid != sg.id) return;
   const int tid = threadIdx.x;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + tid;
+  if (i == 0) *fault = 0u;
   const bool in = i < (int64_t)W * H;
   const bool dir_ok = !(dir.x == 0.0f && dir.y == 0.0f && dir.z == 0.0f) && __builtin_isfinite(dir.x) &&
                       __builtin_isfinite(dir.y) && __builtin_isfinite(dir.z);
@@ -2004,7 +2005,7 @@ __global__ __launch_bounds__(256) void k_shadow_mask_grid(const float* depth, in
 }
 
 void launch_shadow_mask_grid(const float* depth, int W, int H, const float* ivp16, const float* light3,
-                             const SunGridK& sg, const SceneK& sc, float* vis, hipStream_t s)
+                             const SunGridK& sg, const SceneK& sc, float* vis, uint32_t* fault, hipStream_t s)
 {
   Mat4 m;
   for (int k = 0; k < 16; ++k) m.m[k] = ivp16[k];
@@ -2012,7 +2013,7 @@ void launch_shadow_mask_grid(const float* depth, int W, int H, const float* ivp1
   const int64_t n = (int64_t)W * H;
   if (n <= 0) return;
   hipLaunchKernelGGL(k_shadow_mask_grid, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, depth, W, H, m, dir,
-                     sg, sc, vis);
+                     sg, sc, vis, fault);
 }
 
 // ---------------------------------------------------------------------------
