@@ -72,7 +72,9 @@ namespace ane {
 #define ANE_TRACE_SPEC 0  // 1: probe rays keep visiting internal nodes while a leaf waits
 #endif
 static constexpr int kTB = ANE_TRACE_BLOCK;      // threads per traversal block
-static constexpr int kSS = ANE_TRACE_STACK;      // LDS stack entries per lane (ring, any size)
+static constexpr int kSS = ANE_TRACE_STACK;      // LDS stack entries per lane (ring)
+// k_trace_closest wraps its ring of the block's entries by a mask
+static_assert((kSS & (kSS - 1)) == 0 && (kTB & (kTB - 1)) == 0, "the stack ring and the block are powers of two");
 // Rays a wave takes at a time: one per lane.  A claim is a device-scope atomic, and one
 // address takes about 80 of them per microsecond from the 8 XCDs: with a single counter
 // for all waves and 64-ray chunks the 8.4M probe rays of an update waited on their claims
