@@ -211,6 +211,7 @@ bool trace_grid_supported();
 static constexpr int kTraceCounters = 16;
 static constexpr int kTraceCounterStride = 32;
 static constexpr int kTraceWorkWords = kTraceCounters * kTraceCounterStride;
+static_assert((kTraceCounters & (kTraceCounters - 1)) == 0, "claims wrap by a mask");
 
 struct TraceArgs {
   SceneK sc;
@@ -225,8 +226,7 @@ struct TraceArgs {
   ane_hit* hits;          // out: closest hit per ray
   uint8_t* shadow;        // out (probe rays): 0 lit, 1 shadowed, 255 miss
   uint32_t* work;         // [kTraceWorkWords] claim counters (zeroed before launch)
-  uint32_t ncounters;
-  uint32_t chunk;         // rays a wave takes at a time (set by launch_trace)
+  uint32_t ncounters;     // counters in use, a power of two (set by launch_trace)
   uint32_t static_rays;   // rays of the waves' first chunks, which need no claim (set by launch_trace)
   unsigned long long* stats; // counting kernels: nodes, triangles [, shadow nodes, shadow triangles]
   uint32_t* overflow;     // set to 1 when a ray ends without a result: a stack would exceed the

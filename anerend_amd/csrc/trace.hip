@@ -307,13 +307,15 @@ __device__ __forceinline__ f3 hit_geom_pos(const SceneK& sc, int32_t id, float u
 }
 
 // The next chunk of a wave (lanes `im` wait for rays): claim i of counter k is chunk
-// (k + i) % K of the i-th group of K chunks; nrays when every ray was in a first chunk or
-// claimed (in 32 bits: a wave makes one claim past the end).  cend: the chunk's end.
+// (k + i) % K of the i-th group of K chunks, K = a.ncounters; nrays when every ray was in a
+// first chunk or claimed.  Past the end each group of idle lanes claims once more, at most
+// 64 / kRefill + 1 times a wave, so that the sum stays in 32 bits: rays under 2^31 and
+// 5 chunks for each of some thousand waves.  cend: the chunk's end.
 __device__ __forceinline__ uint32_t claim_chunk(const TraceArgs& a, uint32_t nrays, uint64_t im, int lane, uint32_t& cend)
 {
   uint32_t base = nrays;
   if (a.static_rays < nrays) {
-    constexpr uint32_t K = (uint32_t)kTraceCounters;
+    const uint32_t K = a.ncounters;
     const uint32_t k = blockIdx.x & (K - 1u);
     const int who = __ffsll((unsigned long long)im) - 1;
     uint32_t i = 0u;
@@ -1204,6 +1206,9 @@ void launch_trace(const TraceArgs& a, bool any_hit, bool rays, bool count, hipSt
   TraceArgs b = a;
   b.total_lanes = blocks * kTB;
   b.static_rays = (uint32_t)(blocks * (kTB / 64)) * kChunk;
+  // a counter's chunks are claimed by its blocks alone: each has one
+  b.ncounters = (uint32_t)kTraceCounters;
+  while (b.ncounters > (uint32_t)blocks) b.ncounters >>= 1;
 #define ANE_TR(S, R, C)                                                                             \
   do {                                                                                              \
     if (b.sc.qnodes) hipLaunchKernelGGL((k_trace<S, R, C, true>), dim3(blocks), dim3(kTB), 0, s, b);  \
