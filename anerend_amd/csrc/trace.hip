@@ -889,7 +889,10 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
           tbest = tmax0;
           if (RAYS && a.ray_tmax) tbest = a.ray_tmax[gidx];
           start(r);
-          if (none) node = kDone;
+          if (none) {  // its reciprocals would send the wave to the exact slabs
+            node = kDone;
+            exact = false;
+          }
         }
       }
       cbeg += need < avail ? need : avail;
