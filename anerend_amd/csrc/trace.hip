@@ -705,6 +705,8 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
   constexpr uint32_t kSlot = kTB * 4;    // bytes of one stack level of the block
   constexpr uint32_t kRing = kSS * kSlot;
   constexpr uint32_t kLower = 0x0401000Cu, kUpper = 0x0403020Cu;  // 0x3F, a bound pair's lower / upper code, 0
+  constexpr int32_t kWaits = 16;
+  constexpr int32_t kSteps = 7;    // traversal steps between checks, if none ends them early
   constexpr float kMiss = 3.0e38f;  // beyond every entry distance a ray can have
   const bool sgrid = !RAYS && a.sg.list != nullptr && sun_grid_in_use(a.sg);
   __shared__ int32_t stk[kSS * kTB];
@@ -722,9 +724,12 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
   const uint32_t nrays = (uint32_t)a.nrays;
   const int32_t root = (sc.ntri >= 2) ? 0 : (sc.ntri == 1 ? ~0 : kDone);
   const uint32_t lim = sc.ntri >= 2 ? (uint32_t)sc.ntri - 1u : 0u;  // internal nodes
-  // refill checks a ray may live through: far above the visits of any valid hierarchy and
-  // the waits of its lane, so only a malformed one ends a ray here
-  const uint32_t patience = 2u * (uint32_t)sc.ntri + (1u << 22);
+  // visits a ray may make, k_trace's: a valid hierarchy has 2 ntri - 1 nodes and leaves, so
+  // only a malformed one ends a ray here.  Counted at the checks, from below and for the whole
+  // wave: kSteps while leaves are tested at once, so that every step takes every live lane
+  // further; else one, and none if no leaf batch has run since the last check, as a lane may
+  // have waited for it (kWaits checks in turn; then leaves are tested at once up to the next).
+  const int32_t budget = 2 * sc.ntri + 8;
   const char* const nbase = reinterpret_cast<const char*>(sc.hnodes);
   const char* const tbase = reinterpret_cast<const char*>(sc.tris);
   // the frame, in scalar registers (it is the same for every lane)
@@ -755,7 +760,8 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
   int32_t bid = -1, node = kDone;
   const uint32_t sp0 = (uint32_t)tid * 4u;
   uint32_t sp = sp0;  // byte offset of the next stack entry, the ring's wrap not yet taken
-  uint32_t left_checks = 0u;
+  int32_t visits_left = 0;
+  int32_t unbatched = 0;  // wave-uniform: checks in turn without a leaf batch before them
 
   auto entry = [&](uint32_t p) -> int32_t& {
     return *reinterpret_cast<int32_t*>(reinterpret_cast<char*>(stk) + (p & (kRing - 1u)));
@@ -790,7 +796,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
     node = root;
     entry(sp0) = kDone;  // the bottom of the stack ends the traversal
     sp = sp0 + kSlot;
-    left_checks = patience;
+    visits_left = budget;
   };
   auto pop = [&]() {
     sp -= kSlot;
@@ -821,12 +827,15 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
   };
 
   for (;;) {
+    const int32_t pay = dry ? kSteps : (RAYS || unbatched < 0 || unbatched >= kWaits ? 1 : 0);
+    ++unbatched;
     // ---- finish ended traversals; a probe ray that hit continues as its shadow ray ----
     if (out >= 0) {
       // a child index out of range or a ray without end (a malformed hierarchy) is a fault
       const bool bad = node >= 0 ? ((uint32_t)node >= lim && node != kDone) : (uint32_t)~node >= (uint32_t)sc.ntri;
-      if (bad || --left_checks == 0u) {
-        *a.overflow = 1u;
+      visits_left -= pay;
+      if (bad || visits_left < 0) {
+        if (node != kDone) *a.overflow = 1u;
         node = kDone;
       }
       if (node == kDone) {
@@ -902,8 +911,8 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
       continue;
     }
     const bool slow = !grid || __ballot(exact && out >= 0) != 0ull;  // wave-uniform
-    const int leaf_batch = RAYS || dry ? 1 : ANE_CLOSEST_LEAFBATCH;
-    // ---- traversal steps ----
+    const int leaf_batch = RAYS || dry || unbatched >= kWaits ? 1 : ANE_CLOSEST_LEAFBATCH;
+    // ---- traversal steps (kSteps) ----
     // (a chain of calls, for a loop with the early way out is not unrolled: 1.089 ms)
     auto step = [&](bool goes_on) __attribute__((always_inline)) -> bool {
       if ((uint32_t)node < lim) {
@@ -943,6 +952,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(ANE_CLOSEST
       const uint64_t lm = __ballot(node < 0);
       if (lm != 0ull) {
         if (__popcll(lm) >= leaf_batch || __ballot((uint32_t)node < lim) == 0ull) {
+          unbatched = -1;
           if (node < 0 && (uint32_t)~node < (uint32_t)sc.ntri) {
             const float4* tv = reinterpret_cast<const float4*>(tbase + (uint32_t)~node * 48u);
             const float4 v0 = tv[0], v1 = tv[1], v2 = tv[2];
