@@ -1023,6 +1023,15 @@ __device__ __forceinline__ void sun_lookup(const SunGridK& sg, const SunGridPara
   q = sun_local(X, g.x0, g.icw, cx) | sun_local(Y, g.y0, g.ich, cy) << 8;
 }
 
+// Between a wave's stores to the LDS and other lanes' loads of them: the LDS takes a wave's
+// accesses in order, and this keeps the compiler from moving them.  No instruction.
+__device__ __forceinline__ void wave_lds_order()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A wave's queue of candidates that passed the bounds check (LDS)
 struct SunQueue {
   uint32_t id[64 * (kShadowU + 1)], pos[64 * (kShadowU + 1)];
@@ -1059,8 +1068,10 @@ __device__ __forceinline__ void grid_wave_events(const SunGridK& sg, const float
   const uint32_t excl = incl - c;
   constexpr int U = kShadowU;
   uint32_t waiting = 0u;  // wave-uniform: queue entries
+  wave_lds_order();  // the lanes' keys
   // the last (at most 64) entries of the queue
   auto drain = [&]() {
+    wave_lds_order();
     const uint32_t m = waiting < 64u ? waiting : 64u;
     waiting -= m;
     const uint32_t k = waiting + ((uint32_t)lane < m ? (uint32_t)lane : 0u);
@@ -1073,6 +1084,7 @@ __device__ __forceinline__ void grid_wave_events(const SunGridK& sg, const float
       if (tri_test(r, mk(v0.x, v0.y, v0.z), mk(v1.x, v1.y, v1.z), mk(v2.x, v2.y, v2.z), tmin, tmax, tt, uu, vv))
         atomicMin(&key[j], 2u * pos);
     }
+    wave_lds_order();  // read before the next entries are queued
   };
   for (uint32_t t0 = 0; t0 < total; t0 += 64u * U) {
     uint32_t pos[U], qj[U];
@@ -1121,6 +1133,7 @@ __device__ __forceinline__ void grid_wave_events(const SunGridK& sg, const float
     while (waiting >= 64u) drain();
   }
   if (waiting) drain();
+  wave_lds_order();
 }
 
 #ifndef ANE_SHADOW_TB
