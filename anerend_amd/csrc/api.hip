@@ -663,7 +663,7 @@ static int scene_refit_dev(ane_scene* s, hipStream_t st)
   ANE_TRY(scene_fit_qnodes(s, &qn));
   launch_fit(s->d_tris, n, s->d_nodes, s->d_node_box, qn, s->d_topo, s->d_leaf_parent, s->d_units, s->nunits,
              s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, &view, s->d_ids, nullptr, st);
-  launch_grid_nodes(s->d_nodes, n, s->d_hframe, s->d_hnodes, st);
+  if (s->view.hnodes) launch_grid_nodes(s->d_nodes, n, s->d_hframe, s->d_hnodes, st);  // else none reads them
   s->world_stale = true;
   ANE_TRY(scene_apply_node_format(s, st, qn != nullptr));
   ANE_CHECK_HIP(hipGetLastError());
