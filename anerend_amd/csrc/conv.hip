@@ -16,7 +16,7 @@
 //                  wave streams its 16 probes over all rays
 //   k_conv_mfma    16 probes per block, 4 waves splitting the rays: up to 8,192 probes
 //                  (up to 2,048 with the row tiles split over blocks), and weights too
-//                  large for LDS (FP32 beyond 608 rays, 16-bit beyond 1216)
+//                  large for LDS (FP32 beyond 608 rays, 16-bit beyond 1248)
 //   k_conv_jobs    the same blocks over the updates of a serving batch
 //   k_conv_fp32    FP32 register-tiled kernel for ray counts that are not a
 //                  multiple of 32
@@ -601,6 +601,10 @@ static size_t conv_stream_lds(int precision, int rays)
 // quarter of it: with few blocks per CU the chain is the launch.  FP32, 512 rays, split-ray
 // against streaming: 1,024 probes 12.5 / 32.9 us, 4,096 14.1 / 33.5, 8,192 25.7 / 33.5,
 // 16,384 47.7 / 37.1; 16-bit 6.2 / 10.3, 6.4 / 10.7, 10.7 / 12.1, 18.4 / 16.4 us.
+// An update's own probes decide in a batch of the request loop too, so that it runs the kernel
+// that its own launch would; the split rays are also the faster ones there, beside the other
+// batches' traversals: 416 updates of 2,048 probes in FP32 3.4 against 4.5 ms in all, of 8,192
+// (104) 3.2 against 5.6; in 16 bits 1.6 against 1.9 and 1.8 against 2.4.
 static constexpr int kStreamMinProbes = 8192;
 bool conv_stream_fits(int precision, int rays, int num_probes)
 {
