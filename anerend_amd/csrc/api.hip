@@ -421,11 +421,8 @@ struct ane_scene {
   uint32_t* d_tri_inst = nullptr;
   float4* d_tri_rec = nullptr;
   uint32_t* d_inst_off = nullptr;
-  float* d_world = nullptr;
   uint64_t* d_keys = nullptr;
-  uint64_t* d_keys2 = nullptr;
   uint32_t* d_ids = nullptr;
-  uint32_t* d_ids2 = nullptr;
   NodeBuild* d_nodes = nullptr;
   int32_t* d_leaf_parent = nullptr;
   float4* d_tris = nullptr;
@@ -433,7 +430,15 @@ struct ane_scene {
   uint32_t* d_cbounds = nullptr;
   uint32_t* d_cpart = nullptr;  // per-block centroid-bound partials of a build
   uint4* d_qnodes = nullptr;    // quantized traversal nodes (allocated when first used)
-  uint4* d_hnodes = nullptr;    // grid nodes (closest-hit traversal)
+  // grid nodes (closest-hit traversal).  Until a build writes them, as the last of what a ray
+  // reads, its own buffers lie there: the input-order triangles [ntri][9] and the sort's other
+  // buffers, then the plan's scans and the top nodes by index
+  uint4* d_hnodes = nullptr;
+  float* d_world = nullptr;
+  uint64_t* d_keys2 = nullptr;
+  uint32_t* d_ids2 = nullptr;
+  uint32_t* d_uscratch = nullptr;
+  int32_t* d_top = nullptr;
   GridFrame* d_hframe = nullptr;
   int32_t node_format = ANE_NODES_AUTO;
   uint32_t* d_scratch = nullptr;
@@ -443,18 +448,15 @@ struct ane_scene {
   int32_t* d_cross = nullptr;   // top nodes (more leaves than a fit treelet holds), by depth
   int2* d_cross_kids = nullptr; // their children, in the same order (cross_kids_cap entries)
   int64_t cross_kids_cap = 0;
-  int32_t* d_top = nullptr;     // top nodes, by index
   uint8_t* d_ndepth = nullptr;  // depth of the top nodes
   int2* d_units = nullptr;      // leaf ranges of the fit treelets
   int32_t* d_unit_root = nullptr;
   uint8_t* d_uheight = nullptr; // height of each treelet's root
   int32_t* d_stray = nullptr;   // leaves directly under a top node
-  uint32_t* d_uscratch = nullptr;
   int32_t nunits = 0, nstray = 0;
   std::vector<int32_t> cross_begin;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   int32_t depth = 0;
-  bool world_stale = false;  // d_world predates the last refit (rebuilt from d_tris on inspection)
   uint64_t version = 0;  // changes with every build or refit (keys derived data such as sun grids)
   mutable float build_ms = 0.0f;
   mutable bool build_ms_pending = false;  // refit timing not yet read back
@@ -502,11 +504,11 @@ static void scene_free(ane_scene* s)
 {
   dfree(s->d_vertices); dfree(s->d_indices); dfree(s->d_meshes); dfree(s->d_mats);
   dfree(s->d_inst); dfree(s->d_inv); dfree(s->d_tri_inst); dfree(s->d_tri_rec); dfree(s->d_inst_off);
-  dfree(s->d_world); dfree(s->d_keys); dfree(s->d_keys2); dfree(s->d_ids); dfree(s->d_ids2);
+  dfree(s->d_keys); dfree(s->d_ids);
   dfree(s->d_nodes); dfree(s->d_leaf_parent); dfree(s->d_tris);
   dfree(s->d_node_box); dfree(s->d_cbounds); dfree(s->d_cpart); dfree(s->d_qnodes); dfree(s->d_hnodes); dfree(s->d_hframe); dfree(s->d_scratch);
-  dfree(s->d_depth); dfree(s->d_topo); dfree(s->d_cross); dfree(s->d_cross_kids); dfree(s->d_top); dfree(s->d_ndepth); dfree(s->d_units);
-  dfree(s->d_unit_root); dfree(s->d_uheight); dfree(s->d_stray); dfree(s->d_uscratch);
+  dfree(s->d_depth); dfree(s->d_topo); dfree(s->d_cross); dfree(s->d_cross_kids); dfree(s->d_ndepth); dfree(s->d_units);
+  dfree(s->d_unit_root); dfree(s->d_uheight); dfree(s->d_stray);
   dfree(s->d_sh_orig); dfree(s->d_sh_dir); dfree(s->d_sh_hits); dfree(s->d_sh_work);
   dfree(s->d_sh_spill);
   dfree(s->d_lt_lights); dfree(s->d_lt_orig); dfree(s->d_lt_dir); dfree(s->d_lt_tmax); dfree(s->d_lt_hits);
@@ -612,8 +614,8 @@ static int scene_build(ane_scene* s, hipStream_t st, bool write_inst)
   s->version = ++g_scene_version;
   ANE_CHECK_HIP(hipEventRecord(s->ev0, st));
   const int n = s->ntri;
+  s->view.hnodes = nullptr;  // until they are written: the build's buffers lie there
   launch_flatten(s->view, s->d_world, s->d_tri_inst, s->d_tri_rec, s->d_cpart, s->d_cbounds, write_inst, st);
-  s->world_stale = false;
   launch_morton(s->d_world, n, s->d_cbounds, s->d_keys, s->d_ids, st);
   radix_sort_pairs(s->d_keys, s->d_ids, s->d_keys2, s->d_ids2, n, s->d_scratch, st);
   launch_karras(s->d_keys, n, s->d_nodes, s->d_leaf_parent, s->d_topo, st);
@@ -635,10 +637,11 @@ static int scene_build(ane_scene* s, hipStream_t st, bool write_inst)
   ANE_TRY(scene_fit_qnodes(s, &qn));
   launch_fit(s->d_tris, n, s->d_nodes, s->d_node_box, qn, s->d_topo, s->d_leaf_parent, s->d_units, s->nunits,
              s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, nullptr, nullptr, s->d_uheight, st);
-  launch_grid_nodes(s->d_nodes, n, s->d_hframe, s->d_hnodes, st);
-  ANE_TRY(scene_apply_node_format(s, st, qn != nullptr));
   launch_tree_depth(s->d_topo, n, s->d_unit_root, s->d_uheight, s->nunits, s->d_top, s->d_uscratch, s->d_ndepth,
-                    s->d_depth, s->d_hframe, &s->h_info->depth, &s->h_info->frame, st);
+                    s->d_depth, st);
+  launch_grid_nodes(s->d_nodes, n, s->d_hframe, s->d_hnodes, st);  // over the build's buffers
+  ANE_TRY(scene_apply_node_format(s, st, qn != nullptr));
+  launch_build_info(n, s->d_depth, s->d_hframe, &s->h_info->depth, &s->h_info->frame, st);
   ANE_CHECK_HIP(hipGetLastError());
   ANE_CHECK_HIP(hipEventRecord(s->ev1, st));
   ANE_CHECK_HIP(hipStreamSynchronize(st));
@@ -664,7 +667,6 @@ static int scene_refit_dev(ane_scene* s, hipStream_t st)
   launch_fit(s->d_tris, n, s->d_nodes, s->d_node_box, qn, s->d_topo, s->d_leaf_parent, s->d_units, s->nunits,
              s->d_stray, s->nstray, s->d_cross, s->d_cross_kids, s->cross_begin, &view, s->d_ids, nullptr, st);
   if (s->view.hnodes) launch_grid_nodes(s->d_nodes, n, s->d_hframe, s->d_hnodes, st);  // else none reads them
-  s->world_stale = true;
   ANE_TRY(scene_apply_node_format(s, st, qn != nullptr));
   ANE_CHECK_HIP(hipGetLastError());
   ANE_CHECK_HIP(hipEventRecord(s->ev1, st));
@@ -733,13 +735,15 @@ extern "C" int ane_scene_create(const float* vertices, int64_t num_vertices, con
   ANE_A(d_tri_inst, n);
   ANE_A(d_tri_rec, (int64_t)n * 4);
   ANE_A(d_inst_off, (int64_t)num_instances + 1);
-  ANE_A(d_world, n * 9);
   ANE_A(d_keys, n);
-  ANE_A(d_keys2, n);
   ANE_A(d_ids, n);
-  ANE_A(d_ids2, n);
   ANE_A(d_nodes, n > 1 ? n - 1 : 1);
-  ANE_A(d_hnodes, 4 * (n > 1 ? n - 1 : 1));
+  ANE_A(d_hnodes, std::max<int64_t>(4 * (n > 1 ? n - 1 : 1), 3 * n + 1));  // 48 n + 4 bytes of a build
+  s->d_world = reinterpret_cast<float*>(s->d_hnodes);
+  s->d_keys2 = reinterpret_cast<uint64_t*>(s->d_world + 9 * n + (n & 1));
+  s->d_ids2 = reinterpret_cast<uint32_t*>(s->d_keys2 + n);
+  s->d_uscratch = reinterpret_cast<uint32_t*>(s->d_hnodes);  // 3 n + 3 words
+  s->d_top = reinterpret_cast<int32_t*>(s->d_uscratch + 3 * n + 3);
   ANE_A(d_hframe, 1);
   ANE_A(d_leaf_parent, n);
   ANE_A(d_tris, n * 3);
@@ -750,13 +754,11 @@ extern "C" int ane_scene_create(const float* vertices, int64_t num_vertices, con
   ANE_A(d_depth, 1);
   ANE_A(d_topo, n > 1 ? n - 1 : 1);
   ANE_A(d_cross, n > 1 ? n - 1 : 1);
-  ANE_A(d_top, n > 1 ? n - 1 : 1);
   ANE_A(d_ndepth, n > 1 ? n - 1 : 1);
   ANE_A(d_units, n > 1 ? n - 1 : 1);
   ANE_A(d_unit_root, n > 1 ? n - 1 : 1);
   ANE_A(d_uheight, n > 1 ? n - 1 : 1);
   ANE_A(d_stray, n > 0 ? n : 1);
-  ANE_A(d_uscratch, 3 * n + 3);
 #undef ANE_A
   auto bail = [&](int code) { scene_free(s); delete s; return code; };
   hipError_t e = hipSuccess;
@@ -915,12 +917,14 @@ extern "C" int ane_scene_debug_world_tris(const ane_scene* s, float* tris9)
 {
   if (!s || !tris9) return fail(ANE_ERR_INVALID_ARG, "NULL argument");
   ANE_CHECK_HIP(hipDeviceSynchronize());
-  if (s->world_stale) {
-    launch_world_from_tris(s->d_tris, s->ntri, s->d_world, nullptr);
-    ANE_CHECK_HIP(hipGetLastError());
-    ANE_CHECK_HIP(hipDeviceSynchronize());
-  }
-  ANE_CHECK_HIP(hipMemcpy(tris9, s->d_world, sizeof(float) * 9 * (size_t)s->ntri, hipMemcpyDeviceToHost));
+  if (s->ntri == 0) return ANE_OK;
+  float* world = nullptr;
+  ANE_TRY(dalloc(&world, 9 * (int64_t)s->ntri, nullptr));
+  launch_world_from_tris(s->d_tris, s->ntri, world, nullptr);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipMemcpy(tris9, world, sizeof(float) * 9 * (size_t)s->ntri, hipMemcpyDeviceToHost);
+  dfree(world);
+  if (e != hipSuccess) return fail_hip(e, "world triangles", __FILE__, __LINE__);
   return ANE_OK;
 }
 

@@ -1220,11 +1220,17 @@ int launch_fit_plan(const int4* topo, const int32_t* leaf_parent, int n, uint32_
 
 void launch_tree_depth(const int4* topo, int n, const int32_t* unit_root, const uint8_t* uheight, int nunits,
                        const int32_t* top, const uint32_t* uscratch, const uint8_t* ndepth, uint32_t* depth,
-                       const GridFrame* frame, uint32_t* h_depth, GridFrame* h_frame, hipStream_t s)
+                       hipStream_t s)
 {
   if (n < 2) return;
   hipLaunchKernelGGL(k_tree_depth, dim3(64), dim3(256), 0, s, unit_root, uheight, nunits, top, PlanScan{uscratch, n},
                      topo, ndepth, depth);
+}
+
+void launch_build_info(int n, const uint32_t* depth, const GridFrame* frame, uint32_t* h_depth, GridFrame* h_frame,
+                       hipStream_t s)
+{
+  if (n < 2) return;
   hipLaunchKernelGGL(k_build_info, dim3(1), dim3(1), 0, s, (const uint32_t*)depth, frame, h_depth, h_frame);
 }
 

@@ -44,12 +44,15 @@ int launch_fit_plan(const int4* topo, const int32_t* leaf_parent, int n, uint32_
                     int32_t* unit_root, int32_t* stray, std::vector<int32_t>* cross_begin, int* nunits, int* nstray,
                     hipStream_t s);
 // After a build's fit: the number of internal levels on the longest root-leaf path, from
-// the treelet heights and the top-node depths, and the grid's frame, into coherent host
-// memory (complete once the stream is synchronized; nothing for n < 2).  depth: the word
-// cleared by the plan.
+// the treelet heights and the top-node depths, into depth, the word cleared by the plan
+// (nothing for n < 2).
 void launch_tree_depth(const int4* topo, int n, const int32_t* unit_root, const uint8_t* uheight, int nunits,
                        const int32_t* top, const uint32_t* uscratch, const uint8_t* ndepth, uint32_t* depth,
-                       const GridFrame* frame, uint32_t* h_depth, GridFrame* h_frame, hipStream_t s);
+                       hipStream_t s);
+// the depth and the grid's frame into coherent host memory (complete once the stream is
+// synchronized; nothing for n < 2)
+void launch_build_info(int n, const uint32_t* depth, const GridFrame* frame, uint32_t* h_depth, GridFrame* h_frame,
+                       hipStream_t s);
 // two arrays of multiples of 16 bytes from mapped, coherent host memory to the device
 void launch_upload(const void* a, void* da, int64_t a_bytes, const void* b, void* db, int64_t b_bytes, hipStream_t s);
 // Bottom-up boxes: one launch for every treelet (LDS-local walks), then the top
