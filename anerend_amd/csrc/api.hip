@@ -1300,7 +1300,8 @@ static int do_frame_setup(ane_ddgi_ctx* c, const FrameK& fk, bool bake, hipStrea
   return ANE_OK;
 }
 
-extern "C" int ane_ddgi_trace(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame* f, void* stream)
+// ends: the call ends here (else a convolution follows on the stream, whose end is the trace's too)
+static int trace_call(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame* f, void* stream, bool ends)
 {
   if (!c || !s) return fail(ANE_ERR_INVALID_ARG, "NULL context or scene");
   FrameK fk;
@@ -1337,7 +1338,7 @@ extern "C" int ane_ddgi_trace(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddg
                a.probe_base, clk, st);
   ANE_CHECK_HIP(hipGetLastError());
   count_stage(c, clk, kStShade);
-  ANE_TRY(end_call(c, kClkTrace, clk, st));
+  if (ends) ANE_TRY(end_call(c, kClkTrace, clk, st));
   c->rad_begin = fk.layer_begin;
   c->rad_count = fk.layer_count;
   c->rad_bake = bake;
@@ -1345,6 +1346,11 @@ extern "C" int ane_ddgi_trace(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddg
   c->last_count = fk.layer_count;
   c->stats.rays = (uint64_t)nprobes * c->N;
   return ANE_OK;
+}
+
+extern "C" int ane_ddgi_trace(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame* f, void* stream)
+{
+  return trace_call(c, s, f, stream, true);
 }
 
 extern "C" int ane_ddgi_convolve(ane_ddgi_ctx* c, const ane_ddgi_frame* f, void* stream)
@@ -1373,7 +1379,7 @@ extern "C" int ane_ddgi_convolve(ane_ddgi_ctx* c, const ane_ddgi_frame* f, void*
 
 extern "C" int ane_ddgi_update(ane_ddgi_ctx* c, const ane_scene* s, const ane_ddgi_frame* f, void* stream)
 {
-  ANE_TRY(ane_ddgi_trace(c, s, f, stream));
+  ANE_TRY(trace_call(c, s, f, stream, false));
   return ane_ddgi_convolve(c, f, stream);
 }
 
