@@ -273,8 +273,11 @@ int ane_ddgi_translate(ane_ddgi_ctx* ctx, const float* camera_pos3, int32_t* shi
  * scene (no refit or rebuild in between) and the same sun direction, the context
  * keeps a grid of the triangles projected along the sun and a shadow ray tests
  * the triangles of its cell instead of traversing; the decisions are identical.
- * The grid takes about 28 bytes per triangle plus 4 per cell (one cell per
- * triangle) and is rebuilt on the stream when that scene or sun recurs. */
+ * The grid takes about 145 bytes per triangle and is rebuilt on the stream when that
+ * scene or sun recurs.  A new sun over an unchanged scene builds at the first trace
+ * that sees it when the trace has the rays to pay for it (2.5 per triangle and 600k
+ * more) and no grid of the scene was found out of use; under a caller's capture, only
+ * when one was found in use. */
 int ane_ddgi_trace(ane_ddgi_ctx* ctx, const ane_scene* scene, const ane_ddgi_frame* frame,
                    void* stream);
 /* IrradianceProbeConvolve: cosine-weighted octahedral convolution of the stored
@@ -342,7 +345,8 @@ int ane_ddgi_debug_rays(ane_ddgi_ctx* ctx, ane_hit* hits, uint8_t* shadowed, voi
  * cell lookups and candidate triangle tests instead. */
 int ane_ddgi_set_counting(ane_ddgi_ctx* ctx, int32_t mode);
 /* Fills *out; returns ANE_ERR_DEVICE (with *out filled) while a traversal
- * fault is pending. */
+ * fault is pending.  Waits for the context's queued calls (and, as any copy on the null
+ * stream, for that stream and the blocking ones), as ane_ddgi_stats_reset does. */
 int ane_ddgi_stats_get(const ane_ddgi_ctx* ctx, ane_ddgi_stats* out);
 /* Resets the stage timers and clears the traversal fault flags. */
 int ane_ddgi_stats_reset(ane_ddgi_ctx* ctx);
