@@ -295,10 +295,12 @@ struct SunGridCache {
     pending = true;
     return ANE_OK;
   }
-  // judges the current build, whose launches were queued on st
+  // judges the current build, whose launches were queued on st (after a caller's replay the
+  // flag may be another build's: good enough to end the builds of a moving sun, and
+  // known_valid relies on it no more)
   int judge(hipStream_t st)
   {
-    return built.set && !captured && !replayable && !(known == built) ? read_back(built, st) : ANE_OK;
+    return built.set && !captured && !(known == built) ? read_back(built, st) : ANE_OK;
   }
   // device buffers for a scene of ntri triangles: about ANE_SUNGRID_DENSITY cells
   // per triangle (at most 4096 x 4096), ANE_SUNGRID_CAPACITY entries per triangle
@@ -355,7 +357,7 @@ struct SunGridCache {
     const bool callers = capturing && !own_graph;  // a graph of the caller's
     if (!capturing) poll();  // no event queries under capture
     const bool current = built == k;
-    if (current && (capturing || !captured)) {
+    if (current && (callers || !captured)) {
       *use = true;
       if (!capturing) ANE_TRY(judge(st));
       if (valid) *valid = capturing ? -1 : known_valid();  // a graph keeps both ways: the grid may change before a replay

@@ -99,3 +99,37 @@ def test_a_callers_capture_of_a_new_direction_traverses():
         assert np.array_equal(ha, hb) and np.array_equal(sa, sb)
         assert np.array_equal(a.atlas, b.atlas)
     g.close()
+
+
+@pytest.mark.parametrize("update", [direct, library_graph])
+def test_builds_end_beside_a_callers_graph(update):
+    """The same over a scene whose grids are refused, in a context that has a build in a
+    caller's graph."""
+    ds = native.DeviceScene(towers_scene())
+    a, b = native.ProbeGrid(CFG), native.ProbeGrid(CFG)
+    b.set_counting(1)
+    stream = None if update is direct else _stream()
+    same, f = native.DeviceScene(towers_scene()), frame(20, along=True)
+    a.update(same, f)
+    a.update(same, f)  # a first build, over another scene: the grid's buffers
+    native.synchronize()
+    other = frame(21, along=True)
+    graphs = [Graph(lambda st: native.load().ane_ddgi_update(a.handle, ds.handle, ctypes.byref(other), st))
+              for _ in range(2)]
+    update(a, ds, other, stream)  # its build was captured alone
+    native.synchronize(stream)
+    graphs[1].launch()
+    estimates = []
+    for k in range(8):
+        f = frame(k, along=True)
+        update(a, ds, f, stream)
+        native.synchronize(stream)
+        estimates.append(a.stats()["sun_grid_candidates"])
+    assert np.count_nonzero(np.diff(estimates)) <= 1
+    a.atlas = np.zeros(CFG.atlas_shape, np.float32)
+    graphs[1].launch()
+    b.update(ds, other)
+    (ha, sa), (hb, sb) = a.debug_rays(other), b.debug_rays(other)
+    assert np.array_equal(ha, hb) and np.array_equal(sa, sb)
+    for g in graphs:
+        g.close()
