@@ -1285,7 +1285,11 @@ static void count_stage(ane_ddgi_ctx* c, const ClockArg& clk, int stage)
 // a call: 41.6 -> 44.4 us for the convolution of 16,384 probes, were it recorded on each).
 static int end_call(ane_ddgi_ctx* c, int k, const ClockArg& clk, hipStream_t st)
 {
-  if (!clk.c || !st) return ANE_OK;
+  if (!clk.c || !st || st == hipStreamLegacy) return ANE_OK;
+  if (st == hipStreamPerThread) {  // no stream object to ask for flags
+    ANE_CHECK_HIP(hipEventRecord(c->call_end[k], st));
+    return ANE_OK;
+  }
   unsigned flags = 0;
   ANE_CHECK_HIP(hipStreamGetFlags(st, &flags));
   if (flags & hipStreamNonBlocking) ANE_CHECK_HIP(hipEventRecord(c->call_end[k], st));

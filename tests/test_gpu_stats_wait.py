@@ -47,3 +47,18 @@ def test_statistics_wait_for_their_context_alone(flags):
     assert other.stats()["calls"]["convolve"] == 402
     for s in streams:
         assert hip.hipStreamDestroy(s) == 0
+
+
+@pytest.mark.parametrize("handle", [None, 2])  # the null stream, the thread's own (hipStreamPerThread)
+def test_statistics_of_calls_on_implicit_streams(handle):
+    ds = native.DeviceScene(scenegen.room_scene(1, num_boxes=4))
+    cfg = Config.make((16, 4, 16), step=(1.0, 1.0, 1.0), rays=256)
+    grid, frame = native.ProbeGrid(cfg), scenegen.make_frame(1, config=cfg)
+    stream = ctypes.c_void_p(handle)
+    for k in range(8):
+        grid.update(ds, frame, stream)
+        grid.translate((2.0 + k, 0.0, 3.0), stream)
+    s = grid.stats()
+    native.synchronize(stream)
+    assert grid.stats() == s
+    assert s["calls"]["convolve"] == 8 and s["calls"]["translate"] == 8
